@@ -74,6 +74,80 @@ __device__ __forceinline__ void xform_inplace(const double* __restrict__ xf, R* 
 // vector-memory access in the quadrature loop.  Up to JKB_MAX_BRA_PRIMS pairs.
 #define JKB_MAX_BRA_PRIMS 128
 
+// Split of one ket's primitive quartets over adjacent lanes (bra-row kernels).
+// One lane used to walk all of a quartet's primitive quartets (81 x 81 for two
+// contracted cc-pVDZ s pairs: 17 ms for one water, whose whole build has 58
+// MFLOP), while most lanes of a block idled because a bucket of a small molecule
+// holds fewer kets than the block has lanes.  A block therefore gives every ket
+// of such a bucket n = nb * nk lanes: lane sub takes the bra primitive pairs
+// sb, sb + nb, ... and the ket primitive pairs sk, sk + nk, ...; the partial
+// (e0|f0) sets are summed over the n lanes before the horizontal transfer, and
+// lane sub = 0 digests the quartet.  n = 1 (every large bucket) runs the same
+// loops with unit steps.  The rule is local to the block (split_of): lanes are
+// only taken where no ket is waiting for them.
+struct Split {
+  int n, nb, nk;  // lanes per ket, of which along the bra / the ket primitives (powers of two)
+  int lg;         // log2 n
+  int sub, sb, sk;
+};
+// the LDS copies of the bra primitives are padded with zero-coefficient
+// records to a multiple of this, so the bra loop of every lane has one
+// (uniform) trip count
+#define JKB_BRA_PAD 16
+
+// n kets, `threads` lanes, npp bra primitive pairs, kets of bucket b
+__device__ __forceinline__ Split split_of(int n, int threads, int npp, int b, int lane) {
+  // typical primitive-pair counts of the buckets (the last one: cc-pVDZ s pairs)
+  const int kq = b == 0 ? 1 : b == 1 ? 4 : b == 2 ? 9 : b == 3 ? 20 : b == 4 ? 40 : 81;
+  Split s;
+  s.n = 1;
+  s.lg = 0;
+  while (s.n < 64 && 2 * s.n * n <= threads && 2 * s.n <= npp * kq) {
+    s.n *= 2;
+    ++s.lg;
+  }
+  // the factorisation with the fewest iterations of one lane
+  int lb = 0, best = 1 << 30;
+#pragma unroll
+  for (int i = 0; (1 << i) <= JKB_BRA_PAD; ++i) {
+    if ((1 << i) > s.n) break;
+    const int nk = s.n >> i;
+    const int it = ((npp + (1 << i) - 1) >> i) * ((kq + nk - 1) / nk);
+    if (it < best) {
+      best = it;
+      lb = i;
+    }
+  }
+  s.nb = 1 << lb;
+  s.nk = s.n >> lb;
+  s.sub = lane & (s.n - 1);
+  s.sb = s.sub & (s.nb - 1);
+  s.sk = s.sub >> lb;
+  return s;
+}
+__device__ __forceinline__ Split split_none() { return {1, 1, 1, 0, 0, 0, 0}; }
+
+// sum over the n lanes of a ket (all of them active); every lane gets it
+template <int N, typename R>
+__device__ __forceinline__ void split_sum(R (&v)[N], int n) {
+#pragma unroll 1
+  for (int o = 1; o < n; o <<= 1) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += __shfl_xor(v[i], o);
+  }
+}
+
+template <int N, int M, typename R>
+__device__ __forceinline__ void split_sum(R (&v)[N][M], int n) {
+#pragma unroll 1
+  for (int o = 1; o < n; o <<= 1) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int j = 0; j < M; ++j) v[i][j] += __shfl_xor(v[i][j], o);
+  }
+}
+
 // Contracted (e0|f0) of a quartet: Rys quadrature over every surviving
 // primitive quartet.  The FP64 path reads the PrimJK records, the FP32 path
 // the PrimF32 copies (prims32).  UNIFORM_BRA: the caller guarantees one bra per
@@ -87,7 +161,7 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
                                          R (&acc)[Dims<LA, LB, LC, LD>::NE][Dims<LA, LB, LC, LD>::NF],
                                          int& nprim_used, const PrimV<double>* sbra = nullptr,
                                          const PrimV<float>* sbra32 = nullptr, int nbra64 = 0,
-                                         int nbra32 = 0) {
+                                         int nbra32 = 0, const Split& sp = split_none()) {
   using Dm = Dims<LA, LB, LC, LD>;
   constexpr bool F32 = sizeof(R) == 4;
 #pragma unroll
@@ -106,36 +180,49 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
   if (UNIFORM_BRA && sbra) {
     // the LDS copies hold only the bra primitive pairs with |K| >= qcut
     // (nbra64 FP64, nbra32 FP32 records), so the loop needs no test for them
+    // (zero-coefficient records pad it to a multiple of JKB_BRA_PAD)
     const int npp = __builtin_amdgcn_readfirstlane(sbra32 ? nbra32 : nbra64);
+    const int nb = sp.nb, nk = sp.nk, nit = (npp + nb - 1) & ~(nb - 1);
     // small classes, FP32: the next ket primitive pair is loaded while the
     // current one runs against the bra's primitives (where registers are
     // short, i.e. the larger classes and FP64, it costs more than it hides)
     constexpr bool PREF = F32 && Dm::NE * Dm::NF <= 9;
     const int nq = Q.nprim;
-    PrimV<R> qn{};
-    if (PREF && nq > 0) qn = ket(Q.prim0);
-    for (int iq = 0; iq < nq; ++iq) {
-      PrimV<R> qq;
-      if constexpr (PREF) {
-        qq = qn;
-        if (iq + 1 < nq) qn = ket(Q.prim0 + iq + 1);
-      } else {
-        qq = ket(Q.prim0 + iq);
+    auto walk = [&](const int sb, const int sk, const int nb, const int nk, const int nit) {
+      PrimV<R> qn{};
+      if (PREF && sk < nq) qn = ket(Q.prim0 + sk);
+      for (int iq = sk; iq < nq; iq += nk) {
+        PrimV<R> qq;
+        if constexpr (PREF) {
+          qq = qn;
+          if (iq + nk < nq) qn = ket(Q.prim0 + iq + nk);
+        } else {
+          qq = ket(Q.prim0 + iq);
+        }
+        if (fabs(qq.Kg) < qcut) continue;
+        R AQ[3];
+        ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
+        auto run = [&](auto bra) {
+          for (int ip = 0; ip < nit; ip += nb)
+            nprim_used +=
+                rys_accumulate<LA, LB, LC, LD, R>(bra(ip + sb), qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
+        };
+        if constexpr (F32) {
+          if (sbra32) run([&](int i) { return sbra32[i]; });
+          else run([&](int i) { return prim_v<float>(sbra[i]); });
+        } else {
+          run([&](int i) { return sbra[i]; });
+        }
       }
-      if (fabs(qq.Kg) < qcut) continue;
-      R AQ[3];
-      ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
-      auto run = [&](auto bra) {
-        for (int ip = 0; ip < npp; ++ip)
-          nprim_used += rys_accumulate<LA, LB, LC, LD, R>(bra(ip), qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
-      };
-      if constexpr (F32) {
-        if (sbra32) run([&](int i) { return sbra32[i]; });
-        else run([&](int i) { return prim_v<float>(sbra[i]); });
-      } else {
-        run([&](int i) { return sbra[i]; });
-      }
+    };
+    // the smallest classes keep a loop of their own for unsplit kets, whose
+    // bra records are uniform LDS reads (the shared loop costs them 1 %)
+    if (Dm::NE * Dm::NF <= 9 && sp.n == 1) {
+      walk(0, 0, 1, 1, npp);
+      return;
     }
+    walk(sp.sb, sp.sk, nb, nk, nit);
+    if (sp.n > 1) split_sum(acc, sp.n);
     return;
   }
   const int pp0 = UNIFORM_BRA ? __builtin_amdgcn_readfirstlane(P.prim0) : P.prim0;
@@ -259,11 +346,11 @@ __device__ __forceinline__ void quartet_block(const ShellPair& P, const ShellPai
                                               R qcut, R imu2, R (&V)[Dims<LA, LB, LC, LD>::NBLK], int& nprim_used,
                                               const PrimV<double>* sbra = nullptr,
                                               const PrimV<float>* sbra32 = nullptr, int nbra64 = 0,
-                                              int nbra32 = 0) {
+                                              int nbra32 = 0, const Split& sp = split_none()) {
   using Dm = Dims<LA, LB, LC, LD>;
   R acc[Dm::NE][Dm::NF];
   contract<LA, LB, LC, LD, R, UNIFORM_BRA>(P, Q, prims, prims32, tabN, tab32N, qcut, imu2, acc, nprim_used, sbra,
-                                           sbra32, nbra64, nbra32);
+                                           sbra32, nbra64, nbra32, sp);
   R AB[3], CD[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -837,6 +924,15 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       n64 += __popcll(m64);
       n32 += __popcll(m32);
     }
+    // zero-coefficient records up to a multiple of JKB_BRA_PAD (dropped by
+    // the primitive screen)
+    if (lane0 < JKB_BRA_PAD) {
+      if (n64 + lane0 < ((n64 + JKB_BRA_PAD - 1) & ~(JKB_BRA_PAD - 1)))
+        s_bra[n64 + lane0] = {1.0, 0.0, {0.0, 0.0, 0.0}, 0.5};
+      if constexpr (B32)
+        if (n32 + lane0 < ((n32 + JKB_BRA_PAD - 1) & ~(JKB_BRA_PAD - 1)))
+          s_bra32[n32 + lane0] = {1.0f, 0.0f, {0.0f, 0.0f, 0.0f}, 0.5f};
+    }
     if (lane0 == 0) {
       s_nbra[0] = n64;
       s_nbra[1] = n32;
@@ -881,8 +977,11 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
   for (int b = 0; b < OQPH_NBKT; ++b) {
     const int n = __builtin_amdgcn_readfirstlane(item[1 + b]);
     const int kbase = bw.kb[b];
-    for (int k0 = wv * 64; k0 < n; k0 += nw * 64) {
-      const int k = k0 + lane;
+    const Split sp = bra_lds && 2 * n <= nw * 64 ? split_of(n, nw * 64, nbra64, b, lane) : split_none();
+    const int kw = 64 >> sp.lg;  // kets per wavefront
+    const bool head = sp.sub == 0;
+    for (int k0 = wv * kw; k0 < n; k0 += nw * kw) {
+      const int k = k0 + (lane >> sp.lg);
       const bool active = k < n;
       int iq = 0;
       ShellPair Q{};
@@ -908,8 +1007,8 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
         bound = P.Q * Q.Q * dm;
         skip = !mine || (qbra * prm.maxden < prm.cutoff) || (bound < prm.cutoff);
       }
-      n_skip += (active && mine && skip) ? 1 : 0;
-      n_comp += skip ? 0 : 1;
+      n_skip += (head && active && mine && skip) ? 1 : 0;
+      n_comp += (head && !skip) ? 1 : 0;
       double V[NBLK];
 #pragma unroll
       for (int i = 0; i < NOUT; ++i) V[i] = 0.0;
@@ -923,7 +1022,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             quartet_block<LA, LB, LC, LD, PURE, float, true>(P, Q, prm.prims, prm.prims32, tabN, tab32N,
                                                              prm.xform, (float)(1.0e-4 * prm.cutoff),
                                                              (float)prm.inv_mu2, Vf, nprim, sbra, sbra32, nbra64,
-                                                             nbra32);
+                                                             nbra32, sp);
 #pragma unroll
             for (int i = 0; i < NOUT; ++i) V[i] = (double)Vf[i];
           }
@@ -931,12 +1030,17 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
         if (!lowp)
           quartet_block<LA, LB, LC, LD, PURE, double, true>(P, Q, prm.prims, prm.prims32, tabN, tab32N,
                                                             prm.xform, 1.0e-4 * prm.cutoff, prm.inv_mu2, V, nprim,
-                                                            sbra, nullptr, nbra64, nbra32);
+                                                            sbra, nullptr, nbra64, nbra32, sp);
       }
-      n_f32 += (lowp && !skip) ? 1 : 0;
-      n_valid += nprim ? 1 : 0;
       n_prim += (unsigned)nprim;
-      const bool valid = !skip && nprim > 0;
+      if (sp.n > 1) {  // primitive quartets of the ket, over its lanes
+        int t[1] = {nprim};
+        split_sum<1, int>(t, sp.n);
+        nprim = t[0];
+      }
+      n_f32 += (lowp && head && !skip) ? 1 : 0;
+      n_valid += (head && nprim) ? 1 : 0;
+      const bool valid = head && !skip && nprim > 0;
       if (__ballot(valid) == 0ull) continue;  // wave-uniform
       const double c = prm.cutoff;
 #pragma unroll

@@ -136,7 +136,7 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
                                               const double* __restrict__ tabN,
                                               const float* __restrict__ tab32N, R qcut, R imu2,
                                               R (&acc)[NM][Dims<LA, LB, LC, LD>::NE][Dims<LA, LB, LC, LD>::NF],
-                                              int (&np)[NM]) {
+                                              int (&np)[NM], const Split& sp) {
   using Dm = Dims<LA, LB, LC, LD>;
   constexpr int NE = Dm::NE, NF = Dm::NF;
   constexpr bool F32 = sizeof(R) == 4;
@@ -152,6 +152,9 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
 #pragma unroll
   for (int d = 0; d < 3; ++d) AC[d] = (R)(Ac[d] - Q.A[d]);  // formed in FP64
   const R qcut2 = qcut * qcut;
+  // this lane's share of the primitive quartets (Split); the records are
+  // padded to a multiple of JKB_BRA_PAD, so the bra loop's trip count is uniform
+  const int nb = sp.nb, nk = sp.nk, nit = (ncp + nb - 1) & ~(nb - 1);
   int ng = 0;
   auto ket = [&](int i) -> PrimV<R> {
     if constexpr (F32) return prim_v<float>(prims32[i]);
@@ -161,12 +164,12 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
   constexpr bool PREF = F32 && NE * NF <= 9;
   const int nq = Q.nprim;
   PrimV<R> qn{};
-  if (PREF && nq > 0) qn = ket(Q.prim0);
-  for (int iq = 0; iq < nq; ++iq) {
+  if (PREF && sp.sk < nq) qn = ket(Q.prim0 + sp.sk);
+  for (int iq = sp.sk; iq < nq; iq += nk) {
     PrimV<R> qq;
     if constexpr (PREF) {
       qq = qn;
-      if (iq + 1 < nq) qn = ket(Q.prim0 + iq + 1);
+      if (iq + nk < nq) qn = ket(Q.prim0 + iq + nk);
     } else {
       qq = ket(Q.prim0 + iq);
     }
@@ -174,7 +177,7 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
     if (fabs(kq) < qcut) continue;
     R AQ[3];
     ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
-    for (int ip = 0; ip < ncp; ++ip) {
+    for (int ip = sp.sb; ip < nit + sp.sb; ip += nb) {
       const R* r = rec + ip * stride;
       PrimV<R> pp;
       pp.g = r[0];
@@ -212,6 +215,11 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
           for (int f = 0; f < NF; ++f) acc[m][e][f] += w * val[e][f];
       }
     }
+  }
+  if (sp.n > 1) {
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+      if (m < nmem) split_sum(acc[m], sp.n);
   }
   return ng;
 }
@@ -263,7 +271,8 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
   double* s_k2 = s_ds + (drows ? (size_t)nshl * nsh : 0);
   double* s_d2 = s_k2 + (two ? nk : 0);
   double* s_cp = s_d2 + (two && drows ? nk : 0);
-  float* s_cp32 = (float*)(s_cp + (size_t)ncp * stride);
+  const int ncpp = TILE ? ncp : (ncp + JKB_BRA_PAD - 1) & ~(JKB_BRA_PAD - 1);  // records with padding
+  float* s_cp32 = (float*)(s_cp + (size_t)ncpp * stride);
   const int P0 = __builtin_amdgcn_readfirstlane(ch[OQPH_JKG_HDR]);
   const ShellPair PA = prm.pairs[P0];  // the members' common centres A, B
   for (int i = threadIdx.x; i < nk; i += blockDim.x) s_k[i] = 0.0;
@@ -347,9 +356,12 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
       }
     }
   } else {
-    for (int i = threadIdx.x; i < ncp * stride; i += blockDim.x) s_cp[i] = cv.cp[cprim0 + i];
+    // padding: zero prefactors (dropped by the primitive screen), zeta = 1
+    for (int i = threadIdx.x; i < ncpp * stride; i += blockDim.x)
+      s_cp[i] = i < ncp * stride ? cv.cp[cprim0 + i] : (i % stride == 0 ? 1.0 : 0.0);
     if (prm.mixed)
-      for (int i = threadIdx.x; i < ncp * stride; i += blockDim.x) s_cp32[i] = cv.cp32[cprim0 + i];
+      for (int i = threadIdx.x; i < ncpp * stride; i += blockDim.x)
+        s_cp32[i] = i < ncp * stride ? cv.cp32[cprim0 + i] : (i % stride == 0 ? 1.0f : 0.0f);
   }
   __syncthreads();
   const double* tabN = T64 ? (const double*)s_t64 : prm.rys + RYS_OFF[NR];
@@ -364,7 +376,10 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
   for (int b = 0; b < OQPH_NBKT; ++b) {
     const int n = __builtin_amdgcn_readfirstlane(item[1 + b]);
     const int kbase = bw.kb[b];
-    for (int k0 = wv * 64; k0 < n; k0 += nw * 64) {
+    const Split sp = TILE || 2 * n > nw * 64 ? split_none() : split_of(n, nw * 64, ncp, b, lane);
+    const int kw = 64 >> sp.lg;  // kets per wavefront
+    const bool head = sp.sub == 0;
+    for (int k0 = wv * kw; k0 < n; k0 += nw * kw) {
       // the member tables are read from LDS where they are used: an opaque
       // zero offset keeps the compiler from hoisting every member's fields
       // out of the ket loop into registers
@@ -374,7 +389,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
       const double* mq = s_mq + z;
       const double* mthr = s_mthr + z;
       const double* mdab = s_mdab + z;
-      const int k = k0 + lane;
+      const int k = k0 + (lane >> sp.lg);
       const bool active = k < n;
       int iq = 0;
       ShellPair Q{};
@@ -410,10 +425,10 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
             live |= 1u << m;
             bmax = fmax(bmax, bound);
           }
-          n_skip += (tri && mine && skip && Q.Q >= mthr[m]) ? 1 : 0;
+          n_skip += (head && tri && mine && skip && Q.Q >= mthr[m]) ? 1 : 0;
         }
       }
-      n_comp += __popc(live);
+      n_comp += head ? __popc(live) : 0;
       bool lowp = false;
       if constexpr (T32) lowp = prm.mixed && __ballot(live != 0u && bmax >= prm.fp32_cut) == 0ull;
       // each member's final AO block; the (e0|f0) accumulators live only
@@ -439,7 +454,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
             else
               n_grp += contract_group<LA, LB, LC, LD, NM, float>(Q, Ac, prm.prims, prm.prims32, s_cp32, ncp, stride,
                                                                   nmem, live, tabN, tab32N, (float)(1.0e-4 * c),
-                                                                  (float)prm.inv_mu2, accf, np);
+                                                                  (float)prm.inv_mu2, accf, np, sp);
             float ABf[3], CDf[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
@@ -468,7 +483,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
           else
             n_grp += contract_group<LA, LB, LC, LD, NM, double>(Q, Ac, prm.prims, prm.prims32, s_cp, ncp, stride,
                                                                  nmem, live, tabN, tab32N, 1.0e-4 * c, prm.inv_mu2,
-                                                                 acc, np);
+                                                                 acc, np, sp);
 #pragma unroll
           for (int m = 0; m < NM; ++m) {
             if (m >= nmem) break;  // uniform
@@ -479,12 +494,15 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
           }
         }
       }
-      n_f32 += lowp ? __popc(live) : 0;
+      n_f32 += (lowp && head) ? __popc(live) : 0;
       const int oc = Q.ao_a, od = Q.ao_b;
       bool any_valid = false;
 #pragma unroll
+      for (int m = 0; m < NM; ++m) n_prim += (unsigned)np[m];
+      if (sp.n > 1) split_sum<NM, int>(np, sp.n);  // over the ket's lanes; its first lane digests
+#pragma unroll
       for (int m = 0; m < NM; ++m) {
-        n_prim += (unsigned)np[m];
+        if (!head) np[m] = 0;
         n_valid += np[m] ? 1 : 0;
         any_valid |= ((live >> m) & 1u) && np[m] > 0;
       }

@@ -1380,7 +1380,10 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
       if (rows && s->rows_mode == 1 && fit0) {
         const double old_at = (double)nket * (oc * od + (oa + obn) * (oc + od));
         const double new_at = (double)nket * oc * od + (double)nbra * nrow * ncol;
-        rows = new_at < 0.5 * old_at;
+        // launches with fewer kets than the lanes of one block per CU are bound
+        // by the longest lane, not by atomics: the bra-row kernel spreads a
+        // ket's primitive quartets over its idle lanes, k_jk does not
+        rows = new_at < 0.5 * old_at || nket < (long long)s->ncu * 512;
       }
       if (rows) {
         // grouped bra-row kernel: one block per chunk of pairs sharing primitives
@@ -1415,7 +1418,8 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
             t.cost *= cs.ncp[ci];
             its.push_back(t);
             const size_t rows_b = (size_t)cs.nrow[ci] * ncol * sizeof(double);
-            const size_t prims_b = (size_t)cs.ncp[ci] * cs.stride[ci] * (sizeof(double) + sizeof(float));
+            // (the kernel pads the records to a multiple of 16)
+            const size_t prims_b = (size_t)((cs.ncp[ci] + 15) & ~15) * cs.stride[ci] * (sizeof(double) + sizeof(float));
             need_n = std::max(need_n, nd * rows_b + prims_b);
             need_d = std::max(need_d, 2 * nd * rows_b + (size_t)cs.nshl[ci] * s->nsh * sizeof(double) + prims_b);
           }
