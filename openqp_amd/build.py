@@ -41,6 +41,15 @@ GRAD_HL = [(2, 2, 2, 2), (2, 2, 2, 1)]
 F_GRAD = [(3, 0, 0, 0), (3, 0, 1, 0), (3, 0, 1, 1), (3, 0, 2, 0), (3, 0, 3, 0), (3, 1, 0, 0), (3, 1, 1, 0),
           (3, 2, 0, 0), (3, 3, 0, 0)]
 
+# classes with a cooperative J/K kernel (jkc_class.hip; the list matches
+# OQPH_JKC_CLASSES in dispatch.hip)
+JKC = [(1, 1, 1, 1), (2, 0, 1, 1), (2, 0, 2, 0), (2, 1, 1, 0), (2, 1, 1, 1), (2, 1, 2, 0), (2, 1, 2, 1), (2, 2, 1, 0),
+       (2, 2, 1, 1), (2, 2, 2, 0), (2, 2, 2, 1), (2, 2, 2, 2),
+       (3, 0, 1, 1), (3, 0, 2, 0), (3, 0, 2, 1), (3, 0, 2, 2), (3, 0, 3, 0),
+       (3, 1, 1, 0), (3, 1, 1, 1), (3, 1, 2, 0), (3, 1, 2, 1), (3, 1, 2, 2), (3, 1, 3, 0), (3, 1, 3, 1),
+       (3, 2, 1, 0), (3, 2, 1, 1), (3, 2, 2, 0), (3, 2, 2, 1), (3, 2, 2, 2), (3, 2, 3, 0), (3, 2, 3, 1), (3, 2, 3, 2),
+       (3, 3, 1, 0), (3, 3, 1, 1), (3, 3, 2, 0), (3, 3, 2, 1), (3, 3, 2, 2), (3, 3, 3, 0), (3, 3, 3, 1)]
+
 
 def _cost(c):
     a, b, cc, d = c
@@ -50,6 +59,8 @@ def _cost(c):
 # headers each translation unit depends on (cache key = unit + these + flags)
 DEPS = {
     "jk_class.hip": ["jk_device.h", "jkg_device.h", "eri_device.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
+    "jkc_class.hip": ["jkc_device.h", "jk_device.h", "eri_device.h", "oqph_common.h", "rys_table.inc",
+                      "rys_table_f32.inc"],
     "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
     "session.hip": ["oqph_common.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
     "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
@@ -78,7 +89,8 @@ def _jobs():
              ("hl.hip", [], "hl.o"), ("sigma.hip", [], "sigma.o"), ("xc.hip", [], "xc.o")]
     heavy, light = [], []
     per_class = [(c, "jk_class.hip", "jk") for c in CLASSES + F_JK] + \
-                [(c, "grad_class.hip", "gr") for c in CLASSES + F_GRAD if c not in GRAD_HL]
+                [(c, "grad_class.hip", "gr") for c in CLASSES + F_GRAD if c not in GRAD_HL] + \
+                [(c, "jkc_class.hip", "jkc") for c in JKC]
     for c, unit, tag in sorted(per_class, key=lambda t: _cost(t[0]), reverse=True):
         a, b, cc, d = c
         defs = [f"-DXA={a}", f"-DXB={b}", f"-DXC={cc}", f"-DXD={d}"]

@@ -21,6 +21,14 @@ namespace oqph {
   X(2, 0, 1, 1) X(2, 0, 2, 0) X(2, 1, 0, 0) X(2, 1, 1, 0) X(2, 1, 1, 1) X(2, 1, 2, 0) X(2, 1, 2, 1) X(2, 2, 0, 0) \
   X(2, 2, 1, 0) X(2, 2, 1, 1) X(2, 2, 2, 0) X(3, 0, 0, 0) X(3, 0, 1, 0) X(3, 0, 1, 1) X(3, 0, 2, 0) X(3, 0, 3, 0) \
   X(3, 1, 0, 0) X(3, 1, 1, 0) X(3, 2, 0, 0) X(3, 3, 0, 0)
+// cooperative J/K kernel (k_jkc; jkc_class.hip), the JKC list of build.py
+#define OQPH_JKC_CLASSES(X) \
+  X(1, 1, 1, 1) X(2, 0, 1, 1) X(2, 0, 2, 0) X(2, 1, 1, 0) X(2, 1, 1, 1) X(2, 1, 2, 0) X(2, 1, 2, 1) \
+  X(2, 2, 1, 0) X(2, 2, 1, 1) X(2, 2, 2, 0) X(2, 2, 2, 1) X(2, 2, 2, 2) X(3, 0, 1, 1) X(3, 0, 2, 0) \
+  X(3, 0, 2, 1) X(3, 0, 2, 2) X(3, 0, 3, 0) X(3, 1, 1, 0) X(3, 1, 1, 1) X(3, 1, 2, 0) X(3, 1, 2, 1) \
+  X(3, 1, 2, 2) X(3, 1, 3, 0) X(3, 1, 3, 1) X(3, 2, 1, 0) X(3, 2, 1, 1) X(3, 2, 2, 0) X(3, 2, 2, 1) \
+  X(3, 2, 2, 2) X(3, 2, 3, 0) X(3, 2, 3, 1) X(3, 2, 3, 2) X(3, 3, 1, 0) X(3, 3, 1, 1) X(3, 3, 2, 0) \
+  X(3, 3, 2, 1) X(3, 3, 2, 2) X(3, 3, 3, 0) X(3, 3, 3, 1)
 #define OQPH_SCHWARZ_CLASSES(X) X(0, 0) X(1, 0) X(1, 1) X(2, 0) X(2, 1) X(2, 2)
 
 #define OQPH_CODE(a, b, c, d) ((a) * 1000 + (b) * 100 + (c) * 10 + (d))
@@ -37,6 +45,10 @@ namespace oqph {
   bool jkb_info_##a##b##c##d(bool, int*, size_t*, size_t);                                                 \
   bool jk_res_##a##b##c##d(int, bool, KernelRes*);
 OQPH_JK_CLASSES(OQPH_DECL_JK)
+#define OQPH_DECL_JKC(a, b, c, d)                                                   \
+  void launch_jkc_##a##b##c##d(bool, const JKParams&, const WaveWork&, hipStream_t); \
+  bool jkc_res_##a##b##c##d(bool, bool, KernelRes*);
+OQPH_JKC_CLASSES(OQPH_DECL_JKC)
 #define OQPH_DECL_GR(a, b, c, d)                                              \
   void launch_grad_##a##b##c##d(const GradParams&, const WaveWork&, hipStream_t, bool, bool); \
   bool grad_res_##a##b##c##d(KernelRes*, bool, bool);
@@ -98,6 +110,17 @@ bool launch_jkt(int la, int lb, int lc, int ld, bool pure, const JKParams& p, co
   }
 }
 
+bool launch_jkc(int la, int lb, int lc, int ld, bool pure, const JKParams& p, const WaveWork& ww, hipStream_t s) {
+  if (ww.nwaves == 0) return true;
+  switch (OQPH_CODE(la, lb, lc, ld)) {
+#define OQPH_CASE(a, b, c, d) \
+  case OQPH_CODE(a, b, c, d): launch_jkc_##a##b##c##d(pure, p, ww, s); return true;
+    OQPH_JKC_CLASSES(OQPH_CASE)
+#undef OQPH_CASE
+    default: return false;
+  }
+}
+
 // members per tile of the class's tiled bra-row kernel; 0: none
 int jkt_info(int la, int lb, int lc, int ld, bool pure, size_t* static_lds, size_t lds_max) {
   switch (OQPH_CODE(la, lb, lc, ld)) {
@@ -132,9 +155,9 @@ bool jkb_info(int la, int lb, int lc, int ld, bool pure, int* nrow, size_t* stat
 }
 
 // Compiled resources of one class-templated kernel: kind 0 = k_jk, 1 = k_jkb,
-// 2 = k_grad, 3 = k_schwarz (lc, ld ignored), 4 = k_jkg, 6 = tiled k_jkg; false when there is no such
-// kernel.  hipFuncGetAttributes reads the code object, nothing is launched.
-// kind | 16 (k_jk, k_jkb, k_jkg): the open-shell variant
+// 2 = k_grad, 3 = k_schwarz (lc, ld ignored), 4 = k_jkg, 6 = tiled k_jkg, 7 = k_jkc; false when there is no
+// such kernel.  hipFuncGetAttributes reads the code object, nothing is launched.
+// kind | 16 (k_jk, k_jkb, k_jkg, k_jkc): the open-shell variant
 bool kernel_resources(int kind, int la, int lb, int lc, int ld, bool pure, KernelRes* r) {
   const int base = kind & 15;
   if (base == 0 || base == 1 || base == 3 || base == 4 || base == 6) {
@@ -143,6 +166,15 @@ bool kernel_resources(int kind, int la, int lb, int lc, int ld, bool pure, Kerne
 #define OQPH_CASE(a, b, c, d) \
   case OQPH_CODE(a, b, c, d): return jk_res_##a##b##c##d(kind, pure, r);
       OQPH_JK_CLASSES(OQPH_CASE)
+#undef OQPH_CASE
+      default: return false;
+    }
+  }
+  if (base == 7) {
+    switch (OQPH_CODE(la, lb, lc, ld)) {
+#define OQPH_CASE(a, b, c, d) \
+  case OQPH_CODE(a, b, c, d): return jkc_res_##a##b##c##d(pure, (kind & 16) != 0, r);
+      OQPH_JKC_CLASSES(OQPH_CASE)
 #undef OQPH_CASE
       default: return false;
     }

@@ -41,11 +41,26 @@ struct AO {
   static constexpr int N = (PURE && L >= 2) ? 2 * L + 1 : ncart(L);
 };
 
+// Nonzero entries of the canonical-Cartesian -> AO transforms, known at compile
+// time (the coefficients come from memory): a Cartesian AO is one scaled
+// component (order: source/constants.F90:34-60); the pure AO m = o - L has the
+// components x^a y^b z^c with a + b = |m|, |m| + 2, .. and b odd exactly for m < 0.
+template <int L, bool PURE>
+__host__ __device__ constexpr bool xf_nonzero(int o, int i) {
+  if (!PURE) {
+    constexpr int ord2[6] = {0, 3, 5, 1, 2, 4}, ord3[10] = {0, 6, 9, 1, 2, 3, 7, 5, 8, 4};
+    return i == (L == 2 ? ord2[o % 6] : ord3[o % 10]);
+  }
+  const int m = o - L, am = m < 0 ? -m : m, xy = c_lx(L, i) + c_ly(L, i);
+  return xy >= am && (xy - am) % 2 == 0 && (c_ly(L, i) % 2 == 1) == (m < 0);
+}
+
 // AO transform of one index of a 4-index block, in place: V is viewed as
 // [LEFT][NI][RIGHT] on input and [LEFT][NO][RIGHT] on output (NO <= NI).
 // Each (l, r) line is read completely before it is written, in increasing l,
 // so no write lands on an unread input: within one l the lines differ in r,
-// and the outputs of line l end below the first input of line l+1.
+// and the outputs of line l end below the first input of line l+1.  Only the
+// nonzero coefficients take part (9 of 30 for a pure d index, 19 of 70 for f).
 template <int L, bool PURE, int LEFT, int RIGHT, typename R>
 __device__ __forceinline__ void xform_inplace(const double* __restrict__ xf, R* V) {
   constexpr int NI = ncart(L), NO = AO<L, PURE>::N;
@@ -56,16 +71,16 @@ __device__ __forceinline__ void xform_inplace(const double* __restrict__ xf, R* 
       R t[NI];
 #pragma unroll
       for (int i = 0; i < NI; ++i) t[i] = V[(l * NI + i) * RIGHT + r];
-#pragma unroll
-      for (int o = 0; o < NO; ++o) {
+      sfor<NO>([&](auto Oi) {
+        constexpr int o = OQPH_CI(Oi);
         R s = 0;
-#pragma unroll
-        for (int i = 0; i < NI; ++i) {
-          const double c = xf[(((L - 2) * 2 + (PURE ? 1 : 0)) * 10 + o) * 10 + i];
-          s += (R)c * t[i];
-        }
+        sfor<NI>([&](auto Ii) {
+          constexpr int i = OQPH_CI(Ii);
+          if constexpr (xf_nonzero<L, PURE>(o, i))
+            s += (R)xf[(((L - 2) * 2 + (PURE ? 1 : 0)) * 10 + o) * 10 + i] * t[i];
+        });
         V[(l * NO + o) * RIGHT + r] = s;
-      }
+      });
     }
 }
 

@@ -53,6 +53,7 @@ bool kernels_support(int lmax);
 bool jk_template(int la, int lb, int lc, int ld);
 bool grad_template(int la, int lb, int lc, int ld);
 HLDims hl_dims(int la, int lb, int lc, int ld, int pure, int grad, int natm);
+bool launch_jkc(int la, int lb, int lc, int ld, bool pure, const JKParams& p, const WaveWork& ww, hipStream_t s);
 void launch_jkh(const HLDims& h, const JKParams& p, const WaveWork& ww, hipStream_t s);
 void launch_jkh_multi(const JKParams& p, const HLTaskList& tl, long long nblocks, int lds, hipStream_t s);
 void launch_schwarzh(const HLDims& h, const ShellPair* pairs, const PrimJK* prims, const int* list, int n,
@@ -246,6 +247,7 @@ struct oqph_session {
   std::map<int, std::unique_ptr<ChunkSet>> chunksets;  // key: bra class * 16 + cap
   int jkg_mode = 1;  // OQPH_JKG: 0 = segmented bra-row kernel only, 1 = default class pairs, 2 = all
   int jkg_cap = 0;   // OQPH_JKG_CAP: at most this many members per chunk (0: the kernel's)
+  int jkc_mode = 1;  // OQPH_JKC: 0 = no cooperative kernel, 1 = jkc_class(), 2 = every class that has one
   int jkt_mode = 0;  // OQPH_JKT: 0 (default) = no tiles, 1 = (ps|ps), 2 = every class pair with a tiled kernel
   struct WLaunch {
     int la, lb, lc, ld;
@@ -254,6 +256,7 @@ struct oqph_session {
     ChunkView cv{};
     bool rows;   // bra-row kernel (bw, cm, lds) instead of wavefront tasks (ww)
     bool hl;     // run-time-class kernel on the wavefront tasks (f shells), layout hd
+    bool coop = false;  // cooperative kernel (k_jkc) on the wavefront tasks
     HLDims hd;
     WaveWork ww;   // the list pointers are set per build (bind_lists)
     BraWork bw;
@@ -815,6 +818,8 @@ static int prepare_geometry(oqph_session* s) {
     s->hl_multi = (hm && hm[0] == '0') ? 0 : 1;
     const char* g = getenv("OQPH_JKG");
     s->jkg_mode = (g && (g[0] == '0' || g[0] == '2')) ? g[0] - '0' : 1;
+    const char* jc = getenv("OQPH_JKC");
+    s->jkc_mode = (jc && (jc[0] == '0' || jc[0] == '2')) ? jc[0] - '0' : 1;
     const char* jt = getenv("OQPH_JKT");
     s->jkt_mode = (jt && (jt[0] == '1' || jt[0] == '2')) ? jt[0] - '0' : 0;
     const char* gc = getenv("OQPH_JKG_CAP");
@@ -963,12 +968,12 @@ static int prepare_attenuated(oqph_session* s, double mu) {
 // launch of few 64-ket chunks (a small molecule's f or (dd|dd) classes) would
 // leave most of the device idle; such launches split each chunk over 2, 4 or
 // 8 blocks until they have two rounds of resident blocks.
-static int hl_kpb(const oqph_session* s, long long chunks, int lds) {
+static int hl_kpb(const oqph_session* s, long long chunks, int lds, int least = 1) {
   if (s->hl_kpb > 0) return s->hl_kpb;
   const long long per_cu = std::min<long long>(16, (long long)(s->lds_max / (size_t)std::max(lds, 1)));
   const long long target = 2 * std::max<long long>(per_cu, 1) * s->ncu;
   int kpb = 64;
-  while (kpb > 8 && chunks * (64 / kpb) < target) kpb /= 2;
+  while (kpb > least && chunks * (64 / kpb) < target) kpb /= 2;
   return kpb;
 }
 
@@ -1275,6 +1280,30 @@ static int prepare_grad(oqph_session* s) {
   return 0;
 }
 
+// Class pairs on the cooperative kernel k_jkc, by the Cartesian components of
+// a quartet and the quartets of the launch (measured alone on the device, FP64,
+// per-lane template or run-time-class kernel -> k_jkc):
+//   above 150: always.  The run-time classes gain 5-14x ((fd|dd) 14.7 -> 1.06
+//     ms, (dp|dp) + (dd|pp) 39.5 -> 5.3 ms), the spilling templates 1.5-4x
+//     ((dp|pp) 44.2 -> 16.4, (dd|ds) 13.1 -> 3.1, (fs|dp) 16.3 -> 4.7, (fd|ps)
+//     10.6 -> 7.2 ms).
+//   100 .. 150 ((fs|fs), (dp|ds), (dd|ps)): below about 1500 quartets per CU,
+//     where the template's few wavefronts wait on its spills ((dd|ps) 2.5e5
+//     quartets 1.11 -> 0.81 ms); above, the template wins ((dd|ps) 5.3e6 quartets
+//     7.5 vs 13.6 ms).  (fs|fs), ten by ten on both sides, gains there too (2.6 -> 1.7).
+//   30 .. 100 ((pp|pp), (ds|pp), (dp|ps), (ds|ds), ..): below 16 quartets per CU
+//     ((pp|pp), 6 quartets: 0.110 -> 0.087 ms; 1.8e7 quartets: 9.7 vs 29.6 ms).
+static bool jkc_class(const oqph_session* s, int la, int lb, int lc, int ld, bool two, long long quartets,
+                      KernelRes* r) {
+  if (s->jkc_mode == 0 || (s->jk_hl_ng == 0 && jk_template(la, lb, lc, ld))) return false;
+  if (!kernel_resources(7 | (two ? 16 : 0), la, lb, lc, ld, s->pure, r) || r->private_bytes > OQPH_PRIVATE_BUDGET)
+    return false;
+  if (s->jkc_mode == 2) return true;
+  const int nc = ncart(la) * ncart(lb) * ncart(lc) * ncart(ld);
+  if (nc > 150 || (la == 3 && lc == 3)) return true;
+  return quartets < (long long)s->ncu * (nc >= 100 ? 1500 : 16);
+}
+
 // Wavefront tasks for a given maxden.  For bra pair p and ket bucket b the
 // kets that survive Q_bra Q_ket 4 maxD >= c form a prefix of the bucket; for a
 // class with itself each unordered pair is taken once (the bra is the later
@@ -1298,6 +1327,8 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
     size_t lds = 0;
     bool drows = false;
     bool hl = false;  // run-time-class kernel (k_jkh)
+    bool coop = false;  // cooperative kernel (k_jkc), its static LDS
+    int coop_lds = 0;
     bool grouped = false;  // grouped bra-row kernel (k_jkg) on chunk set cv
     bool tiled = false;    // tiled form of k_jkg (tiles in h_items)
     ChunkView cv{};
@@ -1359,14 +1390,17 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
       // run-time-class kernel for the f classes without a class template
       // templates whose private segment exceeds the budget run on k_jkh instead
       KernelRes kr0{}, kr1{};
-      const bool tmpl = !s->general && jk_template(la, lb, lc, ld) && !(!s->f_templates && (la == 3 || lc == 3)) &&
+      KernelRes krc{};
+      const bool coop = !s->general && !(!s->f_templates && (la == 3 || lc == 3)) &&
+                        jkc_class(s, la, lb, lc, ld, two, nket, &krc);
+      const bool tmpl = !s->general && !coop && jk_template(la, lb, lc, ld) && !(!s->f_templates && (la == 3 || lc == 3)) &&
                         !(s->jk_hl_ng > 0 && ncart(la) * ncart(lb) * ncart(lc) * ncart(ld) > s->jk_hl_ng);
       const int variant = two ? 16 : 0;  // the open-shell kernels when two
       const bool fit0 = tmpl && kernel_resources(0 | variant, la, lb, lc, ld, s->pure, &kr0) &&
                         kr0.private_bytes <= OQPH_PRIVATE_BUDGET;
       const bool fit1 = tmpl && kernel_resources(1 | variant, la, lb, lc, ld, s->pure, &kr1) &&
                         kr1.private_bytes <= OQPH_PRIVATE_BUDGET;
-      const bool hl = !fit0 && !fit1;
+      const bool hl = !coop && !fit0 && !fit1;
       bool rows = fit1 && s->rows_mode > 0 && jkb_info(la, lb, lc, ld, s->pure, &nrow, &slds, s->lds_max);
       // dynamic LDS: K rows (nrow x ncol), plus D rows (nrow x ncol) and the
       // bra rows of dsh (2 x nsh) when those fit as well; the open-shell
@@ -1592,7 +1626,7 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
         pend.push_back(q);
         continue;
       }
-      if (!fit0 && !hl) {
+      if (!fit0 && !hl && !coop) {
         set_err("class (%d %d|%d %d): its bra-row kernel does not fit in LDS and its wavefront kernel exceeds the "
                 "private-segment budget", la, lb, lc, ld);
         return 1;
@@ -1626,6 +1660,8 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
       s->h_choff.push_back(waves);  // terminator of this launch's prefix
       pend.push_back({la, lb, lc, ld, ck, seg0, ch0, nseg, waves});
       pend.back().hl = hl;
+      pend.back().coop = coop;
+      pend.back().coop_lds = krc.lds_bytes;
       pend.back().slots = 64ll * waves;
     }
   for (auto& p : pend) {
@@ -1662,6 +1698,9 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
     L.ww.nseg = p.nseg;
     L.ww.nwaves = p.nwaves;
     L.hl = p.hl;
+    L.coop = p.coop;
+    // at least four kets per block: a wavefront takes up to four at a time
+    if (L.coop) L.ww.kpb = hl_kpb(s, L.ww.nwaves, p.coop_lds, 4);
     if (L.hl) {
       L.hd = hl_dims(p.la, p.lb, p.lc, p.ld, s->pure, 0, 0);
       if ((size_t)L.hd.lds > s->lds_max) {
@@ -1988,6 +2027,7 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
     bool ok = true;
     if (L.multi) launch_jkh_multi(p, L.tl, L.nblocks, (int)L.lds, ls);
     else if (L.hl) launch_jkh(L.hd, p, L.ww, ls);
+    else if (L.coop) ok = launch_jkc(L.la, L.lb, L.lc, L.ld, s->pure, p, L.ww, ls);
     else if (L.grouped) ok = launch_jkg(L.la, L.lb, L.lc, L.ld, s->pure, p, L.bw, L.cm, L.cv, L.lds, ls);
     else if (L.tiled) ok = launch_jkt(L.la, L.lb, L.lc, L.ld, s->pure, p, L.bw, L.cm, L.cv, L.lds, ls);
     else if (L.rows) ok = launch_jkb(L.la, L.lb, L.lc, L.ld, s->pure, p, L.bw, L.cm, L.lds, ls);
@@ -2337,7 +2377,7 @@ int oqph_last_profile(oqph_session* s, int maxn, int* cls, double* ms, double* f
     const unsigned long long* c = i * 8 + 8 <= (int)s->prof_ctr.size() ? &s->prof_ctr[8 * i] : nullptr;
     // a multi-class launch reports 40000 + its number of classes
     if (cls) cls[i] = L.multi ? 40000 + L.ntask
-                              : (L.tiled ? 60000 : L.hl ? 20000 : L.grouped ? 30000 : L.rows ? 10000 : 0) +
+                              : (L.coop ? 80000 : L.tiled ? 60000 : L.hl ? 20000 : L.grouped ? 30000 : L.rows ? 10000 : 0) +
                                     L.la * 1000 + L.lb * 100 +
                                     L.lc * 10 + L.ld;
     if (ms) ms[i] = i < (int)s->prof_ms.size() ? s->prof_ms[i] : 0.0;
