@@ -58,14 +58,14 @@ def _cost(c):
 
 # headers each translation unit depends on (cache key = unit + these + flags)
 DEPS = {
-    "jk_class.hip": ["jk_device.h", "jkg_device.h", "eri_device.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
-    "jkc_class.hip": ["jkc_device.h", "jk_device.h", "eri_device.h", "oqph_common.h", "rys_table.inc",
+    "jk_class.hip": ["jk_device.h", "jkg_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
+    "jkc_class.hip": ["jkc_device.h", "jk_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                       "rys_table_f32.inc"],
-    "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
+    "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "session.hip": ["oqph_common.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
-    "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "rys_table.inc", "rys_table_f32.inc"],
-    "int1e.hip": ["../../include/oqph.h", "ao_xform.h", "rys_table.inc", "rys_table_f32.inc"],
-    "hl.hip": ["hl_device.h", "jk_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "rys_table.inc",
+    "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
+    "int1e.hip": ["../../include/oqph.h", "ao_xform.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
+    "hl.hip": ["hl_device.h", "jk_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                "rys_table_f32.inc"],
     "sigma.hip": ["../../include/oqph.h"],
     "xc.hip": ["../../include/oqph.h", "ao_xform.h", "session_view.h"],

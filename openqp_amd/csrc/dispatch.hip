@@ -1,6 +1,7 @@
 // dispatch.hip -- class dispatch of the J/K and Schwarz kernels, the small
 // per-build kernels, and the host copies of the Rys tables.
 #define OQPH_WANT_RYS_DATA
+#include <vector>
 #include "eri_device.h"
 #include "grad_device.h"
 
@@ -384,6 +385,31 @@ __global__ void k_jscatter(const ShellPair* pairs, const int* joff, int npair, i
     }
 }
 
+// The per-pair inputs of a J/K build in device-pair order (JKParams::Dk, dpm),
+// and the ket-side Coulomb buffer cleared
+__global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, int pure, const double* D,
+                          const double* dsh, int nsh, double* Dk, double* dpm, double* Jk) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npair) return;
+  const ShellPair P = pairs[i];
+  const int na = (pure && P.la >= 2) ? 2 * P.la + 1 : (P.la + 1) * (P.la + 2) / 2;
+  const int nb = (pure && P.lb >= 2) ? 2 * P.lb + 1 : (P.lb + 1) * (P.lb + 2) / 2;
+  const int o = joff[i];
+  for (int a = 0; a < na; ++a)
+    for (int b = 0; b < nb; ++b) {
+      Dk[o + a * nb + b] = D[tri_idx_(P.ao_a + a, P.ao_b + b)];
+      Jk[o + a * nb + b] = 0.0;
+    }
+  dpm[i] = dsh[(long long)P.si * nsh + P.sj];
+}
+
+void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
+                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s) {
+  if (npair <= 0) return;
+  hipLaunchKernelGGL(k_dgather, dim3((unsigned)((npair + 63) / 64)), dim3(64), 0, s, pairs, joff, npair, pure ? 1 : 0,
+                     D, dsh, nsh, Dk, dpm, Jk);
+}
+
 void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* Jk, double* F,
                      hipStream_t s) {
   if (npair <= 0) return;
@@ -396,13 +422,24 @@ void launch_max_reduce(const double* x, long long n, unsigned long long* out, hi
 }
 
 
+// the Rys table followed by the Boys table (QTab offsets)
 const double* rys_table_host(size_t* n) {
-  *n = RYS_TABLE_SIZE;
-  return RYS_TABLE;
+  static const std::vector<double> t = [] {
+    std::vector<double> v(RYS_TABLE, RYS_TABLE + RYS_TABLE_SIZE);
+    v.insert(v.end(), BOYS_TABLE, BOYS_TABLE + BOYS_TABLE_SIZE);
+    return v;
+  }();
+  *n = t.size();
+  return t.data();
 }
 const float* rys32_table_host(size_t* n) {
-  *n = RYS32_TABLE_SIZE;
-  return RYS32_TABLE;
+  static const std::vector<float> t = [] {
+    std::vector<float> v(RYS32_TABLE, RYS32_TABLE + RYS32_TABLE_SIZE);
+    v.insert(v.end(), BOYS32_TABLE, BOYS32_TABLE + BOYS32_TABLE_SIZE);
+    return v;
+  }();
+  *n = t.size();
+  return t.data();
 }
 const double* rys_herm_host(size_t* n) {
   *n = sizeof(RYS_HERM) / sizeof(double);

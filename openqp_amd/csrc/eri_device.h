@@ -57,9 +57,11 @@ __device__ __forceinline__ void sfor(F&& f) {
 #define OQPH_CI(x) decltype(x)::value
 
 // ------------------------------------------------------------------ FP64 rcp
-// Hardware reciprocal / reciprocal square root seeds refined by two Newton
-// steps (quadratic convergence from the seed's ~2^-22 to full precision);
-// arguments are positive normal numbers (exponent sums, Boys arguments).
+// Hardware reciprocal / reciprocal square root seeds (relative error about
+// 2^-22) refined to full precision: two Newton steps for the reciprocal, one
+// third-order step (residual e^3, 2^-64) for the reciprocal square root, two
+// operations shorter than two Newton steps; arguments are positive normal
+// numbers (exponent sums, Boys arguments).
 __device__ __forceinline__ double rcp64(double x) {
   double y = __builtin_amdgcn_rcp(x);
   double e = fma(-x, y, 1.0);
@@ -68,12 +70,9 @@ __device__ __forceinline__ double rcp64(double x) {
   return fma(y, e, y);
 }
 __device__ __forceinline__ double rsq64(double x) {
-  const double h = 0.5 * x;
-  double y = __builtin_amdgcn_rsq(x);
-  double e = fma(-h * y, y, 0.5);
-  y = fma(y, e, y);
-  e = fma(-h * y, y, 0.5);
-  return fma(y, e, y);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);  // 1 - x y^2
+  return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
 // Load a primitive pair whose index is uniform across the wavefront through
@@ -115,6 +114,78 @@ __device__ __forceinline__ PrimPair load_uniform(const PrimPair* p, int i) {
 // ------------------------------------------------------------------ Rys roots
 #include "rys_table.inc"
 #include "rys_table_f32.inc"
+
+// ------------------------------------------------------------ Boys functions
+// The Boys tables follow the Rys tables in the device buffers.
+#include "boys_table.inc"
+
+// F[0..M], M <= 3, at T.  tab: the m0 = max(M - 1, 0) block of the table,
+// rows of one polynomial in u = T_k - T around the nearest grid point T_k =
+// k/2, whose value is F_m0 and whose derivative is F_m0+1; the lower orders
+// follow from e^-T = (2 m0 + 1) F_m0 - 2 T F_m0+1 and the downward recursion.
+// One row is 12 (FP64) or 8 (FP32) coefficients, against 26 (14) for a root
+// and weight of the Rys fits and 52 (28) for two.  The step of 1/2 is a
+// balance: 1/4 needs two coefficients less but 5 KB more LDS per block, which
+// costs (ps|ss) its third block per CU.
+template <int M, typename R>
+__device__ __forceinline__ void boys(R T, const R* __restrict__ tab, R (&F)[M + 1]) {
+  constexpr bool F32 = sizeof(R) == 4;
+  constexpr int m0 = M > 0 ? M - 1 : 0, deg = F32 ? BOYS32_DEG : BOYS_DEG;
+  if (T >= (R)BOYS_TMAX[m0]) {
+    const R rs = F32 ? (R)__builtin_amdgcn_rsqf((float)T) : (R)rsq64((double)T);
+    F[0] = (R)0.88622692545275801364 * rs;
+    const R h = (R)0.5 * rs * rs;
+#pragma unroll
+    for (int m = 1; m <= M; ++m) F[m] = (R)(2 * m - 1) * h * F[m - 1];
+    return;
+  }
+  // nearest multiple of 1/2: adding 1.5 2^51 (2^22) leaves an ulp of 1/2, and
+  // the low bits of the sum count halves
+  R Tk;
+  int k;
+  if constexpr (F32) {
+    const float x = (float)T + 6291456.0f;
+    k = __float_as_int(x) & 0x3ff;
+    Tk = x - 6291456.0f;
+  } else {
+    const double x = (double)T + 3377699720527872.0;
+    k = __double2loint(x) & 0x3ff;
+    Tk = x - 3377699720527872.0;
+  }
+  const R u = Tk - T;
+  R c[deg + 1];
+  // rows are 16-byte aligned
+  typedef typename std::conditional<F32, float4, double2>::type V;
+  constexpr int nv = 16 / sizeof(R);
+  const V* r = (const V*)(tab + k * (deg + 1));
+#pragma unroll
+  for (int j = 0; j <= deg; j += nv) {
+    const V t = r[j / nv];
+    c[j] = t.x;
+    c[j + 1] = t.y;
+    if constexpr (F32) {
+      c[j + 2] = t.z;
+      c[j + 3] = t.w;
+    }
+  }
+  R v = c[deg], d = c[deg];
+  v = v * u + c[deg - 1];
+#pragma unroll
+  for (int j = deg - 2; j >= 0; --j) {
+    if (M > 0) d = d * u + v;
+    v = v * u + c[j];
+  }
+  F[m0] = v;
+  if constexpr (M > 0) {
+    F[M] = d;
+    if constexpr (M > 1) {
+      const R T2 = T + T;
+      const R e = (R)(2 * m0 + 1) * v - T2 * d;
+#pragma unroll
+      for (int m = m0; m > 0; --m) F[m - 1] = (T2 * F[m] + e) * (R)(1.0 / (2 * m - 1));
+    }
+  }
+}
 
 // length of the N-root block of each table (entries); the blocks start at
 // RYS_OFF[N] / RYS32_OFF[N]
@@ -271,6 +342,93 @@ __host__ __device__ constexpr long long flops_grad_prim_rt(int LA, int LB, int L
                           6 * (LA + 2) * (LB + 2) * (LC + 2) * (LD + 1) + 3 * 4 * nc);
 }
 
+// Classes whose total angular momentum is at most 3: the (e0|f0) integrals
+// come from F_0..F_3 by the Obara-Saika vertical recursion (J. Chem. Phys. 84,
+// 3963 (1986)) instead of one or two Rys roots.  What bounds these classes is
+// the instructions per primitive quartet (lane divergence apart) and the LDS
+// reads of the fit; the recursion needs 2-6 Boys values from one table row and,
+// for (ps|ps), 33 operations instead of the 90 of two roots.
+template <int LA, int LB, int LC, int LD>
+constexpr bool use_os() {
+  return LA + LB + LC + LD <= 3;
+}
+// The class's table block: Boys functions or Rys roots (offset in the device
+// buffers, length; in doubles / floats).
+template <int LA, int LB, int LC, int LD>
+struct QTab {
+  static constexpr bool os = use_os<LA, LB, LC, LD>();
+  static constexpr int NR = Dims<LA, LB, LC, LD>::NROOT;
+  static constexpr int L = LA + LB + LC + LD, m0 = os ? (L > 0 ? L - 1 : 0) : 0;
+  static constexpr int off64 = os ? RYS_TABLE_SIZE + BOYS_OFF[m0] : RYS_OFF[NR];
+  static constexpr int len64 = os ? BOYS_OFF[m0 + 1] - BOYS_OFF[m0] : rys_len<NR>();
+  static constexpr int off32 = os ? RYS32_TABLE_SIZE + BOYS32_OFF[m0] : RYS32_OFF[NR];
+  static constexpr int len32 = os ? BOYS32_OFF[m0 + 1] - BOYS32_OFF[m0] : rys32_len<NR>();
+};
+
+// Recursion axis of component (x, y, z): an exponent of one where there is
+// one (no (n - 1) term), else the first nonzero
+__host__ __device__ constexpr int os_axis(int x, int y, int z) {
+  return x == 1 ? 0 : y == 1 ? 1 : z == 1 ? 2 : x ? 0 : y ? 1 : 2;
+}
+
+// Adds pref (e0|f0) of one primitive quartet to acc from pF[m] = pref F_m.
+// Ket classes of these classes have LCD <= 1 (the bra class is never the
+// smaller one).  WP = W - P = -rz PQ, WQ = W - Q = re PQ.
+template <int LA, int LB, int LC, int LD, typename R>
+__device__ __forceinline__ void os_add(const R (&PA)[3], const R (&QC)[3], const R (&PQ)[3], R rz, R re, R h2z, R h2ze,
+                                       const R (&pF)[LA + LB + LC + LD + 1],
+                                       R (&acc)[Dims<LA, LB, LC, LD>::NE][Dims<LA, LB, LC, LD>::NF]) {
+  constexpr int LAB = LA + LB, LCD = LC + LD, M = LAB + LCD, NC = ncum(LAB), E0 = ncum(LA - 1);
+  static_assert(LCD <= 1 && M <= 3, "os_add: class out of range");
+  R E[M + 1][NC], WP[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) WP[d] = -rz * PQ[d];
+#pragma unroll
+  for (int m = 0; m <= M; ++m) E[m][0] = pF[m];
+  sfor<NC>([&](auto Ei) {
+    constexpr int e = OQPH_CI(Ei);
+    if constexpr (e > 0) {
+      constexpr int L = range_level<0>(e), c = range_local<0>(e);
+      constexpr int x = c_lx(L, c), y = c_ly(L, c), z = c_lz(L, c), ax = os_axis(x, y, z);
+      constexpr int n = (ax == 0 ? x : ax == 1 ? y : z) - 1;  // exponent of the lower component
+      constexpr int lo = range_index<0>(L - 1, c_idx(x - (ax == 0), y - (ax == 1), z - (ax == 2)));
+      constexpr int lo2 = n > 0 ? range_index<0>(L - 2, c_idx(x - 2 * (ax == 0), y - 2 * (ax == 1), z - 2 * (ax == 2))) : 0;
+      sfor<M - L + 1>([&](auto Mi) {
+        constexpr int m = OQPH_CI(Mi);
+        R v = PA[ax] * E[m][lo];
+        v = WP[ax] * E[m + 1][lo] + v;
+        if constexpr (n > 0) v = (R)n * h2z * (E[m][lo2] - rz * E[m + 1][lo2]) + v;
+        E[m][e] = v;
+      });
+    }
+  });
+  if constexpr (LCD == 0) {
+#pragma unroll
+    for (int e = 0; e < Dims<LA, LB, LC, LD>::NE; ++e) acc[e][0] += E[0][E0 + e];
+  } else {
+    // |p_i): QC_i (e|^(0) + WQ_i (e|^(1) + e_i / (2 (zeta + eta)) (e - 1_i|^(1)
+    R WQ[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) WQ[d] = re * PQ[d];
+    sfor<Dims<LA, LB, LC, LD>::NE>([&](auto Ei) {
+      constexpr int e = OQPH_CI(Ei) + E0;
+      constexpr int L = range_level<0>(e), c = range_local<0>(e);
+      sfor<3>([&](auto Di) {
+        constexpr int d = OQPH_CI(Di), n = c_l(L, c, d);
+        // component order of a p shell: x, y, z
+        R v = acc[OQPH_CI(Ei)][d];
+        v = QC[d] * E[0][e] + v;
+        v = WQ[d] * E[1][e] + v;
+        if constexpr (n > 0) {
+          constexpr int lo = range_index<0>(L - 1, c_idx(c_lx(L, c) - (d == 0), c_ly(L, c) - (d == 1), c_lz(L, c) - (d == 2)));
+          v = (R)n * h2ze * E[1][lo] + v;
+        }
+        acc[OQPH_CI(Ei)][d] = v;
+      });
+    });
+  }
+}
+
 // The fields of a primitive pair that the quadrature reads, in one precision:
 // X is the product centre relative to the pair's first centre.
 template <typename R>
@@ -296,7 +454,7 @@ __device__ __forceinline__ void rys_add(const PrimV<R>& pp, const PrimV<R>& qq, 
 // classes have no registers to spare.
 template <int LA, int LB, int LC, int LD, typename R>
 constexpr bool hoist_ket() {
-  return sizeof(R) == 4 && Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF <= 9;
+  return use_os<LA, LB, LC, LD>() || (sizeof(R) == 4 && Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF <= 9);
 }
 template <int LA, int LB, int LC, int LD, typename R>
 __device__ __forceinline__ void ket_offset(const R (&AC)[3], const PrimV<R>& qq, R (&AQ)[3]) {
@@ -321,6 +479,16 @@ __device__ __forceinline__ bool rys_accumulate(const PrimV<R>& pp, const PrimV<R
   constexpr bool F32 = sizeof(R) == 4;
   const R zeta = pp.g, eta = qq.g;
   const R fqz = pp.Kg * qq.Kg;
+  if constexpr (use_os<LA, LB, LC, LD>()) {
+    // (1 + eta / mu^2) is constant over the bra primitives, and the survivors
+    // need the prefactor anyway: it is screened itself
+    const R ze = zeta * ((R)1 + eta * imu2) + eta;
+    const R sq = F32 ? (R)__builtin_amdgcn_rsqf((float)ze) : (R)rsq64((double)ze);
+    const R pref = fqz * sq;
+    if (pref * pref < qcut2) return false;
+    rys_add<LA, LB, LC, LD, R>(pp, qq, AQ, ze, sq, sq * sq, pref, tabN, tab32N, acc);
+    return true;
+  }
   const R ze = zeta + eta + zeta * eta * imu2;
   if (fqz * fqz < qcut2 * ze) return false;
   // 1/sqrt(ze) and its square: one transcendental (FP32: hardware rsq)
@@ -354,6 +522,15 @@ __device__ __forceinline__ void rys_add(const PrimV<R>& pp, const PrimV<R>& qq, 
   const R T = rho * pq2;
   // rho/zeta = eta/(zeta+eta), rho/eta = zeta/(zeta+eta): no further divisions
   const R rz = eta * ize, re = zeta * ize;
+  if constexpr (use_os<LA, LB, LC, LD>()) {
+    R F[LAB + LCD + 1];
+    if constexpr (F32) boys<LAB + LCD, R>(T, tab32N, F);
+    else boys<LAB + LCD, R>(T, tabN, F);
+#pragma unroll
+    for (int m = 0; m <= LAB + LCD; ++m) F[m] *= pref;
+    os_add<LA, LB, LC, LD, R>(PA, QC, PQ, rz, re, pp.h, (R)0.5 * ize, F, acc);
+    return;
+  }
   const R h2z = pp.h, h2e = qq.h, h2ze = (R)0.5 * ize;
   // one root: 2D integrals G_d(i, k) by the vertical recursion, then the
   // (e0|f0) products

@@ -217,25 +217,24 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
         if (fabs(qq.Kg) < qcut) continue;
         R AQ[3];
         ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
+        // the bra records come in decreasing |K|: once K_ab^2 K_cd^2 < qcut^2 eta
+        // (eta <= zeta + eta), no later one passes the primitive screen
+        const R stop = qcut2 * qq.g;
         auto run = [&](auto bra) {
-          for (int ip = 0; ip < nit; ip += nb)
-            nprim_used +=
-                rys_accumulate<LA, LB, LC, LD, R>(bra(ip + sb), qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
+          for (int ip = 0; ip < nit; ip += nb) {
+            const PrimV<R> pp = bra(ip + sb);
+            const R fq = pp.Kg * qq.Kg;
+            if (fq * fq < stop) break;
+            nprim_used += rys_accumulate<LA, LB, LC, LD, R>(pp, qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
+          }
         };
-        if constexpr (F32) {
-          if (sbra32) run([&](int i) { return sbra32[i]; });
-          else run([&](int i) { return prim_v<float>(sbra[i]); });
-        } else {
-          run([&](int i) { return sbra[i]; });
-        }
+        // (the classes with an FP32 copy of the bra records always have it in
+        // the mixed mode, the only one with an FP32 path)
+        if constexpr (F32 && Dm::NE * Dm::NF <= 4) run([&](int i) { return sbra32[i]; });
+        else if constexpr (F32) run([&](int i) { return prim_v<float>(sbra[i]); });
+        else run([&](int i) { return sbra[i]; });
       }
     };
-    // the smallest classes keep a loop of their own for unsplit kets, whose
-    // bra records are uniform LDS reads (the shared loop costs them 1 %)
-    if (Dm::NE * Dm::NF <= 9 && sp.n == 1) {
-      walk(0, 0, 1, 1, npp);
-      return;
-    }
     walk(sp.sb, sp.sk, nb, nk, nit);
     if (sp.n > 1) split_sum(acc, sp.n);
     return;
@@ -409,13 +408,13 @@ __device__ __forceinline__ void count_wave(unsigned long long* ctr, bool pred) {
     atomicAdd(ctr, (unsigned long long)__popcll(m));
 }
 
-// Root tables of the class's root count are copied into LDS once per block
+// The class's block of the Boys or root tables is copied into LDS once per block
 // when they fit (FP64 for up to 3 roots, FP32 for every class that has an
 // FP32 path): the table lookups are per-lane gathers at random intervals,
 // which LDS serves at a fraction of the vector-memory cost.
-template <int NR>
+template <int LA, int LB, int LC, int LD>
 struct RysLds {
-  static constexpr bool f64 = rys_len<NR>() * 8 <= 36 * 1024;
+  static constexpr bool f64 = QTab<LA, LB, LC, LD>::len64 * 8 <= 36 * 1024;
 };
 
 // TWO: the open-shell pass (prm.D2 / prm.F2 set), compiled separately so the
@@ -423,19 +422,19 @@ struct RysLds {
 template <int LA, int LB, int LC, int LD, bool PURE, bool TWO>
 __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
   using Dm = Dims<LA, LB, LC, LD>;
-  constexpr int NR = Dm::NROOT;
-  constexpr bool T64 = RysLds<NR>::f64 && !Big<LA, LB, LC, LD>::value;
+  using QT = QTab<LA, LB, LC, LD>;
+  constexpr bool T64 = RysLds<LA, LB, LC, LD>::f64 && !Big<LA, LB, LC, LD>::value;
   constexpr bool T32 = Dm::NE * Dm::NF <= 256 && !Big<LA, LB, LC, LD>::value;  // classes with an FP32 path
-  __shared__ double s_t64[T64 ? rys_len<NR>() : 1];
-  __shared__ float s_t32[T32 ? rys32_len<NR>() : 1];
+  __shared__ __align__(16) double s_t64[T64 ? QT::len64 : 1];
+  __shared__ __align__(16) float s_t32[T32 ? QT::len32 : 1];
   if constexpr (T64)
-    for (int i = threadIdx.x; i < rys_len<NR>(); i += blockDim.x) s_t64[i] = prm.rys[RYS_OFF[NR] + i];
+    for (int i = threadIdx.x; i < QT::len64; i += blockDim.x) s_t64[i] = prm.rys[QT::off64 + i];
   if constexpr (T32)
     if (prm.mixed)
-      for (int i = threadIdx.x; i < rys32_len<NR>(); i += blockDim.x) s_t32[i] = prm.rys32[RYS32_OFF[NR] + i];
+      for (int i = threadIdx.x; i < QT::len32; i += blockDim.x) s_t32[i] = prm.rys32[QT::off32 + i];
   __syncthreads();
-  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + RYS_OFF[NR];
-  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + RYS32_OFF[NR];
+  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + QT::off64;
+  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + QT::off32;
 
   // one wavefront = one chunk of 64 kets of one segment; the bra is uniform
   const long long wave = __builtin_amdgcn_readfirstlane(
@@ -457,7 +456,7 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
   double bound = 0.0;
   bool mine = true;  // the quartet belongs to this share (OpenQP's MPI split, int2.F90:759-761)
   if (active) {
-    iq = ww.ket[ww.seg_k0[seg] + k];
+    iq = ww.kofs + ww.seg_k0[seg] + k;  // the class lists are consecutive device pairs
     Q = prm.pairs[iq];
     // ---- OpenQP screening (int2.F90:763-800)
     const bool p_first = (P.si > Q.si) || (P.si == Q.si && P.sj >= Q.sj);
@@ -465,7 +464,7 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
     const double qbra = p_first ? P.Q : Q.Q;
     const int n = prm.nsh;
     const double* ds = prm.dsh;
-    double dm = fmax(4.0 * ds[P.si * n + P.sj], 4.0 * ds[Q.si * n + Q.sj]);
+    double dm = 4.0 * fmax(prm.dpm[ip], prm.dpm[iq]);
     dm = fmax(dm, fmax(ds[P.sj * n + Q.sj], ds[P.sj * n + Q.si]));
     dm = fmax(dm, fmax(ds[P.si * n + Q.sj], ds[P.si * n + Q.si]));
     bound = P.Q * Q.Q * dm;
@@ -514,10 +513,9 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
 #pragma unroll
       for (int d = 0; d < OD; ++d) Dbd[b * OD + d] = Dp[tri_idx(ob + b, od + d)];
     }
+    const double* Dk = prm.Dk + ww.jbase + (long long)(iq - ww.kofs) * (OC * OD);
 #pragma unroll
-    for (int c = 0; c < OC; ++c)
-#pragma unroll
-      for (int d = 0; d < OD; ++d) Dcd[c * OD + d] = Dp[tri_idx(oc + c, od + d)];
+    for (int cd = 0; cd < OC * OD; ++cd) Dcd[cd] = Dk[cd];
     double Jcd[OC * OD], Kac[OA * OC], Kad[OA * OD], Kbc[OB * OC], Kbd[OB * OD];
 #pragma unroll
     for (int i = 0; i < OC * OD; ++i) Jcd[i] = 0.0;
@@ -713,10 +711,9 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
   // J blocks
   {
     double Dcd[OC * OD], Dab[OA * OB];
+    const double* Dk = prm.Dk + ww.jbase + (long long)(iq - ww.kofs) * (OC * OD);
 #pragma unroll
-    for (int x = 0; x < OC; ++x)
-#pragma unroll
-      for (int y = 0; y < OD; ++y) Dcd[x * OD + y] = Dp[tri_idx(oc + x, od + y)];
+    for (int cd = 0; cd < OC * OD; ++cd) Dcd[cd] = valid ? Dk[cd] : 0.0;
 #pragma unroll
     for (int x = 0; x < OA; ++x)
 #pragma unroll
@@ -855,33 +852,29 @@ struct JKB {
   // spill heavily under it)
   static constexpr int NEF = Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF;
   static constexpr int threads = NEF <= 4 ? OQPH_JKB_SMALL_THREADS : (NEF <= 9 ? 1024 : 512);
-  // (ss|ss) fits in 64 VGPRs without spilling: eight waves per SIMD;
-  // OQPH_JKB_WAVES3 sets the target for (e0|f0) sets of 2..4 ((ps|ss))
-#ifndef OQPH_JKB_WAVES3
-#define OQPH_JKB_WAVES3 1
-#endif
-  static constexpr int min_waves = (Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF == 1)  ? 8
-                                   : (Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF <= 4) ? OQPH_JKB_WAVES3
-                                                                                                 : 1;
+  // waves per SIMD the register allocation aims at: (ss|ss) 5 (96 VGPRs; 6 and
+  // 8 spill: 14.9 -> 18.5, 23.7 ms FP64 on (H2O)64/cc-pVDZ), the others
+  // unhinted ((ps|ss) 122 VGPRs, 4 waves; 5 and 6 spill: 103 -> 136, 182 ms)
+  static constexpr int min_waves = NEF == 1 ? 5 : 1;
 };
 
 template <int LA, int LB, int LC, int LD, bool PURE, bool TWO>
 __global__ __launch_bounds__((JKB<LA, LB, LC, LD>::threads))
 __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(JKParams prm, BraWork bw, ColMap cm) {
   using Dm = Dims<LA, LB, LC, LD>;
-  constexpr int NR = Dm::NROOT;
-  constexpr bool T64 = RysLds<NR>::f64;
+  using QT = QTab<LA, LB, LC, LD>;
+  constexpr bool T64 = RysLds<LA, LB, LC, LD>::f64;
   constexpr bool T32 = Dm::NE * Dm::NF <= 256;
   constexpr int OA = AO<LA, PURE>::N, OB = AO<LB, PURE>::N, OC = AO<LC, PURE>::N, OD = AO<LD, PURE>::N;
   constexpr int NROW = OA + OB, NOUT = OA * OB * OC * OD, NBLK = Dm::NBLK;
-  __shared__ double s_t64[T64 ? rys_len<NR>() : 1];
+  __shared__ __align__(16) double s_t64[T64 ? QT::len64 : 1];
   __shared__ PrimV<double> s_bra[JKB_MAX_BRA_PRIMS];
   // FP32 copy of the bra primitives for the smallest classes, whose FP32
   // quadrature is short enough that converting the FP64 copy per primitive
   // quartet shows (5 % of (ps|ss)); larger classes keep the LDS for blocks
   constexpr bool B32 = T32 && Dm::NE * Dm::NF <= 4;
   __shared__ PrimV<float> s_bra32[B32 ? JKB_MAX_BRA_PRIMS : 1];
-  __shared__ float s_t32[T32 ? rys32_len<NR>() : 1];
+  __shared__ __align__(16) float s_t32[T32 ? QT::len32 : 1];
   __shared__ double s_jab[OA * OB];
   // dynamic LDS: K rows [NROW][ncol] (accumulated); when cm.drows, also D rows
   // [NROW][ncol] (the density at the same positions) and the bra shells' rows
@@ -901,10 +894,10 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
     for (int i = threadIdx.x; i < nk; i += blockDim.x) s_k2[i] = 0.0;
   if (threadIdx.x < OA * OB) s_jab[threadIdx.x] = 0.0;
   if constexpr (T64)
-    for (int i = threadIdx.x; i < rys_len<NR>(); i += blockDim.x) s_t64[i] = prm.rys[RYS_OFF[NR] + i];
+    for (int i = threadIdx.x; i < QT::len64; i += blockDim.x) s_t64[i] = prm.rys[QT::off64 + i];
   if constexpr (T32)
     if (prm.mixed)
-      for (int i = threadIdx.x; i < rys32_len<NR>(); i += blockDim.x) s_t32[i] = prm.rys32[RYS32_OFF[NR] + i];
+      for (int i = threadIdx.x; i < QT::len32; i += blockDim.x) s_t32[i] = prm.rys32[QT::off32 + i];
   const int* item = bw.item + (size_t)blockIdx.x * (1 + OQPH_NBKT);
   const int ip = __builtin_amdgcn_readfirstlane(item[0]);
   const ShellPair P = prm.pairs[ip];
@@ -969,8 +962,8 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
     }
   }
   __syncthreads();
-  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + RYS_OFF[NR];
-  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + RYS32_OFF[NR];
+  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + QT::off64;
+  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + QT::off32;
   const PrimV<double>* sbra = bra_lds ? (const PrimV<double>*)s_bra : nullptr;
   const PrimV<float>* sbra32 = (B32 && bra_lds && prm.mixed) ? (const PrimV<float>*)s_bra32 : nullptr;
   const int nbra64 = bra_lds ? s_nbra[0] : 0, nbra32 = bra_lds ? s_nbra[1] : 0;
@@ -986,6 +979,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
   double jab[OA * OB];
 #pragma unroll
   for (int i = 0; i < OA * OB; ++i) jab[i] = 0.0;
+  const double dab_max = prm.dpm[ip];
   // per-lane statistics (32-bit; the model FLOPs follow from n_prim and n_valid)
   unsigned n_comp = 0, n_skip = 0, n_f32 = 0, n_valid = 0, n_prim = 0;
 
@@ -1003,14 +997,14 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       bool skip = true, mine = true;
       double bound = 0.0;
       if (active) {
-        iq = bw.ket[kbase + k];
+        iq = bw.kofs + kbase + k;  // the class lists are consecutive device pairs
         Q = prm.pairs[iq];
         // ---- OpenQP screening (int2.F90:763-800); the bra shells' rows of
         // the shell-pair maxima come from LDS
         const bool p_first = (P.si > Q.si) || (P.si == Q.si && P.sj >= Q.sj);
         if (prm.own) mine = prm.own[p_first ? ip : iq] != 0;
         const double qbra = p_first ? P.Q : Q.Q;
-        double dm = fmax(4.0 * prm.dsh[P.si * nsh + P.sj], 4.0 * prm.dsh[Q.si * nsh + Q.sj]);
+        double dm = 4.0 * fmax(dab_max, prm.dpm[iq]);
         if (drows) {
           dm = fmax(dm, fmax(s_ds[nsh + Q.sj], s_ds[nsh + Q.si]));
           dm = fmax(dm, fmax(s_ds[Q.sj], s_ds[Q.si]));
@@ -1071,10 +1065,9 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       // J_ab in registers; J_cd to memory
       {
         double Dcd[OC * OD];
+        const double* Dk = prm.Dk + bw.jbase + (long long)(iq - bw.kofs) * (OC * OD);
 #pragma unroll
-        for (int x = 0; x < OC; ++x)
-#pragma unroll
-          for (int y = 0; y < OD; ++y) Dcd[x * OD + y] = valid ? Dp[tri_idx(oc + x, od + y)] : 0.0;
+        for (int cd = 0; cd < OC * OD; ++cd) Dcd[cd] = valid ? Dk[cd] : 0.0;
 #pragma unroll
         for (int ab = 0; ab < OA * OB; ++ab) {
           double t = 0.0;
@@ -1098,7 +1091,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       // K rows a (0..OA-1) and b (OA..OA+OB-1) in LDS; the density in those
       // rows comes from the LDS copy at the same positions
       auto krows = [&](const double* sd, const double* __restrict__ Dg, double* sk) {
-        const int colC = cm.colidx[Q.sa], colD = cm.dofs + cm.colidx[Q.sb];
+        const int colC = Q.ca, colD = cm.dofs + Q.cb;
         double Dbd[OB * OD], Dbc[OB * OC], Dad[OA * OD], Dac[OA * OC];
         if (drows) {
 #pragma unroll
@@ -1140,7 +1133,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             for (int bb = 0; bb < OB; ++bb)
 #pragma unroll
               for (int d = 0; d < OD; ++d) t += VV(a, bb, cc, d) * Dbd[bb * OD + d];
-            if (t != 0.0) atomicAdd(&sk[a * ncol + colC + cc], ck * t);
+            atomicAdd(&sk[a * ncol + colC + cc], ck * t);
           }
 #pragma unroll
           for (int d = 0; d < OD; ++d) {
@@ -1149,7 +1142,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             for (int bb = 0; bb < OB; ++bb)
 #pragma unroll
               for (int cc = 0; cc < OC; ++cc) t += VV(a, bb, cc, d) * Dbc[bb * OC + cc];
-            if (t != 0.0) atomicAdd(&sk[a * ncol + colD + d], ck * t);
+            atomicAdd(&sk[a * ncol + colD + d], ck * t);
           }
         }
 #pragma unroll
@@ -1161,7 +1154,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             for (int a = 0; a < OA; ++a)
 #pragma unroll
               for (int d = 0; d < OD; ++d) t += VV(a, bb, cc, d) * Dad[a * OD + d];
-            if (t != 0.0) atomicAdd(&sk[(OA + bb) * ncol + colC + cc], ck * t);
+            atomicAdd(&sk[(OA + bb) * ncol + colC + cc], ck * t);
           }
 #pragma unroll
           for (int d = 0; d < OD; ++d) {
@@ -1170,7 +1163,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             for (int a = 0; a < OA; ++a)
 #pragma unroll
               for (int cc = 0; cc < OC; ++cc) t += VV(a, bb, cc, d) * Dac[a * OC + cc];
-            if (t != 0.0) atomicAdd(&sk[(OA + bb) * ncol + colD + d], ck * t);
+            atomicAdd(&sk[(OA + bb) * ncol + colD + d], ck * t);
           }
         }
       };
@@ -1244,7 +1237,7 @@ __global__ __launch_bounds__(256) void k_schwarz(const ShellPair* pairs, const P
   int nprim;
   if constexpr (Big<LA, LB, LA, LB>::value) {
     double acc[Dims<LA, LB, LA, LB>::NE][Dims<LA, LB, LA, LB>::NF];
-    contract<LA, LB, LA, LB, double>(P, P, prims, nullptr, tab + RYS_OFF[Dims<LA, LB, LA, LB>::NROOT], nullptr,
+    contract<LA, LB, LA, LB, double>(P, P, prims, nullptr, tab + QTab<LA, LB, LA, LB>::off64, nullptr,
                                      qcut, imu2, acc, nprim);
     if (nprim)
       stream_slices<LA, LB, LA, LB, PURE>(P, P, xf, acc, [&](int, int, double* S) {
@@ -1253,7 +1246,7 @@ __global__ __launch_bounds__(256) void k_schwarz(const ShellPair* pairs, const P
       });
   } else {
     double V[Dims<LA, LB, LA, LB>::NBLK];
-    quartet_block<LA, LB, LA, LB, PURE, double>(P, P, prims, nullptr, tab + RYS_OFF[Dims<LA, LB, LA, LB>::NROOT],
+    quartet_block<LA, LB, LA, LB, PURE, double>(P, P, prims, nullptr, tab + QTab<LA, LB, LA, LB>::off64,
                                                 nullptr, xf, qcut, imu2, V, nprim);
     if (nprim) {
 #pragma unroll

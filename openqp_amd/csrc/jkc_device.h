@@ -92,7 +92,7 @@ void k_jkc(JKParams prm, WaveWork ww) {
   int iq = 0;
   bool skip = true, mine = true;
   if (active) {
-    iq = ww.ket[ww.seg_k0[seg] + k];
+    iq = ww.kofs + ww.seg_k0[seg] + k;  // the class lists are consecutive device pairs
     const ShellPair Q = prm.pairs[iq];
     // OpenQP screening (int2.F90:763-800)
     const bool p_first = (P.si > Q.si) || (P.si == Q.si && P.sj >= Q.sj);
@@ -100,7 +100,7 @@ void k_jkc(JKParams prm, WaveWork ww) {
     const double qbra = p_first ? P.Q : Q.Q;
     const int n = prm.nsh;
     const double* ds = prm.dsh;
-    double dm = fmax(4.0 * ds[P.si * n + P.sj], 4.0 * ds[Q.si * n + Q.sj]);
+    double dm = 4.0 * fmax(prm.dpm[ip], prm.dpm[iq]);
     dm = fmax(dm, fmax(ds[P.sj * n + Q.sj], ds[P.sj * n + Q.si]));
     dm = fmax(dm, fmax(ds[P.si * n + Q.sj], ds[P.si * n + Q.si]));
     skip = !mine || (qbra * prm.maxden < prm.cutoff) || (P.Q * Q.Q * dm < prm.cutoff);
@@ -190,7 +190,8 @@ void k_jkc(JKParams prm, WaveWork ww) {
       for (int t = l; t < OB * OC; t += W) Dbc[t] = Dp[tri_idx(ob + t / OC, oc + t % OC)];
       for (int t = l; t < OB * OD; t += W) Dbd[t] = Dp[tri_idx(ob + t / OD, od + t % OD)];
     };
-    for (int t = l; t < OCD; t += W) Dcd[t] = prm.D[tri_idx(oc + t / OD, od + t % OD)];
+    const double* Dk = prm.Dk + ww.jbase + (long long)(jq - ww.kofs) * OCD;
+    for (int t = l; t < OCD; t += W) Dcd[t] = Dk[t];
     load_d(prm.D);
 #pragma unroll
     for (int d = 0; d < 3; ++d) ACl[d] = P.A[d] - Q.A[d];

@@ -36,6 +36,10 @@ struct JKG {
   static constexpr int nm = (LA == LB && NEF <= 4) ? 4 : (NEF <= 18 ? 2 : 1);
 #endif
   static constexpr int threads = 512;
+  // (ss|ss): 128 VGPRs, so that two blocks share a CU (four waves per SIMD;
+  // unhinted it takes 139 and one block: 49 -> 31 ms FP64 on (H2O)64/cc-pVDZ);
+  // for (ps|ps) the same cap spills (15.5 -> 27.5 ms)
+  static constexpr int waves = NEF == 1 ? 4 : 1;
 };
 
 // Members per tile of the tiled form: the (e0|f0) accumulators and AO blocks
@@ -189,7 +193,9 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
       const R zeta = pp.g, eta = qq.g;
       const R ze = zeta + eta + zeta * eta * imu2;
       const R fq = pp.Kg * kq;  // the largest member prefactor: no member passes below it
-      if (fq * fq < qcut2 * ze) continue;
+      const R fq2 = fq * fq;
+      if (fq2 < qcut2 * eta) break;  // records in decreasing prefactor: none of the rest passes
+      if (fq2 < qcut2 * ze) continue;
       const R sq = F32 ? (R)__builtin_amdgcn_rsqf((float)ze) : (R)rsq64((double)ze);
       const R ize = sq * sq;
       R val[NE][NF];
@@ -227,18 +233,19 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
 // TILE: the tiled form; its item[0] is the tile's offset in cv.pool (the
 // launch's work lists) and cv.hdr, cv.cp, cv.cp32 are unused.
 template <int LA, int LB, int LC, int LD, bool PURE, bool TWO, bool TILE>
-__global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm, ChunkView cv) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(JKG<LA, LB, LC, LD>::waves)))
+void k_jkg(JKParams prm, BraWork bw, ColMap cm, ChunkView cv) {
   using Dm = Dims<LA, LB, LC, LD>;
   constexpr int NM = TILE ? JKT<LA, LB, LC, LD>::nm : JKG<LA, LB, LC, LD>::nm;
   constexpr int NE = Dm::NE, NF = Dm::NF;
-  constexpr int NR = Dm::NROOT;
-  constexpr bool T64 = RysLds<NR>::f64;
+  using QT = QTab<LA, LB, LC, LD>;
+  constexpr bool T64 = RysLds<LA, LB, LC, LD>::f64;
   constexpr bool T32 = NE * NF <= 256;
   constexpr int OA = AO<LA, PURE>::N, OB = AO<LB, PURE>::N, OC = AO<LC, PURE>::N, OD = AO<LD, PURE>::N;
   constexpr int NOUT = OA * OB * OC * OD, NBLK = Dm::NBLK;
   constexpr bool SAME = (LA == LC && LB == LD);  // bra and ket pairs from one class list
-  __shared__ double s_t64[T64 ? rys_len<NR>() : 1];
-  __shared__ float s_t32[T32 ? rys32_len<NR>() : 1];
+  __shared__ __align__(16) double s_t64[T64 ? QT::len64 : 1];
+  __shared__ __align__(16) float s_t32[T32 ? QT::len32 : 1];
   __shared__ double s_jab[NM * OA * OB];
   __shared__ double s_dab[NM * OA * OB];  // each member's bra density block
   __shared__ double s_mq[NM], s_mthr[NM], s_mdab[NM];
@@ -280,10 +287,10 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
     for (int i = threadIdx.x; i < nk; i += blockDim.x) s_k2[i] = 0.0;
   for (int i = threadIdx.x; i < NM * OA * OB; i += blockDim.x) s_jab[i] = 0.0;
   if constexpr (T64)
-    for (int i = threadIdx.x; i < rys_len<NR>(); i += blockDim.x) s_t64[i] = prm.rys[RYS_OFF[NR] + i];
+    for (int i = threadIdx.x; i < QT::len64; i += blockDim.x) s_t64[i] = prm.rys[QT::off64 + i];
   if constexpr (T32)
     if (prm.mixed)
-      for (int i = threadIdx.x; i < rys32_len<NR>(); i += blockDim.x) s_t32[i] = prm.rys32[RYS32_OFF[NR] + i];
+      for (int i = threadIdx.x; i < QT::len32; i += blockDim.x) s_t32[i] = prm.rys32[QT::off32 + i];
   if (threadIdx.x < NM) {
     const int m = threadIdx.x;
     if (m < nmem) {
@@ -364,8 +371,8 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
         s_cp32[i] = i < ncp * stride ? cv.cp32[cprim0 + i] : (i % stride == 0 ? 1.0f : 0.0f);
   }
   __syncthreads();
-  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + RYS_OFF[NR];
-  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + RYS32_OFF[NR];
+  const double* tabN = T64 ? (const double*)s_t64 : prm.rys + QT::off64;
+  const float* tab32N = T32 ? (const float*)s_t32 : prm.rys32 + QT::off32;
   const int lane = (int)__lane_id(), wv = (int)(threadIdx.x >> 6), nw = (int)(blockDim.x >> 6);
   const double* Dp = prm.D;
   double* F = prm.F;
@@ -396,9 +403,9 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
       unsigned live = 0;
       double bmax = 0.0;
       if (active) {
-        iq = bw.ket[kbase + k];
+        iq = bw.kofs + kbase + k;  // the class lists are consecutive device pairs
         Q = prm.pairs[iq];
-        const double dcd4 = 4.0 * prm.dsh[Q.si * nsh + Q.sj];
+        const double dcd4 = 4.0 * prm.dpm[iq];
 #pragma unroll 1
         for (int m = 0; m < nmem; ++m) {
           const int id = mi[m][0], si = mi[m][5], sj = mi[m][6];
@@ -508,14 +515,13 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
       }
       if (__ballot(any_valid) == 0ull) continue;  // wave-uniform
       double Dcd[OC * OD];
+      const double* Dk = prm.Dk + bw.jbase + (long long)(iq - bw.kofs) * (OC * OD);
 #pragma unroll
-      for (int x = 0; x < OC; ++x)
-#pragma unroll
-        for (int y = 0; y < OD; ++y) Dcd[x * OD + y] = any_valid ? Dp[tri_idx(oc + x, od + y)] : 0.0;
+      for (int cd = 0; cd < OC * OD; ++cd) Dcd[cd] = any_valid ? Dk[cd] : 0.0;
       double tcd[OC * OD];
 #pragma unroll
       for (int i = 0; i < OC * OD; ++i) tcd[i] = 0.0;
-      const int colC = active ? cm.colidx[Q.sa] : 0, colD = active ? cm.dofs + cm.colidx[Q.sb] : 0;
+      const int colC = Q.ca, colD = cm.dofs + Q.cb;
 #pragma unroll
       for (int m = 0; m < NM; ++m) {
         if (m >= nmem) break;  // uniform
@@ -595,7 +601,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
               for (int bb = 0; bb < OB; ++bb)
 #pragma unroll
                 for (int d = 0; d < OD; ++d) t += VV(a, bb, cc, d) * Dbd[bb * OD + d];
-              if (t != 0.0) atomicAdd(&sk[(ra + a) * ncol + colC + cc], ck * t);
+              atomicAdd(&sk[(ra + a) * ncol + colC + cc], ck * t);
             }
 #pragma unroll
             for (int d = 0; d < OD; ++d) {
@@ -604,7 +610,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
               for (int bb = 0; bb < OB; ++bb)
 #pragma unroll
                 for (int cc = 0; cc < OC; ++cc) t += VV(a, bb, cc, d) * Dbc[bb * OC + cc];
-              if (t != 0.0) atomicAdd(&sk[(ra + a) * ncol + colD + d], ck * t);
+              atomicAdd(&sk[(ra + a) * ncol + colD + d], ck * t);
             }
           }
 #pragma unroll
@@ -616,7 +622,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
               for (int a = 0; a < OA; ++a)
 #pragma unroll
                 for (int d = 0; d < OD; ++d) t += VV(a, bb, cc, d) * Dad[a * OD + d];
-              if (t != 0.0) atomicAdd(&sk[(rb + bb) * ncol + colC + cc], ck * t);
+              atomicAdd(&sk[(rb + bb) * ncol + colC + cc], ck * t);
             }
 #pragma unroll
             for (int d = 0; d < OD; ++d) {
@@ -625,7 +631,7 @@ __global__ __launch_bounds__(512) void k_jkg(JKParams prm, BraWork bw, ColMap cm
               for (int a = 0; a < OA; ++a)
 #pragma unroll
                 for (int cc = 0; cc < OC; ++cc) t += VV(a, bb, cc, d) * Dac[a * OC + cc];
-              if (t != 0.0) atomicAdd(&sk[(rb + bb) * ncol + colD + d], ck * t);
+              atomicAdd(&sk[(rb + bb) * ncol + colD + d], ck * t);
             }
           }
         };

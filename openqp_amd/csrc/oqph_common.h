@@ -27,6 +27,7 @@ struct ShellPair {
   int prim0, nprim;            // primitive-pair range in prims[]
   int si, sj;                  // reference order: si >= sj (shell indices)
   int la, lb;                  // angular momenta of a, b (la >= lb)
+  int ca, cb;                  // first AO of a, b among the AOs of its angular momentum (ColMap; J/K records)
 };
 
 struct PrimPair {              // 64 bytes: one cache line per primitive pair
@@ -179,7 +180,6 @@ struct ChunkView {
 // LDS column space of the K rows of one launch: the AOs of the shells of
 // angular momentum lc (C space) and, when ld != lc, of ld (D space, after C).
 struct ColMap {
-  const int* colidx;  // per shell: AO offset among the shells of its angular momentum
   const int* aoC;     // global AO index of each C-space column
   const int* aoD;     // global AO index of each D-space column
   int ncolC;          // C-space columns
@@ -211,6 +211,11 @@ struct JKParams {
   // pass after the launches adds the blocks into F (with the diagonal
   // doubling).  Random FP64 atomics into F were the J_cd bottleneck.
   double* Jk;
+  // The density blocks D_cd and the maxima dsh of the device pairs in the
+  // same order, gathered once per build: the kets of a wavefront read them
+  // coalesced instead of through three dependent gathers.
+  const double* Dk;
+  const double* dpm;
   const double* dsh;    // nsh*nsh shell-pair max |D|
   unsigned long long* counters;  // [0] computed quartets, [1] skipped by fine screen, [2] fp32 quartets
   int nsh;

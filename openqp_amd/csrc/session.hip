@@ -48,6 +48,8 @@ void launch_shell_density(const double* D, const double* D2, const int* ao_off, 
 void launch_sumdiff(const double* a, const double* b, double* p, double* m, double c, long long n, hipStream_t s);
 void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* Jk, double* F,
                      hipStream_t s);
+void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
+                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s);
 void launch_max_reduce(const double* x, long long n, unsigned long long* out, hipStream_t s);
 bool kernels_support(int lmax);
 bool jk_template(int la, int lb, int lc, int ld);
@@ -204,6 +206,7 @@ struct oqph_session {
   std::vector<int> h_joff, jbase;
   DBuf<int> d_joff;
   DBuf<double> d_jk;
+  DBuf<double> d_dk, d_dpm;                  // JKParams::Dk, dpm (allocated with the geometry)
   DBuf<int> d_kbs;                           // per class: bucket starts (NBKT+1)
   std::vector<std::vector<int>> kbs;
   std::vector<size_t> cls_off;
@@ -273,7 +276,7 @@ struct oqph_session {
   };
   // bra-row kernel: LDS column spaces per angular momentum and its work items
   std::vector<int> h_colidx, h_colao, colbase, ncolL;
-  DBuf<int> d_colidx, d_colao, d_items;
+  DBuf<int> d_colao, d_items;
   std::vector<int> h_items;
   size_t lds_max = 0;
   // OQPH_JK_ROWS: 0 = wavefront-task kernel only, 2 = bra-row kernel wherever its
@@ -666,10 +669,18 @@ static int build_chunkset(oqph_session* s, int cb, int cap, const std::vector<Pr
         for (int k = 0; k < s->nao[shl[t]]; ++k) cs.pool.push_back(s->aooff[shl[t]] + k);
       cs.pool.insert(cs.pool.end(), shl.begin(), shl.end());
       (void)o;
+      // records in decreasing largest prefactor (the kernel's loop ends at the
+      // first that cannot pass the primitive screen)
+      std::vector<double> kmax(base.size(), 0.0);
+      std::vector<int> ord(base.size());
       for (size_t g = 0; g < base.size(); ++g) {
+        ord[g] = (int)g;
+        for (int m = 0; m < nm; ++m) kmax[g] = std::max(kmax[g], std::fabs(kg[g][m]));
+      }
+      std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return kmax[x] > kmax[y]; });
+      for (const int g : ord) {
         const PrimPair& q = *base[g];
-        double km = 0.0;
-        for (int m = 0; m < nm; ++m) km = std::max(km, std::fabs(kg[g][m]));
+        const double km = kmax[g];
         const double rec[6] = {q.g, q.P[0] - p0.A[0], q.P[1] - p0.A[1], q.P[2] - p0.A[2], q.h, km};
         for (double v : rec) {
           cp.push_back(v);
@@ -830,7 +841,15 @@ static int prepare_geometry(oqph_session* s) {
   // regular pair data (int2.F90:266-272): quartet 1e-4 c, exponent 25 ln 10
   std::vector<PrimPair> prims;
   build_pairs(*s, Cut{1.0e-4 * s->cutoff, 25.0 * std::log(10.0)}, s->pairs, prims);
-  for (size_t pid = 0; pid < np; ++pid) s->pairs[pid].Q = s->Q[pid];
+  // each pair's primitive pairs in decreasing |K|: the primitive screen then
+  // ends a bra loop at its first certain failure, and the lanes of a wavefront
+  // (kets of one class) keep step
+  for (size_t pid = 0; pid < np; ++pid) {
+    s->pairs[pid].Q = s->Q[pid];
+    PrimPair* pp = prims.data() + s->pairs[pid].prim0;
+    const auto more = [](const PrimPair& x, const PrimPair& y) { return std::fabs(x.Kg) > std::fabs(y.Kg); };
+    if (s->pairs[pid].nprim > 1) std::sort(pp, pp + s->pairs[pid].nprim, more);
+  }
   // class lists of significant pairs, Q descending
   s->cls.assign(10, {});
   s->clsQ.assign(10, {});
@@ -861,6 +880,23 @@ static int prepare_geometry(oqph_session* s) {
   }
   s->cls_off[10] = all.size();
   s->dev_pid.assign(all.begin(), all.end());
+  // LDS column spaces of the bra-row kernel: the AOs of the shells of each
+  // angular momentum, in shell order
+  s->h_colidx.assign(s->nsh, 0);
+  s->h_colao.clear();
+  s->colbase.assign(s->lmax + 1, 0);
+  s->ncolL.assign(s->lmax + 1, 0);
+  for (int L = 0; L <= s->lmax; ++L) {
+    s->colbase[L] = (int)s->h_colao.size();
+    int off = 0;
+    for (int i = 0; i < s->nsh; ++i)
+      if (s->am[i] == L) {
+        s->h_colidx[i] = off;
+        for (int k = 0; k < s->nao[i]; ++k) s->h_colao.push_back(s->aooff[i] + k);
+        off += s->nao[i];
+      }
+    s->ncolL[L] = off;
+  }
   // Device pair and primitive-pair records in class-list order: device pair
   // id i is s->pairs[all[i]], so the 64 kets of a wavefront (consecutive
   // list entries) read consecutive records; the class lists on the device
@@ -875,6 +911,8 @@ static int prepare_geometry(oqph_session* s) {
       dp[i] = s->pairs[all[i]];
       dp[i].prim0 = (int)dpr.size();
       const ShellPair& o = s->pairs[all[i]];
+      dp[i].ca = s->h_colidx[o.sa];
+      dp[i].cb = s->h_colidx[o.sb];
       for (int k = o.prim0; k < o.prim0 + o.nprim; ++k) {
         dpr.push_back(jk_record(prims[k], o));
         dpr32.push_back(f32_record(dpr.back()));
@@ -886,7 +924,8 @@ static int prepare_geometry(oqph_session* s) {
       s->h_joff[i + 1] = s->h_joff[i] + nao_of(dp[i].la, s->pure) * nao_of(dp[i].lb, s->pure);
     s->jbase.assign(11, 0);
     for (int c = 0; c <= 10; ++c) s->jbase[c] = s->h_joff[s->cls_off[c]];
-    if ((rc = s->d_joff.ensure(s->h_joff.size())) ||
+    if ((rc = s->d_dk.ensure(std::max<size_t>((size_t)s->h_joff.back(), 1))) ||
+        (rc = s->d_dpm.ensure(std::max<size_t>(dp.size(), 1))) || (rc = s->d_joff.ensure(s->h_joff.size())) ||
         (rc = upload_sync(s->d_joff.p, s->h_joff.data(), s->h_joff.size() * sizeof(int), s->stream)))
       return rc;
     std::vector<int> ident(all.size());
@@ -909,25 +948,7 @@ static int prepare_geometry(oqph_session* s) {
   if ((rc = s->d_aooff.ensure(s->nsh)) || (rc = s->d_nao.ensure(s->nsh))) return rc;
   if ((rc = upload_sync(s->d_aooff.p, s->aooff.data(), s->nsh * sizeof(int), s->stream))) return rc;
   if ((rc = upload_sync(s->d_nao.p, s->nao.data(), s->nsh * sizeof(int), s->stream))) return rc;
-  // LDS column spaces of the bra-row kernel: the AOs of the shells of each
-  // angular momentum, in shell order
-  s->h_colidx.assign(s->nsh, 0);
-  s->h_colao.clear();
-  s->colbase.assign(s->lmax + 1, 0);
-  s->ncolL.assign(s->lmax + 1, 0);
-  for (int L = 0; L <= s->lmax; ++L) {
-    s->colbase[L] = (int)s->h_colao.size();
-    int off = 0;
-    for (int i = 0; i < s->nsh; ++i)
-      if (s->am[i] == L) {
-        s->h_colidx[i] = off;
-        for (int k = 0; k < s->nao[i]; ++k) s->h_colao.push_back(s->aooff[i] + k);
-        off += s->nao[i];
-      }
-    s->ncolL[L] = off;
-  }
-  if ((rc = s->d_colidx.ensure(s->nsh)) || (rc = s->d_colao.ensure(s->h_colao.size()))) return rc;
-  if ((rc = upload_sync(s->d_colidx.p, s->h_colidx.data(), s->nsh * sizeof(int), s->stream)) ||
+  if ((rc = s->d_colao.ensure(s->h_colao.size())) ||
       (rc = upload_sync(s->d_colao.p, s->h_colao.data(), s->h_colao.size() * sizeof(int), s->stream)))
     return rc;
   const size_t ntri = (size_t)s->nbf * (s->nbf + 1) / 2;
@@ -1681,7 +1702,6 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
       L.bw.kofs = (int)s->cls_off[p.ck];
       for (int b = 0; b <= NBKT; ++b) L.bw.kb[b] = s->kbs[p.ck][b];
       L.bw.nitem = p.nitem;
-      L.cm.colidx = s->d_colidx.p;
       L.cm.aoC = s->d_colao.p + s->colbase[p.lc];
       L.cm.aoD = s->d_colao.p + s->colbase[p.ld];
       L.cm.ncolC = p.ncolC;
@@ -2001,8 +2021,11 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   p.rys = s->d_rys.p;
   p.rys32 = s->d_rys32.p;
   p.xform = s->d_xform.p;
-  HIPCHK(hipMemsetAsync(Jk, 0, njk * sizeof(double), stream));
+  launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, dD, dsh, s->nsh, s->d_dk.p,
+                 s->d_dpm.p, Jk, stream);
   p.Jk = Jk;
+  p.Dk = s->d_dk.p;
+  p.dpm = s->d_dpm.p;
   p.D = dD;
   p.F = dF;
   p.D2 = dF2 ? dD2 : nullptr;
@@ -2240,7 +2263,7 @@ int oqph_session_destroy(oqph_session* s) {
   s->d_xform.release(); s->d_rys32.release(); s->d_kbs.release(); s->d_seg.release(); s->d_choff.release();
   s->d_gpairs.release(); s->d_gprims.release(); s->d_gcls.release(); s->d_coff.release(); s->d_satom.release();
   s->d_am.release(); s->d_pure.release(); s->d_gseg.release(); s->d_gchoff.release(); s->d_Dc.release(); s->d_de.release();
-  s->d_aooff.release(); s->d_nao.release(); s->d_colidx.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
+  s->d_aooff.release(); s->d_nao.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
   s->d_tmp.release(); s->d_off.release(); s->d_ctr.release();
   s->d_gD.release(); s->d_gF.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
   for (auto e : s->pev) hipEventDestroy(e);
