@@ -50,6 +50,10 @@ JKC = [(1, 1, 1, 1), (2, 0, 1, 1), (2, 0, 2, 0), (2, 1, 1, 0), (2, 1, 1, 1), (2,
        (3, 2, 1, 0), (3, 2, 1, 1), (3, 2, 2, 0), (3, 2, 2, 1), (3, 2, 2, 2), (3, 2, 3, 0), (3, 2, 3, 1), (3, 2, 3, 2),
        (3, 3, 1, 0), (3, 3, 1, 1), (3, 3, 2, 0), (3, 3, 2, 1), (3, 3, 2, 2), (3, 3, 3, 0), (3, 3, 3, 1)]
 
+# classes with a cooperative gradient kernel (gradc_class.hip; the list matches
+# OQPH_GRC_CLASSES in dispatch.hip): those of more than 64 Cartesian components
+GRC = [c for c in JKC if c not in [(2, 0, 1, 1), (2, 0, 2, 0), (2, 1, 1, 0), (3, 0, 2, 0)]]
+
 
 def _cost(c):
     a, b, cc, d = c
@@ -64,6 +68,8 @@ DEPS = {
     "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "session.hip": ["oqph_common.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
     "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
+    "gradc_class.hip": ["gradc_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc",
+                        "rys_table.inc", "rys_table_f32.inc"],
     "int1e.hip": ["../../include/oqph.h", "ao_xform.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "hl.hip": ["hl_device.h", "jk_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                "rys_table_f32.inc"],
@@ -90,7 +96,7 @@ def _jobs():
     heavy, light = [], []
     per_class = [(c, "jk_class.hip", "jk") for c in CLASSES + F_JK] + \
                 [(c, "grad_class.hip", "gr") for c in CLASSES + F_GRAD if c not in GRAD_HL] + \
-                [(c, "jkc_class.hip", "jkc") for c in JKC]
+                [(c, "jkc_class.hip", "jkc") for c in JKC] + [(c, "gradc_class.hip", "grc") for c in GRC]
     for c, unit, tag in sorted(per_class, key=lambda t: _cost(t[0]), reverse=True):
         a, b, cc, d = c
         defs = [f"-DXA={a}", f"-DXB={b}", f"-DXC={cc}", f"-DXD={d}"]

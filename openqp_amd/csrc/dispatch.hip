@@ -30,6 +30,13 @@ namespace oqph {
   X(3, 1, 2, 2) X(3, 1, 3, 0) X(3, 1, 3, 1) X(3, 2, 1, 0) X(3, 2, 1, 1) X(3, 2, 2, 0) X(3, 2, 2, 1) \
   X(3, 2, 2, 2) X(3, 2, 3, 0) X(3, 2, 3, 1) X(3, 2, 3, 2) X(3, 3, 1, 0) X(3, 3, 1, 1) X(3, 3, 2, 0) \
   X(3, 3, 2, 1) X(3, 3, 2, 2) X(3, 3, 3, 0) X(3, 3, 3, 1)
+// cooperative gradient kernel (k_gradc; gradc_class.hip), the GRC list of build.py
+#define OQPH_GRC_CLASSES(X) \
+  X(1, 1, 1, 1) X(2, 1, 1, 1) X(2, 1, 2, 0) X(2, 1, 2, 1) X(2, 2, 1, 0) X(2, 2, 1, 1) X(2, 2, 2, 0) \
+  X(2, 2, 2, 1) X(2, 2, 2, 2) X(3, 0, 1, 1) X(3, 0, 2, 1) X(3, 0, 2, 2) X(3, 0, 3, 0) X(3, 1, 1, 0) \
+  X(3, 1, 1, 1) X(3, 1, 2, 0) X(3, 1, 2, 1) X(3, 1, 2, 2) X(3, 1, 3, 0) X(3, 1, 3, 1) X(3, 2, 1, 0) \
+  X(3, 2, 1, 1) X(3, 2, 2, 0) X(3, 2, 2, 1) X(3, 2, 2, 2) X(3, 2, 3, 0) X(3, 2, 3, 1) X(3, 2, 3, 2) \
+  X(3, 3, 1, 0) X(3, 3, 1, 1) X(3, 3, 2, 0) X(3, 3, 2, 1) X(3, 3, 2, 2) X(3, 3, 3, 0) X(3, 3, 3, 1)
 #define OQPH_SCHWARZ_CLASSES(X) X(0, 0) X(1, 0) X(1, 1) X(2, 0) X(2, 1) X(2, 2)
 
 #define OQPH_CODE(a, b, c, d) ((a) * 1000 + (b) * 100 + (c) * 10 + (d))
@@ -50,6 +57,10 @@ OQPH_JK_CLASSES(OQPH_DECL_JK)
   void launch_jkc_##a##b##c##d(bool, const JKParams&, const WaveWork&, hipStream_t); \
   bool jkc_res_##a##b##c##d(bool, bool, KernelRes*);
 OQPH_JKC_CLASSES(OQPH_DECL_JKC)
+#define OQPH_DECL_GRC(a, b, c, d)                                                  \
+  void launch_gradc_##a##b##c##d(const GradParams&, const WaveWork&, hipStream_t); \
+  bool gradc_res_##a##b##c##d(KernelRes*);
+OQPH_GRC_CLASSES(OQPH_DECL_GRC)
 #define OQPH_DECL_GR(a, b, c, d)                                              \
   void launch_grad_##a##b##c##d(const GradParams&, const WaveWork&, hipStream_t, bool, bool); \
   bool grad_res_##a##b##c##d(KernelRes*, bool, bool);
@@ -156,8 +167,8 @@ bool jkb_info(int la, int lb, int lc, int ld, bool pure, int* nrow, size_t* stat
 }
 
 // Compiled resources of one class-templated kernel: kind 0 = k_jk, 1 = k_jkb,
-// 2 = k_grad, 3 = k_schwarz (lc, ld ignored), 4 = k_jkg, 6 = tiled k_jkg, 7 = k_jkc; false when there is no
-// such kernel.  hipFuncGetAttributes reads the code object, nothing is launched.
+// 2 = k_grad, 3 = k_schwarz (lc, ld ignored), 4 = k_jkg, 6 = tiled k_jkg, 7 = k_jkc, 8 = k_gradc; false when there
+// is no such kernel.  hipFuncGetAttributes reads the code object, nothing is launched.
 // kind | 16 (k_jk, k_jkb, k_jkg, k_jkc): the open-shell variant
 bool kernel_resources(int kind, int la, int lb, int lc, int ld, bool pure, KernelRes* r) {
   const int base = kind & 15;
@@ -176,6 +187,15 @@ bool kernel_resources(int kind, int la, int lb, int lc, int ld, bool pure, Kerne
 #define OQPH_CASE(a, b, c, d) \
   case OQPH_CODE(a, b, c, d): return jkc_res_##a##b##c##d(pure, (kind & 16) != 0, r);
       OQPH_JKC_CLASSES(OQPH_CASE)
+#undef OQPH_CASE
+      default: return false;
+    }
+  }
+  if (base == 8) {
+    switch (OQPH_CODE(la, lb, lc, ld)) {
+#define OQPH_CASE(a, b, c, d) \
+  case OQPH_CODE(a, b, c, d): return gradc_res_##a##b##c##d(r);
+      OQPH_GRC_CLASSES(OQPH_CASE)
 #undef OQPH_CASE
       default: return false;
     }
@@ -211,6 +231,17 @@ bool launch_grad(int la, int lb, int lc, int ld, const GradParams& p, const Wave
 #define OQPH_CASE(a, b, c, d) \
   case OQPH_CODE(a, b, c, d): launch_grad_##a##b##c##d(p, ww, s, f32, mrsf); return true;
     OQPH_GRAD_CLASSES(OQPH_CASE)
+#undef OQPH_CASE
+    default: return false;
+  }
+}
+
+bool launch_gradc(int la, int lb, int lc, int ld, const GradParams& p, const WaveWork& ww, hipStream_t s) {
+  if (ww.nwaves == 0) return true;
+  switch (OQPH_CODE(la, lb, lc, ld)) {
+#define OQPH_CASE(a, b, c, d) \
+  case OQPH_CODE(a, b, c, d): launch_gradc_##a##b##c##d(p, ww, s); return true;
+    OQPH_GRC_CLASSES(OQPH_CASE)
 #undef OQPH_CASE
     default: return false;
   }

@@ -11,14 +11,23 @@ namespace oqph {
 // components (its two-particle density is gathered per element)
 constexpr bool MRSF_T = ncart(XA) * ncart(XB) * ncart(XC) * ncart(XD) <= 27;
 
+constexpr bool SPLIT_T = ncart(XA) * ncart(XB) * ncart(XC) * ncart(XD) <= OQPH_GRAD_SPLIT_NG;
+
 // f32: the FP32 form (quartets the host assigned to FP32); mrsf: the MRSF
-// two-particle density (FP64)
+// two-particle density (FP64); ww.kpb below 64: the split form (FP64)
 void OQPH_GR_LAUNCHER(XA, XB, XC, XD)(const GradParams& p, const WaveWork& ww, hipStream_t s, bool f32, bool mrsf) {
   const int bs = 256;  // four wavefronts
   const long long nb = (ww.nwaves + 3) / 4;
   if constexpr (MRSF_T)
     if (mrsf) {
       hipLaunchKernelGGL((k_grad<XA, XB, XC, XD, double, true>), dim3((unsigned)nb), dim3(bs),
+                         sizeof(double) * 3 * p.natm, s, p, ww);
+      return;
+    }
+  if constexpr (SPLIT_T)
+    if (!f32 && ww.kpb > 0 && ww.kpb < 64) {
+      const long long ns = (ww.nwaves * (64 / ww.kpb) + 3) / 4;
+      hipLaunchKernelGGL((k_grad<XA, XB, XC, XD, double, false, true>), dim3((unsigned)ns), dim3(bs),
                          sizeof(double) * 3 * p.natm, s, p, ww);
       return;
     }

@@ -59,8 +59,13 @@ __host__ __device__ constexpr long long flops_grad_prim() {
   return flops_grad_prim_rt(LA, LB, LC, LD);
 }
 
-// MRSF: Gamma from the MRSF matrices (prm.Mc) instead of the density
-template <int LA, int LB, int LC, int LD, typename R, bool MRSF = false>
+// MRSF: Gamma from the MRSF matrices (prm.Mc) instead of the density.
+// SPLIT: a launch of few wavefronts is bound by the longest lane (one lane
+// walks up to 81 x 81 primitive quartets of a cc-pVDZ (ss|ss) quartet), so a
+// chunk of 64 kets is spread over 64 / kpb wavefronts, each ket on 64 / kpb
+// lanes that take every (64 / kpb)-th primitive quartet and sum at the end.
+// One water's gradient in cc-pVTZ 50.8 -> 25.3 ms, in 6-31G(d) 5.9 -> 2.7.
+template <int LA, int LB, int LC, int LD, typename R, bool MRSF = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
   extern __shared__ double s_de[];
   constexpr bool F32 = sizeof(R) == 4;
@@ -86,7 +91,12 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
   // Waves past the end still reach the block barrier below.
   const long long wave = __builtin_amdgcn_readfirstlane(
       (int)((blockIdx.x * (long long)blockDim.x + threadIdx.x) >> 6));
-  const bool wave_ok = wave < ww.nwaves;
+  const int kpb = SPLIT ? ww.kpb : 64, per = SPLIT ? 64 / kpb : 1;  // kets per wavefront, lanes per ket
+  const long long chunk = SPLIT ? wave / per : wave;
+  const int lane = (int)__lane_id();
+  const int psub = SPLIT ? lane & (per - 1) : 0;  // this lane's share of its ket's primitive quartets
+  const bool head = !SPLIT || psub == 0;
+  const bool wave_ok = chunk < ww.nwaves;
   bool active = false;
   bool skip = true;
   ShellPair P{}, Q{};
@@ -97,10 +107,10 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
     int lo = 0, hi = ww.nseg;
     while (hi - lo > 1) {  // scalar binary search over the chunk prefix
       const int mid = (lo + hi) >> 1;
-      if (ww.choff[mid] <= wave) lo = mid; else hi = mid;
+      if (ww.choff[mid] <= chunk) lo = mid; else hi = mid;
     }
     const int seg = __builtin_amdgcn_readfirstlane(lo);
-    const int k = (int)(wave - ww.choff[seg]) * 64 + (int)__lane_id();
+    const int k = (int)(chunk - ww.choff[seg]) * 64 + (SPLIT ? (int)(wave - chunk * per) * kpb + lane / per : lane);
     active = k < ww.seg_n[seg];
     ip = __builtin_amdgcn_readfirstlane(ww.seg_bra[seg]);
     P = prm.pairs[ip];
@@ -133,16 +143,29 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
     skip = gm * P.Q * Q.Q < 0.5 * prm.gcut;
   }
   unsigned long long* ctr = prm.counters + 8 * (int)(wave & (OQPH_CTR_SLOTS - 1));
-  count_wave_g(ctr + 1, active && skip);
-  count_wave_g(ctr + 0, !skip);
+  count_wave_g(ctr + 1, head && active && skip);
+  count_wave_g(ctr + 0, head && !skip);
   R fd[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
   int nprim = 0;
-  if (!skip) {
+  if (!skip && P.nprim > 0) {
     const double dab2 = gm * gm;
-    for (int iqq = 0; iqq < Q.nprim; ++iqq) {
+    const int NP = P.nprim;
+    // SPLIT: primitive quartets psub, psub + per, ... of the flattened list;
+    // else ket primitives outside, the wavefront's bra primitives inside
+    int iqq = 0, ipp = psub;
+    if constexpr (SPLIT)
+      while (ipp >= NP) { ipp -= NP; ++iqq; }
+    while (iqq < Q.nprim) {
       const PrimPair qq = prm.prims[Q.prim0 + iqq];
-      for (int ipp = 0; ipp < P.nprim; ++ipp) {
-        const PrimPair pp = load_uniform(prm.prims, P.prim0 + ipp);
+      const int ip0 = SPLIT ? ipp : 0, ip1 = SPLIT ? ipp + 1 : NP;
+      if constexpr (SPLIT) {
+        ipp += per;
+        while (ipp >= NP) { ipp -= NP; ++iqq; }
+      } else {
+        ++iqq;
+      }
+      for (int ipr = ip0; ipr < ip1; ++ipr) {
+        const PrimPair pp = SPLIT ? prm.prims[P.prim0 + ipr] : load_uniform(prm.prims, P.prim0 + ipr);
         const double zeta = pp.g, eta = qq.g, ze = zeta + eta;
         const double fqz = pp.Kg * qq.Kg;
         // primitive screens (grd2_rys.F90:375-376), prefactor cutoff (1e-20)^2
@@ -246,8 +269,22 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
       }
     }
   }
-  sum_wave_g(ctr + 3, (unsigned long long)nprim * flops_grad_prim<LA, LB, LC, LD>());
-  sum_wave_g(ctr + 4, (unsigned long long)nprim);
+  if constexpr (SPLIT) {
+    // sums over the lanes of a ket (they skip together); its first lane digests
+    sum_wave_g(ctr + 3, (unsigned long long)nprim * flops_grad_prim<LA, LB, LC, LD>());
+    sum_wave_g(ctr + 4, (unsigned long long)nprim);
+    for (int o = 1; o < per; o <<= 1) {
+      nprim += __shfl_xor(nprim, o);
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) fd[c][d] += __shfl_xor(fd[c][d], o);
+    }
+    if (!head) nprim = 0;
+  } else {
+    sum_wave_g(ctr + 3, (unsigned long long)nprim * flops_grad_prim<LA, LB, LC, LD>());
+    sum_wave_g(ctr + 4, (unsigned long long)nprim);
+  }
   if (!skip && nprim > 0) {
     double deg = 1.0;
     if (P.sa == P.sb) deg *= 0.5;

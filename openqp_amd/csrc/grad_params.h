@@ -9,6 +9,10 @@ namespace oqph {
 // by the host, so thousands of blocks do not serialise on the same lines.
 #define OQPH_DE_SLOTS 32
 
+// Classes up to this many Cartesian components have the split form of k_grad
+// (a ket's primitive quartets over several lanes).
+#define OQPH_GRAD_SPLIT_NG 54
+
 struct GradParams {
   const ShellPair* pairs;
   const PrimPair* prims;

@@ -65,6 +65,7 @@ void launch_gradh(const HLDims& h, const GradParams& p, const WaveWork& ww, hipS
 void launch_gradh_multi(const GradParams& p, const HLTaskList& tl, long long nblocks, int lds, hipStream_t s);
 bool launch_grad(int la, int lb, int lc, int ld, const GradParams& p, const WaveWork& ww, hipStream_t s, bool f32,
                  bool mrsf);
+bool launch_gradc(int la, int lb, int lc, int ld, const GradParams& p, const WaveWork& ww, hipStream_t s);
 void launch_cart_matrix(const double* M, int nbf, int nsh, const int* am, const int* pure, const int* ao_off,
                         const int* coff, const double* xf, int ncf, double* Mc, hipStream_t s);
 void launch_cart_density(const double* D, int nsh, const int* am, const int* pure, const int* ao_off, const int* coff,
@@ -233,6 +234,7 @@ struct oqph_session {
     long long nblocks = 0;
     int lds = 0;
     bool f32 = false;  // the FP32 form of the class template (mixed-precision gradient)
+    bool coop = false;  // cooperative kernel (k_gradc)
   };
   // Grouped bra-row kernel (k_jkg): per shell, the shell whose primitive set
   // it is contracted from (fam[i] = i for a family's master); per bra class
@@ -250,6 +252,7 @@ struct oqph_session {
   std::map<int, std::unique_ptr<ChunkSet>> chunksets;  // key: bra class * 16 + cap
   int jkg_mode = 1;  // OQPH_JKG: 0 = segmented bra-row kernel only, 1 = default class pairs, 2 = all
   int jkg_cap = 0;   // OQPH_JKG_CAP: at most this many members per chunk (0: the kernel's)
+  bool gradc_on = true;  // OQPH_GRADC=0: no cooperative gradient kernel
   int jkc_mode = 1;  // OQPH_JKC: 0 = no cooperative kernel, 1 = jkc_class(), 2 = every class that has one
   int jkt_mode = 0;  // OQPH_JKT: 0 (default) = no tiles, 1 = (ps|ps), 2 = every class pair with a tiled kernel
   struct WLaunch {
@@ -831,6 +834,8 @@ static int prepare_geometry(oqph_session* s) {
     s->jkg_mode = (g && (g[0] == '0' || g[0] == '2')) ? g[0] - '0' : 1;
     const char* jc = getenv("OQPH_JKC");
     s->jkc_mode = (jc && (jc[0] == '0' || jc[0] == '2')) ? jc[0] - '0' : 1;
+    const char* gk = getenv("OQPH_GRADC");
+    s->gradc_on = !(gk && gk[0] == '0');
     const char* jt = getenv("OQPH_JKT");
     s->jkt_mode = (jt && (jt[0] == '1' || jt[0] == '2')) ? jt[0] - '0' : 0;
     const char* gc = getenv("OQPH_JKG_CAP");
@@ -1006,6 +1011,24 @@ static long long class_weight(int la, int lb, int lc, int ld, bool runtime) {
   return runtime ? w + (1ll << 40) : w;
 }
 
+// Class pairs on the cooperative gradient kernel k_gradc: all that have one,
+// which are those of more than 64 Cartesian components.  Measured against the
+// per-lane templates (k_grad) and, from 256 components, the run-time-class
+// kernel, summed kernel time of one gradient of (H2O)16/cc-pVTZ and of
+// C20H42/6-31G(d): (dp|pp) 50 -> 13 ms and 3.9 -> 1.6, (pp|pp) 26 -> 20 and
+// 3.4 -> 1.0, (dp|ds) 22 -> 17 and 1.4 -> 1.6, (dd|ps) 13 -> 10 and 1.2 -> 0.9,
+// (dd|ds) 9.7 -> 4.5 and 1.05 -> 0.41, (fs|pp) 11 -> 6.4, (fs|fs) 5.7 -> 3.3, all
+// classes of the run-time kernel 425 -> 110 and 3.6 -> 1.4.  Below the line the
+// lanes and LDS round trips cost more than they save: (dp|ps), 54 components,
+// 17 -> 34 and 0.9 -> 3.1; (ds|pp) 10 -> 20; (ds|ds) 4.4 -> 13; (fs|ds) 3.9 -> 7.8.
+// The FP32 classes of a mixed gradient and the MRSF gradient keep k_grad / k_gradh.
+static bool gradc_class(const oqph_session* s, int la, int lb, int lc, int ld, KernelRes* r) {
+  if (!s->gradc_on || s->grad_all_hl || (s->grad_hl_ng == 0 && grad_template(la, lb, lc, ld))) return false;
+  if (!s->f_templates && (la == 3 || lc == 3)) return false;
+  return kernel_resources(8, la, lb, lc, ld, s->pure, r) && r->private_bytes <= OQPH_PRIVATE_BUDGET &&
+         (size_t)r->lds_bytes + 24 * (size_t)s->natm <= s->lds_max;
+}
+
 // gradient pair data and coarse-screened quartet lists (grd2.F90:219-328):
 // pair data with exponent cutoff 20 ln 10 and prefactor cutoff 1e-20; a
 // quartet survives the coarse screen when Q_ij Q_kl >= grad_cutoff.
@@ -1075,7 +1098,7 @@ static int prepare_grad(oqph_session* s) {
   // once, with the bra the later entry of the (bucket, Q) order
   std::vector<int> sbra, sk0, sn;
   std::vector<long long> choff;
-  struct Pend { int la, lb, lc, ld, ck; size_t seg0, ch0; int nseg; long long nwaves; bool f32; };
+  struct Pend { int la, lb, lc, ld, ck; size_t seg0, ch0; int nseg; long long nwaves; bool f32; long long maxcost; };
   std::vector<Pend> pend;
   const int ncls = class_of(s->lmax, s->lmax) + 1;
   for (int cb = 0; cb < ncls; ++cb)
@@ -1141,7 +1164,7 @@ static int prepare_grad(oqph_session* s) {
         waves += (g.n + 63) / 64;
       }
       choff.push_back(waves);
-      pend.push_back({la, lb, lc, ld, ck, seg0, ch0, (int)segs_.size(), waves, f32 != 0});
+      pend.push_back({la, lb, lc, ld, ck, seg0, ch0, (int)segs_.size(), waves, f32 != 0, segs_[0].cost});
       }
     }
   const size_t nseg = sbra.size();
@@ -1164,6 +1187,13 @@ static int prepare_grad(oqph_session* s) {
     L.ww.ket = s->d_gcls.p + coff[p.ck];
     L.ww.nseg = p.nseg;
     L.ww.nwaves = p.nwaves;
+    KernelRes krc{};
+    L.coop = !p.f32 && gradc_class(s, p.la, p.lb, p.lc, p.ld, &krc);
+    if (L.coop) {
+      L.ww.kpb = hl_kpb(s, L.ww.nwaves, krc.lds_bytes + 24 * s->natm, 4);
+      s->glaunches.push_back(L);
+      continue;
+    }
     L.hl = !grad_template(p.la, p.lb, p.lc, p.ld) || (!s->f_templates && (p.la == 3 || p.lc == 3)) ||
            (s->grad_hl_ng > 0 && ncart(p.la) * ncart(p.lb) * ncart(p.lc) * ncart(p.ld) > s->grad_hl_ng);
     if (!L.hl) {  // templates whose private segment exceeds the budget run on k_gradh
@@ -1176,6 +1206,14 @@ static int prepare_grad(oqph_session* s) {
       KernelRes kr{};
       L.f32 = kernel_resources(2 | 16, p.la, p.lb, p.lc, p.ld, s->pure, &kr) &&
               kr.private_bytes <= OQPH_PRIVATE_BUDGET && (size_t)kr.lds_bytes + 24 * (size_t)s->natm <= s->lds_max;
+    }
+    if (!L.hl && !p.f32 && !s->grad_all_hl &&
+        ncart(p.la) * ncart(p.lb) * ncart(p.lc) * ncart(p.ld) <= OQPH_GRAD_SPLIT_NG) {
+      // few wavefronts: several lanes per ket, until the launch has eight
+      // wavefronts per CU or a lane is left with one primitive quartet
+      int kpb = 64;
+      while (kpb > 1 && L.ww.nwaves * (64 / kpb) < 8ll * s->ncu && 2 * (64 / kpb) <= p.maxcost) kpb /= 2;
+      L.ww.kpb = kpb;
     }
     if (L.hl) {
       L.hd = hl_dims(p.la, p.lb, p.lc, p.ld, s->pure, 1, s->natm);
@@ -2649,6 +2687,8 @@ static int grad_run(oqph_session* s, GradParams& p, double* de, oqph_stats* st) 
       launch_gradh_multi(p, L.tl, L.nblocks, L.lds, ls);
     } else if (L.hl) {
       launch_gradh(L.hd, p, L.ww, ls);
+    } else if (L.coop) {
+      launch_gradc(L.la, L.lb, L.lc, L.ld, p, L.ww, ls);
     } else if (!launch_grad(L.la, L.lb, L.lc, L.ld, p, L.ww, ls, L.f32, p.Mc != nullptr)) {
       set_err("no gradient kernel for class (%d %d|%d %d)", L.la, L.lb, L.lc, L.ld);
       return 1;
