@@ -66,7 +66,7 @@ DEPS = {
     "jkc_class.hip": ["jkc_device.h", "jk_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                       "rys_table_f32.inc"],
     "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
-    "session.hip": ["oqph_common.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
+    "session.hip": ["oqph_common.h", "response.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
     "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "gradc_class.hip": ["gradc_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc",
                         "rys_table.inc", "rys_table_f32.inc"],
@@ -74,6 +74,7 @@ DEPS = {
     "hl.hip": ["hl_device.h", "jk_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                "rys_table_f32.inc"],
     "sigma.hip": ["../../include/oqph.h"],
+    "response.hip": ["response.h"],
     "xc.hip": ["../../include/oqph.h", "ao_xform.h", "session_view.h"],
 }
 
@@ -92,7 +93,7 @@ def _key(unit: str, defs) -> str:
 
 def _jobs():
     units = [("session.hip", [], "session.o"), ("dispatch.hip", [], "dispatch.o"), ("int1e.hip", [], "int1e.o"),
-             ("hl.hip", [], "hl.o"), ("sigma.hip", [], "sigma.o"), ("xc.hip", [], "xc.o")]
+             ("hl.hip", [], "hl.o"), ("sigma.hip", [], "sigma.o"), ("xc.hip", [], "xc.o"), ("response.hip", [], "response.o")]
     heavy, light = [], []
     per_class = [(c, "jk_class.hip", "jk") for c in CLASSES + F_JK] + \
                 [(c, "grad_class.hip", "gr") for c in CLASSES + F_GRAD if c not in GRAD_HL] + \

@@ -417,7 +417,7 @@ __global__ void k_jscatter(const ShellPair* pairs, const int* joff, int npair, i
 }
 
 // The per-pair inputs of a J/K build in device-pair order (JKParams::Dk, dpm),
-// and the ket-side Coulomb buffer cleared
+// and the ket-side Coulomb buffer cleared; D null (response pass): dpm only
 __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, int pure, const double* D,
                           const double* dsh, int nsh, double* Dk, double* dpm, double* Jk) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -426,11 +426,12 @@ __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, in
   const int na = (pure && P.la >= 2) ? 2 * P.la + 1 : (P.la + 1) * (P.la + 2) / 2;
   const int nb = (pure && P.lb >= 2) ? 2 * P.lb + 1 : (P.lb + 1) * (P.lb + 2) / 2;
   const int o = joff[i];
-  for (int a = 0; a < na; ++a)
-    for (int b = 0; b < nb; ++b) {
-      Dk[o + a * nb + b] = D[tri_idx_(P.ao_a + a, P.ao_b + b)];
-      Jk[o + a * nb + b] = 0.0;
-    }
+  if (D)
+    for (int a = 0; a < na; ++a)
+      for (int b = 0; b < nb; ++b) {
+        Dk[o + a * nb + b] = D[tri_idx_(P.ao_a + a, P.ao_b + b)];
+        Jk[o + a * nb + b] = 0.0;
+      }
   dpm[i] = dsh[(long long)P.si * nsh + P.sj];
 }
 

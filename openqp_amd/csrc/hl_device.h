@@ -616,6 +616,15 @@ __device__ __forceinline__ void jkh_chunk(const JKParams& prm, const WaveWork& w
     if (Q.sa == Q.sb) deg *= 0.5;
     if (ip == jq) deg *= 0.5;
     if constexpr (GEN) {
+      if (prm.T) {  // dense response pass
+        const TSlots ts{P.sa == P.sb, Q.sa == Q.sb, ip == jq};
+        for (int i = lane; i < h.oa * h.ob * h.oc * h.od; i += HL_BLOCK) {
+          const int d = i % h.od, c = i / h.od % h.oc, ab = i / (h.od * h.oc);
+          const double v = V[i];
+          ts.put(prm, oa + ab / h.ob, ob + ab % h.ob, Q.ao_a + c, Q.ao_b + d, fabs(v) < cut ? 0.0 : v);
+        }
+        continue;
+      }
       hl_general(h, V, P, Q, deg, prm, lane);
       continue;
     }

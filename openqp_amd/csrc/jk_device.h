@@ -408,6 +408,27 @@ __device__ __forceinline__ void count_wave(unsigned long long* ctr, bool pred) {
     atomicAdd(ctr, (unsigned long long)__popcll(m));
 }
 
+// One integral (xy|zw) of the dense response pass into its places of prm.T
+// (cleared before): pairs whose two shells coincide keep x >= y, a quartet of
+// one pair with itself fills each place from its own element.
+struct TSlots {
+  bool same_p, same_q, same_pq;
+  __device__ __forceinline__ void put(const JKParams& prm, int x, int y, int z, int w, double v) const {
+    if (v == 0.0) return;
+    const long long n = prm.nbf, ld = prm.tld;
+    if (!same_p || x >= y) {
+      double* t = prm.T + tri_idx(x, y) * n * ld;
+      t[z * ld + w] = v;
+      if (!same_q) t[w * ld + z] = v;
+    }
+    if (!same_pq && (!same_q || z >= w)) {
+      double* t = prm.T + tri_idx(z, w) * n * ld;
+      t[x * ld + y] = v;
+      if (!same_p) t[y * ld + x] = v;
+    }
+  }
+};
+
 // The class's block of the Boys or root tables is copied into LDS once per block
 // when they fit (FP64 for up to 3 roots, FP32 for every class that has an
 // FP32 path): the table lookups are per-lane gathers at random intervals,
@@ -686,8 +707,8 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
                                                         1.0e-4 * prm.cutoff, prm.inv_mu2, V, nprim);
   }
   count_wave(ctr + 2, lowp && !skip);
-  sum_wave(ctr + 3, (unsigned long long)nprim * flops_prim<LA, LB, LC, LD>() +
-                        (nprim ? (TWO ? 24ull : 12ull) * NOUT : 0ull));
+  const unsigned long long fdig = TWO ? 24ull : prm.T ? 20ull * prm.gnd : 12ull;  // digestion, per integral
+  sum_wave(ctr + 3, (unsigned long long)nprim * flops_prim<LA, LB, LC, LD>() + (nprim ? fdig * NOUT : 0ull));
   sum_wave(ctr + 4, (unsigned long long)nprim);
   const bool valid = !skip && nprim > 0;
   // all lanes stay converged through the digestion; invalid lanes carry V = 0
@@ -703,6 +724,15 @@ __global__ __launch_bounds__(JK_BLOCK) void k_jk(JKParams prm, WaveWork ww) {
   const int oa = P.ao_a, ob = P.ao_b, oc = Q.ao_a, od = Q.ao_b;
   const double* Dp = prm.D;
   double* F = prm.F;
+  if constexpr (!TWO)
+    if (prm.T) {  // dense response pass
+      const TSlots ts{P.sa == P.sb, Q.sa == Q.sb, ip == iq};
+      if (valid)
+#pragma unroll
+        for (int i = 0; i < NOUT; ++i)
+          ts.put(prm, oa + i / (OB * OC * OD), ob + i / (OC * OD) % OB, oc + i / OD % OC, od + i % OD, V[i]);
+      return;
+    }
   // wave-uniform bra: the J_ab block is reduced across the wavefront first
   const unsigned long long vmask = __ballot(valid);
   if (vmask == 0ull) return;  // wave-uniform exit: no lane has anything to digest

@@ -358,6 +358,18 @@ void k_jkc(JKParams prm, WaveWork ww) {
         jab[t] += cj * jt;
       }
     }
+    if constexpr (!TWO)
+      if (prm.T) {  // dense response pass: the integrals themselves
+        const TSlots ts{P.sa == P.sb, Q.sa == Q.sb, ip == jq};
+#pragma unroll
+        for (int t = 0; t < AT; ++t) {
+          const int ab = l + W * t;
+          if (ab < OAB)
+#pragma unroll
+            for (int cd = 0; cd < OCD; ++cd) ts.put(prm, oa + ab / OB, ob + ab % OB, oc + cd / OD, od + cd % OD, V[t][cd]);
+        }
+        continue;
+      }
     __syncthreads();
     // shares of the exchange blocks of row (a, b): K_ac from b, K_ad from b,
     // K_bc from a, K_bd from a; then their sums, one atomic per element
@@ -434,6 +446,7 @@ void k_jkc(JKParams prm, WaveWork ww) {
   // ---- J_ab over the wavefront's kets, statistics
 #pragma unroll
   for (int t = 0; t < AT; ++t) {
+    if (prm.T) break;
     double v = jab[t];
 #pragma unroll
     for (int o = W; o < 64; o <<= 1) v += __shfl_xor(v, o);
@@ -444,7 +457,7 @@ void k_jkc(JKParams prm, WaveWork ww) {
     }
   }
   sum_wave(ctr + 3, (unsigned long long)n_prim * flops_prim<LA, LB, LC, LD>() +
-                        (unsigned long long)n_valid * (TWO ? 24ull : 12ull) * (OAB * OCD));
+                        (unsigned long long)n_valid * (TWO ? 24ull : prm.T ? 20ull * prm.gnd : 12ull) * (OAB * OCD));
   sum_wave(ctr + 4, (unsigned long long)n_prim);
 }
 

@@ -242,4 +242,10 @@ struct JKParams {
   const int* gcoul;
   int gnd;
   int nbf;
+  // Dense form of the response pass: when T is set, a quartet only stores its
+  // integrals, T[tri(x, y)][z][w] = (xy|zw) for every pair x >= y and every z,
+  // w, rows of tld doubles (k_response contracts them with the densities).
+  // D and Dk then point at memory that is read but not used.
+  double* T;
+  int tld;
 };

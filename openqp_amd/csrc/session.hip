@@ -27,6 +27,7 @@
 #include "../../include/oqph.h"
 #include "oqph_common.h"
 #include "grad_params.h"
+#include "response.h"
 #include "session_view.h"
 
 namespace oqph {
@@ -214,15 +215,17 @@ struct oqph_session {
   DBuf<int> d_aooff, d_nao;
   // per build
   DBuf<double> d_D, d_F, d_dsh, d_tmp;
-  DBuf<double> d_gD, d_gF;  // response-pass densities and outputs (nd x nbf x nbf)
-  DBuf<int> d_gcoul;
+  DBuf<double> d_gD, d_gF;  // response-pass densities (nd x nbf x row length) and outputs (nd x nbf x nbf)
+  DBuf<double> d_gR;        // the caller's array, before and after
+  DBuf<double> d_gT;        // integrals of the dense response pass
+  DBuf<int> d_gcoul;        // per density: Coulomb or not; then the two column lists of k_response
   DBuf<long long> d_off;
   DBuf<unsigned long long> d_ctr;
   double cached_maxden = -1.0;
   bool cached_two = false;  // lists prepared for the open-shell pass (K rows of two densities in LDS)
   // response pass over non-symmetric densities (oqph_mrsf_int2): every class
   // on the run-time-class kernel
-  bool general = false, cached_general = false;
+  int general = 0, cached_general = 0;  // lists of a response pass: 1 = k_jkh with its digestion, 2 = dense
   std::vector<long long> h_off;
   struct GLaunch {
     int la, lb, lc, ld;
@@ -1450,17 +1453,19 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
       // templates whose private segment exceeds the budget run on k_jkh instead
       KernelRes kr0{}, kr1{};
       KernelRes krc{};
-      const bool coop = !s->general && !(!s->f_templates && (la == 3 || lc == 3)) &&
+      const bool coop = s->general != 1 && !(!s->f_templates && (la == 3 || lc == 3)) &&
                         jkc_class(s, la, lb, lc, ld, two, nket, &krc);
-      const bool tmpl = !s->general && !coop && jk_template(la, lb, lc, ld) && !(!s->f_templates && (la == 3 || lc == 3)) &&
+      const bool tmpl = s->general != 1 && !coop && jk_template(la, lb, lc, ld) && !(!s->f_templates && (la == 3 || lc == 3)) &&
                         !(s->jk_hl_ng > 0 && ncart(la) * ncart(lb) * ncart(lc) * ncart(ld) > s->jk_hl_ng);
       const int variant = two ? 16 : 0;  // the open-shell kernels when two
       const bool fit0 = tmpl && kernel_resources(0 | variant, la, lb, lc, ld, s->pure, &kr0) &&
                         kr0.private_bytes <= OQPH_PRIVATE_BUDGET;
       const bool fit1 = tmpl && kernel_resources(1 | variant, la, lb, lc, ld, s->pure, &kr1) &&
                         kr1.private_bytes <= OQPH_PRIVATE_BUDGET;
-      const bool hl = !coop && !fit0 && !fit1;
-      bool rows = fit1 && s->rows_mode > 0 && jkb_info(la, lb, lc, ld, s->pure, &nrow, &slds, s->lds_max);
+      // the dense response pass stores from k_jk where it keeps the whole block
+      // in registers, the classes that also have a bra-row kernel
+      const bool hl = !coop && (s->general == 2 ? !(fit0 && fit1) : !fit0 && !fit1);
+      bool rows = fit1 && !s->general && s->rows_mode > 0 && jkb_info(la, lb, lc, ld, s->pure, &nrow, &slds, s->lds_max);
       // dynamic LDS: K rows (nrow x ncol), plus D rows (nrow x ncol) and the
       // bra rows of dsh (2 x nsh) when those fit as well; the open-shell
       // pass holds the K rows (and D rows) of both densities
@@ -2135,20 +2140,44 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   return 0;
 }
 
-// Response pass over nd full nbf x nbf densities (device slabs dD, outputs
-// dF): every class on k_jkh / k_jkh_multi with the general digestion; dsh and
-// maxden come from the caller (the reference's screening density).
-static int build_general(oqph_session* s, int nd, const double* dD, double* dF, const int* dcoul, double maxden,
-                         double se, double sc, oqph_stats* st, hipStream_t stream) {
+// The response pass stores its integrals and contracts them with k_response
+// (session buffer d_gT, npair x nbf x nbf doubles, given back with the session)
+// up to 16 GiB of them (nbf about 250) when that is at most half of the free
+// memory; beyond that, or if the allocation fails, k_jkh adds every quartet into
+// all densities.  One pass, 28 densities, k_jkh -> dense: one water/6-31G 1.9 ->
+// 0.66 ms, (H2O)8/6-31G 50.9 -> 1.75, (H2O)14/6-31G 137 -> 8.1, (H2O)8/cc-pVDZ (192
+// AOs, 5.7 GB) 391 -> 14.6, one water/cc-pVTZ 51 -> 5.5; 7 densities of (H2O)8/6-31G
+// 32 -> 1.4: dense wins at every size it fits.
+static bool response_dense(oqph_session* s) {
+  const char* e = getenv("OQPH_RESPONSE");  // 0: never
+  if (e && e[0] == '0') return false;
+  const size_t n = (size_t)s->nbf, ld = (n + 15) & ~(size_t)15, need = n * (n + 1) / 2 * n * ld;
+  if (need * sizeof(double) > ((size_t)16 << 30)) return false;
+  if (need <= s->d_gT.n && s->d_gT.p) return true;
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess || 2 * need * sizeof(double) > avail || s->d_gT.ensure(need)) {
+    (void)hipGetLastError();  // out of memory: the other path needs none
+    return false;
+  }
+  return true;
+}
+
+// Response pass over nd full nbf x nbf densities (device slabs dD with rows of
+// ldd doubles, outputs dF): with dense the integrals into d_gT and k_response,
+// else every class on k_jkh / k_jkh_multi with the general digestion (ldd =
+// nbf); dsh and maxden come from the caller (the reference's screening density).
+// dcoul: nd Coulomb flags, then the densities 0 .. nd - 1, then the ncoul flagged ones.
+static int build_general(oqph_session* s, bool dense, int nd, const double* dD, int ldd, double* dF, const int* dcoul,
+                         int ncoul, double maxden, double se, double sc, oqph_stats* st, hipStream_t stream) {
   int rc;
   if ((rc = prepare_share(s))) return rc;
   const size_t n2 = (size_t)s->nbf * s->nbf;
   HIPCHK(hipMemsetAsync(dF, 0, (size_t)nd * n2 * sizeof(double), stream));
   if (st) memset(st, 0, sizeof(*st));
   if (maxden <= 0.0) return 0;
-  s->general = true;
+  s->general = dense ? 2 : 1;
   rc = prepare_lists(s, maxden, false);
-  s->general = false;
+  s->general = 0;
   if (rc) return rc;
   const size_t nl = s->launches.size();
   const size_t nc = 8 * (size_t)OQPH_CTR_SLOTS;
@@ -2176,7 +2205,18 @@ static int build_general(oqph_session* s, int nd, const double* dD, double* dF, 
   p.gcoul = dcoul;
   p.gnd = nd;
   p.nbf = s->nbf;
+  const long long n = s->nbf, npair = n * (n + 1) / 2;
   HIPCHK(hipEventRecord(s->ev0, stream));
+  if (dense) {
+    p.T = s->d_gT.p;
+    p.tld = ldd;
+    p.D = dD;
+    p.Dk = s->d_dk.p;
+    p.dpm = s->d_dpm.p;
+    launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, nullptr, s->d_dsh.p, s->nsh, nullptr,
+                   s->d_dpm.p, nullptr, stream);
+    HIPCHK(hipMemsetAsync(p.T, 0, (size_t)(npair * n * ldd) * sizeof(double), stream));
+  }
   const int nst = s->nstreams;
   if ((rc = streams_fork(s, stream, nst))) return rc;
   for (size_t i = 0; i < nl; ++i) {
@@ -2185,13 +2225,23 @@ static int build_general(oqph_session* s, int nd, const double* dD, double* dF, 
     p.counters = ctr + nc * i;
     if (L.multi) launch_jkh_multi(p, L.tl, L.nblocks, (int)L.lds, ls);
     else if (L.hl) launch_jkh(L.hd, p, L.ww, ls);
-    else {
-      set_err("response pass: class (%d %d|%d %d) is not on the run-time-class kernel", L.la, L.lb, L.lc, L.ld);
+    else if (!(dense && L.coop ? launch_jkc(L.la, L.lb, L.lc, L.ld, s->pure, p, L.ww, ls)
+                               : dense && launch_jk(L.la, L.lb, L.lc, L.ld, s->pure, p, L.ww, ls))) {
+      set_err("response pass: no kernel for class (%d %d|%d %d)", L.la, L.lb, L.lc, L.ld);
       return 1;
     }
   }
   HIPCHK(hipGetLastError());
   if ((rc = streams_join(s, stream, nst))) return rc;
+  if (dense) {
+    ResponseParams r{p.T, dD, dF, dcoul + nd, nd, s->nbf, ldd, s->ncu, npair, -se};
+    if (se != 0.0) launch_response(false, r, stream);
+    r.col = dcoul + 2 * nd;
+    r.ncol = ncoul;
+    r.scale = sc;
+    if (sc != 0.0) launch_response(true, r, stream);
+    HIPCHK(hipGetLastError());
+  }
   HIPCHK(hipEventRecord(s->ev1, stream));
   std::vector<unsigned long long> raw(nc * nl);
   if (nl) HIPCHK(hipMemcpyAsync(raw.data(), ctr, nc * nl * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream));
@@ -2303,7 +2353,7 @@ int oqph_session_destroy(oqph_session* s) {
   s->d_am.release(); s->d_pure.release(); s->d_gseg.release(); s->d_gchoff.release(); s->d_Dc.release(); s->d_de.release();
   s->d_aooff.release(); s->d_nao.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
   s->d_tmp.release(); s->d_off.release(); s->d_ctr.release();
-  s->d_gD.release(); s->d_gF.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
+  s->d_gD.release(); s->d_gF.release(); s->d_gR.release(); s->d_gT.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
   for (auto e : s->pev) hipEventDestroy(e);
   if (s->ev0) hipEventDestroy(s->ev0);
   if (s->ev1) hipEventDestroy(s->ev1);
@@ -2605,15 +2655,14 @@ int oqph_mrsf_int2(oqph_session* s, int nf, int nmat, int ncoul, const double* d
   if (rc) return rc;
   const int nbf = s->nbf, nsh = s->nsh;
   const size_t n2 = (size_t)nbf * nbf, nd = (size_t)nf * nmat;
-  // slabs q = v nmat + c, each in the reference's (mu, nu) column order
-  std::vector<double> h(nd * n2);
-  size_t x = 0;
-  for (int nu = 0; nu < nbf; ++nu)
-    for (int mu = 0; mu < nbf; ++mu)
-      for (int c = 0; c < nmat; ++c)
-        for (int v = 0; v < nf; ++v) h[((size_t)v * nmat + c) * n2 + (size_t)nu * nbf + mu] = d3[x++];
-  std::vector<int> coul(nd);
-  for (size_t q = 0; q < nd; ++q) coul[q] = (int)(q % nmat) < ncoul;
+  // densities q = v nmat + c: Coulomb flags, then all, then the flagged ones
+  std::vector<int> coul(3 * nd);
+  size_t nco = 0;
+  for (size_t q = 0; q < nd; ++q) {
+    coul[q] = (int)(q % nmat) < ncoul;
+    coul[nd + q] = (int)q;
+    if (coul[q]) coul[2 * nd + nco++] = (int)q;
+  }
   // shell_den_screen_mrsf (tdhf_mrsf_lib.F90:176-204): the last component
   // only, dsh(i, j) = dsh(j, i) = max |M(mu, nu)|, mu in shell j, nu in
   // shell i >= j
@@ -2622,30 +2671,33 @@ int oqph_mrsf_int2(oqph_session* s, int nf, int nmat, int ncoul, const double* d
   for (int si = 0; si < nsh; ++si)
     for (int sj = 0; sj <= si; ++sj) {
       double dm = 0.0;
-      for (int v = 0; v < nf; ++v) {
-        const double* M = h.data() + ((size_t)v * nmat + nmat - 1) * n2;
-        for (int nu = s->aooff[si]; nu < s->aooff[si] + s->nao[si]; ++nu)
-          for (int mu = s->aooff[sj]; mu < s->aooff[sj] + s->nao[sj]; ++mu) dm = std::max(dm, fabs(M[(size_t)nu * nbf + mu]));
-      }
+      for (int nu = s->aooff[si]; nu < s->aooff[si] + s->nao[si]; ++nu)
+        for (int mu = s->aooff[sj]; mu < s->aooff[sj] + s->nao[sj]; ++mu) {
+          const double* M = d3 + ((size_t)nu * nbf + mu) * nd + (size_t)(nmat - 1) * nf;
+          for (int v = 0; v < nf; ++v) dm = std::max(dm, fabs(M[v]));
+        }
       dsh[(size_t)si * nsh + sj] = dsh[(size_t)sj * nsh + si] = dm;
       maxden = std::max(maxden, dm);
     }
-  if ((rc = s->d_dsh.ensure((size_t)nsh * nsh)) || (rc = s->d_gD.ensure(nd * n2)) ||
-      (rc = s->d_gF.ensure(nd * n2)) || (rc = s->d_gcoul.ensure(nd)))
+  const bool dense = response_dense(s);
+  const int ldd = dense ? (nbf + 15) & ~15 : nbf;
+  if ((rc = s->d_dsh.ensure((size_t)nsh * nsh)) || (rc = s->d_gD.ensure(nd * nbf * ldd)) ||
+      (rc = s->d_gR.ensure(nd * n2)) || (rc = s->d_gF.ensure(nd * n2)) || (rc = s->d_gcoul.ensure(3 * nd)))
     return rc;
-  // synchronous: h, dsh and coul are host locals that an early return frees
-  if ((rc = upload_sync(s->d_gD.p, h.data(), nd * n2 * sizeof(double), s->stream)) ||
+  // synchronous: dsh and coul are host locals that an early return frees
+  if ((rc = upload_sync(s->d_gR.p, d3, nd * n2 * sizeof(double), s->stream)) ||
       (rc = upload_sync(s->d_dsh.p, dsh.data(), dsh.size() * sizeof(double), s->stream)) ||
-      (rc = upload_sync(s->d_gcoul.p, coul.data(), nd * sizeof(int), s->stream)))
+      (rc = upload_sync(s->d_gcoul.p, coul.data(), coul.size() * sizeof(int), s->stream)))
     return rc;
-  if ((rc = build_general(s, (int)nd, s->d_gD.p, s->d_gF.p, s->d_gcoul.p, maxden, se, sc, st, s->stream))) return rc;
-  HIPCHK(hipMemcpyAsync(h.data(), s->d_gF.p, nd * n2 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+  // the reference's (v, c, mu, nu) order into one matrix per density, and back
+  launch_rsp_pack(s->d_gR.p, nbf, ldd, nmat, nf, s->d_gD.p, s->stream);
+  if ((rc = build_general(s, dense, (int)nd, s->d_gD.p, ldd, s->d_gF.p, s->d_gcoul.p, (int)nco, maxden, se, sc, st,
+                          s->stream)))
+    return rc;
+  launch_rsp_unpack(s->d_gF.p, nbf, nmat, nf, s->d_gR.p, s->stream);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(f3, s->d_gR.p, nd * n2 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
-  x = 0;
-  for (int nu = 0; nu < nbf; ++nu)
-    for (int mu = 0; mu < nbf; ++mu)
-      for (int c = 0; c < nmat; ++c)
-        for (int v = 0; v < nf; ++v) f3[x++] = h[((size_t)v * nmat + c) * n2 + (size_t)nu * nbf + mu];
   return 0;
 }
 
