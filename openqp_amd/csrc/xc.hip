@@ -8,22 +8,20 @@
 // alpha = 0.6, per-element xi) times a Gauss-Legendre (cos theta) x uniform
 // (phi) product angular grid, Stratmann-Scuseria-Frisch partition weights
 // (a = 0.64) computed on the device, points with weight <= 1e-20 dropped.
-// The kept points are sorted into cubic boxes (4 bohr) and cut into batches
+// The kept points are sorted into cubic boxes (2 bohr) and cut into batches
 // of at most 32768 points; a batch sees only the shells whose most diffuse
-// primitive reaches its bounding box (|c| exp(-alpha r^2) >= 1e-12).
-// Per-batch matrices are stored point-fastest (column-major npts x nb), so
-// the basis-function and per-point kernels (one thread per point) coalesce.
+// primitive reaches its bounding box (|c| exp(-alpha r^2) >= 2.5e-13).
+// Per-batch matrices are stored point-fastest (element (p, m) at m ld + p), so
+// the kernels with one lane per point coalesce.
 //
-// Per batch and spin: phi, grad phi (k_ao) -> X = phi D_b (rocBLAS dgemm on
-// the gathered D_b) -> per point rho, grad rho, the functional and its
-// derivatives (forward-mode dual numbers), Y = w (vrho/2 phi + v . grad phi)
-// (k_xc_point) -> V_b = phi^T Y (dgemm) -> V += V_b + V_b^T (k_scatter),
-// on three streams (lanes) with their own buffers.
+// Per group of batches, one launch each: phi (k_ao) -> X = phi D_b on the FP64
+// matrix units and rho, grad rho from it (k_rho) -> the functional and its
+// derivatives (forward-mode dual numbers, k_xc_point) -> Y = w (vrho/2 phi + v .
+// grad phi) (k_y) -> V_b = phi^T Y (k_vmat) -> V += V_b (k_vsum); at the end V + V^T.
 // Functionals: Slater, Becke 88, VWN (Ceperley-Alder "VWN5" and RPA fits),
 // Lee-Yang-Parr, combined as libxc combines them for the names the reference
 // accepts (source/dftlib/libxc.F90:300-460).
 #include <hip/hip_runtime.h>
-#include <rocblas/rocblas.h>
 
 #include <algorithm>
 #include <cmath>
@@ -50,10 +48,15 @@ constexpr double PI = 3.14159265358979323846;
 constexpr double RHO_CUT = 1e-10;    // points below this total density contribute nothing
 constexpr double RHO_FLOOR = 1e-30;  // spin densities are floored here
 constexpr double SSF_A = 0.64;
-constexpr double BOX = 4.0;          // bohr
+// bohr; the smaller, the fewer functions reach a batch and the more V_b there are.
+// (H2O)32/6-31G(d): 4 bohr 23.2 ms per build (1.7e11 functions^2 points), 3 19.6, 2 15.9
+// (0.94e11), 1.5 15.5 with twice the batches (13820) of 2
+constexpr double BOX = 2.0;
 constexpr int MAX_BATCH = 32768;
-constexpr int KCHUNK = 2048;         // points per partial V_b (split of the long GEMM dimension)
-constexpr double AO_EPS = 1e-12;
+constexpr long long GROUP_ELEMS = 1ll << 28;  // basis-function values of a group of batches: 2 GB
+// shells below it over a whole box are left out; with 1e-12 and 4-bohr boxes a build's
+// error against exact functions was 7.9e-13 relative, on 2-bohr boxes 9.3e-13
+constexpr double AO_EPS = 2.5e-13;
 
 void err(const char* fmt, ...) __attribute__((format(printf, 1, 2)));
 void err(const char* fmt, ...) {
@@ -330,147 +333,296 @@ __global__ void k_grid(GridArgs g) {
   o[3] = w;
 }
 
-// ------------------------------------------------------------ basis functions
-struct AOArgs {
-  const double* pts;  // batch points, 4 per point
-  int npts, nsh, nb;  // points, significant shells, columns of the batch
-  const int* shl;     // significant shells (session indices)
-  const int* col;     // their first column
-  const int *am, *harm, *atom, *nprim, *poff;
-  const double *ex, *cc, *xyz, *xf;
-  double *phi, *dphi;  // column-major npts x nb (point fastest), 3 of them
-  int grad;
+// ------------------------------------------------------------ batches and groups
+// The batches are cut into groups of at most GROUP_ELEMS basis-function values;
+// a build takes one launch of each kernel per group, over all its batches.  A
+// launch per batch, three gathers of the density and three library products with
+// phi, its gradient, X and Y in memory took 65 ms for (H2O)32/6-31G(d) with its
+// 1045 batches of 4 bohr; this 15.9 (groups of 2^25 values: 28.1 against 23.8 for
+// 2^28, both on boxes of 4 bohr).
+struct DBatch {
+  long long p0;   // first point of the grid
+  long long off;  // first element of the batch's matrices in the group's arrays
+  long long vb;   // first element of its partial V_b in the group's array
+  int npts, ld;   // points, and rounded up to whole tiles of TILE
+  int sh0, nsh, ao0, nb, nparts, pad;
 };
 
-__global__ void k_ao(AOArgs a) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)a.npts * a.nsh) return;
-  const int p = (int)(t % a.npts);
-  const int q = (int)(t / a.npts);
-  const int sh = a.shl[q], l = a.am[sh], A = a.atom[sh];
-  const double dx = a.pts[4 * (size_t)p] - a.xyz[3 * A], dy = a.pts[4 * (size_t)p + 1] - a.xyz[3 * A + 1],
-               dz = a.pts[4 * (size_t)p + 2] - a.xyz[3 * A + 2];
-  const double r2 = dx * dx + dy * dy + dz * dz;
-  double R = 0.0, dR = 0.0;
-  for (int k = 0; k < a.nprim[sh]; ++k) {
-    const double al = a.ex[a.poff[sh] + k], e = a.cc[a.poff[sh] + k] * exp(-al * r2);
-    R += e;
-    dR -= 2.0 * al * e;
-  }
-  const int nc = (l + 1) * (l + 2) / 2;
-  double c[10], gx[10], gy[10], gz[10];
-  double px[5], py[5], pz[5];
+struct AOTab {
+  const int *am, *harm, *atom, *nprim, *poff;
+  const double *ex, *cc, *xyz, *xf;
+};
+
+struct XArgs {
+  AOTab ao;
+  const double* pts;        // 4 per point (weight in [3])
+  const DBatch* batch;      // all batches
+  const int2* tile;         // the group's point tiles: batch, tile of the batch
+  const int4* vt;           // the group's V_b tiles: batch, part, row tile, column tile (batch < 0: none)
+  const int *shl, *col;     // significant shells and their first columns
+  const int* idx;           // AO of every column
+  double *phi, *Y;          // per batch and spin, point fastest: element (p, m) at off + m ld + p
+  double *rho, *coef;       // [spin][4][npad]
+  double* Vb;               // [spin][..]
+  long long npad, ngrp, nvb;  // points of the group in whole tiles; elements of phi; of Vb per spin
+};
+
+constexpr int TILE = 64;
+
+// Components of a shell at one point, in AO order: f(o, value, gradient)
+template <int L, bool PURE, bool GRAD, typename F>
+__device__ __forceinline__ void ao_shell_l(double dx, double dy, double dz, double R, double dR,
+                                           const double* __restrict__ xf, F&& f) {
+  constexpr int NC = (L + 1) * (L + 2) / 2;
+  double px[L + 1], py[L + 1], pz[L + 1];
   px[0] = py[0] = pz[0] = 1.0;
-  for (int k = 1; k <= l + 1 && k < 5; ++k) {
+#pragma unroll
+  for (int k = 1; k <= L; ++k) {
     px[k] = px[k - 1] * dx;
     py[k] = py[k - 1] * dy;
     pz[k] = pz[k - 1] * dz;
   }
-  // canonical order: lx descending, then ly descending
-  int i = 0;
-  for (int lx = l; lx >= 0; --lx)
-    for (int ly = l - lx; ly >= 0; --ly, ++i) {
-      const int lz = l - lx - ly;
+  double c[NC], g[3][GRAD ? NC : 1];
+  int i = 0;  // canonical order: lx descending, then ly descending
+#pragma unroll
+  for (int lx = L; lx >= 0; --lx)
+#pragma unroll
+    for (int ly = L - lx; ly >= 0; --ly) {
+      const int lz = L - lx - ly;
       const double m = px[lx] * py[ly] * pz[lz];
       c[i] = m * R;
-      gx[i] = (lx ? lx * px[lx - 1] * py[ly] * pz[lz] * R : 0.0) + m * dR * dx;
-      gy[i] = (ly ? ly * px[lx] * py[ly - 1] * pz[lz] * R : 0.0) + m * dR * dy;
-      gz[i] = (lz ? lz * px[lx] * py[ly] * pz[lz - 1] * R : 0.0) + m * dR * dz;
-    }
-  const size_t ld = (size_t)a.npts, row = (size_t)a.col[q] * ld + p, plane = (size_t)a.npts * a.nb;
-  if (l < 2) {
-    for (int o = 0; o < nc; ++o) {
-      a.phi[row + o * ld] = c[o];
-      if (a.grad) {
-        a.dphi[row + o * ld] = gx[o];
-        a.dphi[plane + row + o * ld] = gy[o];
-        a.dphi[2 * plane + row + o * ld] = gz[o];
+      if constexpr (GRAD) {
+        g[0][i] = (lx ? lx * px[lx > 0 ? lx - 1 : 0] * py[ly] * pz[lz] * R : 0.0) + m * dR * dx;
+        g[1][i] = (ly ? ly * px[lx] * py[ly > 0 ? ly - 1 : 0] * pz[lz] * R : 0.0) + m * dR * dy;
+        g[2][i] = (lz ? lz * px[lx] * py[ly] * pz[lz > 0 ? lz - 1 : 0] * R : 0.0) + m * dR * dz;
       }
+      ++i;
     }
-    return;
-  }
-  const int pure = a.harm[sh] ? 1 : 0;
-  const int no = pure ? 2 * l + 1 : nc;
-  const double* X = a.xf + ((l - 2) * 2 + pure) * 100;
-  for (int o = 0; o < no; ++o) {
-    double v = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
-    for (int k = 0; k < nc; ++k) {
-      const double f = X[o * 10 + k];
-      v += f * c[k];
-      vx += f * gx[k];
-      vy += f * gy[k];
-      vz += f * gz[k];
-    }
-    a.phi[row + o * ld] = v;
-    if (a.grad) {
-      a.dphi[row + o * ld] = vx;
-      a.dphi[plane + row + o * ld] = vy;
-      a.dphi[2 * plane + row + o * ld] = vz;
+  if constexpr (L < 2) {
+#pragma unroll
+    for (int o = 0; o < NC; ++o) f(o, c[o], GRAD ? g[0][o] : 0.0, GRAD ? g[1][o] : 0.0, GRAD ? g[2][o] : 0.0);
+  } else {
+    constexpr int NO = PURE ? 2 * L + 1 : NC;
+    const double* X = xf + ((L - 2) * 2 + (PURE ? 1 : 0)) * 100;
+#pragma unroll
+    for (int o = 0; o < NO; ++o) {
+      double v = 0.0, vx = 0.0, vy = 0.0, vz = 0.0;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        const double x = X[o * 10 + k];
+        v += x * c[k];
+        if constexpr (GRAD) {
+          vx += x * g[0][k];
+          vy += x * g[1][k];
+          vz += x * g[2][k];
+        }
+      }
+      f(o, v, vx, vy, vz);
     }
   }
 }
 
-// ------------------------------------------------------------ per-point XC
-struct PointArgs {
-  const double* pts;  // 4 per point (weight in [3])
-  int npts, nb, ns, gga;
-  const double *phi, *dphi, *X;  // X: ns x npts x nb
-  double* Y;                     // ns x npts x nb
-  double* acc;                   // [0] E_xc, [1] N_elec
-  XCFunc f;
-};
+// one shell (wavefront-uniform) at the lane's point
+template <bool GRAD, typename F>
+__device__ __forceinline__ void ao_shell(const AOTab& t, int sh, const double* r, F&& f) {
+  const int l = t.am[sh], A = t.atom[sh], n = t.nprim[sh], k0 = t.poff[sh];
+  const double dx = r[0] - t.xyz[3 * A], dy = r[1] - t.xyz[3 * A + 1], dz = r[2] - t.xyz[3 * A + 2];
+  const double r2 = dx * dx + dy * dy + dz * dz;
+  double R = 0.0, dR = 0.0;
+  for (int k = 0; k < n; ++k) {
+    const double al = t.ex[k0 + k], e = t.cc[k0 + k] * exp(-al * r2);
+    R += e;
+    if constexpr (GRAD) dR -= 2.0 * al * e;
+  }
+  if (l == 0) ao_shell_l<0, false, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+  else if (l == 1) ao_shell_l<1, false, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+  else if (l == 2 && t.harm[sh]) ao_shell_l<2, true, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+  else if (l == 2) ao_shell_l<2, false, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+  else if (t.harm[sh]) ao_shell_l<3, true, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+  else ao_shell_l<3, false, GRAD>(dx, dy, dz, R, dR, t.xf, f);
+}
+
+// the lane's point of tile t (the last one again past the end), its coordinates
+__device__ __forceinline__ long long tile_point(const XArgs& a, const DBatch& b, int t, int lane, double* r) {
+  const long long p = b.p0 + min(t * TILE + lane, b.npts - 1);
+  for (int k = 0; k < 3; ++k) r[k] = a.pts[4 * p + k];
+  return p;
+}
+
+// phi of one tile; a wavefront takes every fourth shell.  Bound by the 8 bytes it
+// writes per value.  The gradients are evaluated again where they are used
+// (k_rho, k_y): an exponential per primitive costs less than writing and reading
+// three more arrays.
+__global__ __launch_bounds__(256) void k_ao(XArgs a) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int2 tl = a.tile[blockIdx.x];
+  const DBatch b = a.batch[tl.x];
+  double r[3];
+  tile_point(a, b, tl.y, lane, r);
+  for (int q = wave; q < b.nsh; q += 4) {
+    const int sh = a.shl[b.sh0 + q];
+    double* out = a.phi + b.off + (size_t)a.col[b.sh0 + q] * b.ld + tl.y * TILE + lane;
+    ao_shell<false>(a.ao, sh, r, [&](int o, double v, double, double, double) { out[(size_t)o * b.ld] = v; });
+  }
+}
+
+// ------------------------------------------------------------ density on the grid
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+
+// rho and grad rho of one tile and spin: X = phi D_b on the FP64 matrix units,
+// NV tiles of 16 columns per wavefront; phi through LDS (the four wavefronts share
+// it), D through the column list (it stays in L2).  X meets phi and grad phi,
+// evaluated per lane = point, through LDS and is never written.  Bound by the matrix
+// units next to the exponentials: 7.0 ms for 9.4e10 columns^2 points ((H2O)32/
+// 6-31G(d)), of which 5.1 the product (37 TFLOP/s) and 3.1 the functions alone.  Three
+// wavefronts per SIMD (112 bytes of scratch in the f path) 7.0, two 7.6 ms; one pass
+// over up to 192 columns with 12 tiles in registers 8.1.
+template <int NV>
+__device__ __forceinline__ void rho_pass(const double* __restrict__ ph, const double* __restrict__ Ds, int nbf, int nb,
+                                         int ld, const int* s_idx, double* s_a, int n0, v4d (&acc)[4][2]) {
+  constexpr int AS = 80;  // row length of the staged phi: rows 32 banks apart
+  const int lane = threadIdx.x & 63, row = lane & 15, g = lane >> 4, sk = threadIdx.x >> 4, sp = (threadIdx.x & 15) * 4;
+  const double* Dn[NV];
+#pragma unroll
+  for (int j = 0; j < NV; ++j) Dn[j] = Ds + s_idx[min(n0 + 16 * j + row, nb - 1)];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int j = 0; j < NV; ++j) acc[t][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  v2d ra[2];
+  double rb[4][NV];
+  auto fetch = [&](int m0) {
+    const bool ok = m0 + sk < nb;
+    const double* pa = ph + (size_t)min(m0 + sk, nb - 1) * ld + sp;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) ra[h] = ok ? *(const v2d*)(pa + 2 * h) : v2d{0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const size_t dr = (size_t)s_idx[min(m0 + 4 * k + g, nb - 1)] * nbf;
+#pragma unroll
+      for (int j = 0; j < NV; ++j) rb[k][j] = Dn[j][dr];
+    }
+  };
+  fetch(0);
+  for (int m0 = 0, cur = 0; m0 < nb; m0 += 16, cur ^= 1) {
+    double* A = s_a + cur * 16 * AS;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) *(v2d*)(A + sk * AS + sp + 2 * h) = ra[h];
+    double y[4][NV];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int j = 0; j < NV; ++j) y[k][j] = rb[k][j];
+    __syncthreads();
+    if (m0 + 16 < nb) fetch(m0 + 16);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double x[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[t] = A[(4 * k + g) * AS + 16 * t + row];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) acc[t][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], y[k][j], acc[t][j], 0, 0, 0);
+    }
+  }
+  __syncthreads();
+}
+
+template <bool GGA>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_rho(XArgs a,
+                                                                                   const double* __restrict__ D, int nbf) {
+  extern __shared__ __align__(16) double s_dyn[];
+  constexpr int XS = 16 * (TILE + 1);
+  const int lane = threadIdx.x & 63, row = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double* s_x = s_dyn + wave * XS;
+  int* s_idx = (int*)(s_dyn + 4 * XS);
+  const int2 tl = a.tile[blockIdx.x];
+  const DBatch b = a.batch[tl.x];
+  const int nb = b.nb, ld = b.ld;
+  for (int i = threadIdx.x; i < nb; i += 256) s_idx[i] = a.idx[b.ao0 + i];
+  __syncthreads();
+  const double* Ds = D + (size_t)blockIdx.y * nbf * nbf;
+  double r[3];
+  tile_point(a, b, tl.y, lane, r);
+  const double* ph = a.phi + b.off + tl.y * TILE;
+  double o0 = 0.0, o1 = 0.0, o2 = 0.0, o3 = 0.0;
+  int q = 0;  // first shell that reaches the present columns
+  for (int base = 0; base < nb;) {
+    // 128 columns, or 64 where no more are left
+    const int nv = nb - base <= 64 ? 1 : 2, n0 = base + 16 * nv * wave;
+    v4d acc[4][2];
+    if (nv == 1) rho_pass<1>(ph, Ds, nbf, nb, ld, s_idx, s_dyn, n0, acc);
+    else rho_pass<2>(ph, Ds, nbf, nb, ld, s_idx, s_dyn, n0, acc);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int c0 = n0 + 16 * j;
+      if (j >= nv || c0 >= nb) break;
+      // element i of a lane's result: point 16 t + 4 i + lane / 16, column lane % 16
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s_x[row * (TILE + 1) + 16 * t + 4 * i + g] = acc[t][j][i];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      while (q + 1 < b.nsh && a.col[b.sh0 + q + 1] <= c0) ++q;
+      for (int k = q; k < b.nsh && a.col[b.sh0 + k] < c0 + 16; ++k) {
+        const int cs = a.col[b.sh0 + k] - c0;
+        ao_shell<GGA>(a.ao, a.shl[b.sh0 + k], r, [&](int o, double v, double vx, double vy, double vz) {
+          const int c = cs + o;
+          if (c < 0 || c >= 16) return;
+          const double x = s_x[c * (TILE + 1) + lane];
+          o0 += x * v;
+          if constexpr (GGA) {
+            o1 += x * vx;
+            o2 += x * vy;
+            o3 += x * vz;
+          }
+        });
+      }
+    }
+    base += 64 * nv;
+    __syncthreads();
+  }
+  double* red = s_dyn + wave * 4 * TILE;
+  red[lane] = o0;
+  red[TILE + lane] = o1;
+  red[2 * TILE + lane] = o2;
+  red[3 * TILE + lane] = o3;
+  __syncthreads();
+  // thread = (quantity, point): the sum over the four wavefronts
+  double v = 0.0;
+  for (int w = 0; w < 4; ++w) v += s_dyn[w * 4 * TILE + threadIdx.x];
+  a.rho[((size_t)blockIdx.y * 4 + wave) * a.npad + (size_t)blockIdx.x * TILE + lane] = v;
+}
 
 __device__ inline double wsum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
-// 64 points per block (one per lane) x XC_SLICES wavefronts that split the
-// basis functions; matrices point-fastest: element (p, m) at m npts + p
-#define XC_SLICES 8
-__global__ __launch_bounds__(64 * XC_SLICES) void k_xc_point(PointArgs a) {
-  const int lane = threadIdx.x & 63, sl = threadIdx.x >> 6;
-  const long long p = (long long)blockIdx.x * 64 + lane;
-  __shared__ double part[XC_SLICES][2][4][64];  // per slice: rho, grad rho per spin
-  __shared__ double coef[2][4][64];             // per spin: c0, v (3)
-  __shared__ double red[2][64];
-  const bool live = p < a.npts;
-  const int n = a.nb;
-  const size_t ld = (size_t)a.npts, plane = ld * n;
-  const int m0 = (int)((long long)n * sl / XC_SLICES), m1 = (int)((long long)n * (sl + 1) / XC_SLICES);
-  for (int s = 0; s < a.ns; ++s) {
-    double r = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
-    if (live) {
-      const double* X = a.X + s * plane + p;
-      const double* phi = a.phi + p;
-      const double* gp = a.dphi + p;
-      if (a.gga) {
-        for (int m = m0; m < m1; ++m) {
-          const double x = X[m * ld];
-          r += x * phi[m * ld];
-          g0 += x * gp[m * ld];
-          g1 += x * gp[plane + m * ld];
-          g2 += x * gp[2 * plane + m * ld];
-        }
-      } else {
-        for (int m = m0; m < m1; ++m) r += X[m * ld] * phi[m * ld];
-      }
+// The functional, lane = point: rho, grad rho -> the coefficients of phi and grad
+// phi in Y; E_xc and the electron count into acc
+__global__ __launch_bounds__(256) void k_xc_point(XArgs a, long long ntile, int ns, XCFunc f, double* acc) {
+  const int lane = threadIdx.x & 63;
+  double es = 0.0, nel = 0.0;
+  for (long long tile = (long long)blockIdx.x * 4 + (threadIdx.x >> 6); tile < ntile; tile += 4ll * gridDim.x) {
+    const int2 tl = a.tile[tile];
+    const DBatch& b = a.batch[tl.x];
+    const int p = tl.y * TILE + lane;
+    const size_t at = (size_t)tile * TILE + lane;
+    const bool live = p < b.npts;
+    double rho[2], g[2][3];
+    for (int s = 0; s < ns; ++s) {
+      rho[s] = a.rho[(size_t)s * 4 * a.npad + at];
+      for (int k = 0; k < 3; ++k) g[s][k] = 2.0 * a.rho[((size_t)s * 4 + k + 1) * a.npad + at];
     }
-    part[sl][s][0][lane] = r;
-    part[sl][s][1][lane] = g0;
-    part[sl][s][2][lane] = g1;
-    part[sl][s][3][lane] = g2;
-  }
-  __syncthreads();
-  if (sl == 0) {
-    double rho[2] = {0.0, 0.0}, g[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
-    for (int s = 0; s < a.ns; ++s)
-      for (int j = 0; j < XC_SLICES; ++j) {
-        rho[s] += part[j][s][0][lane];
-        for (int k = 0; k < 3; ++k) g[s][k] += 2.0 * part[j][s][k + 1][lane];
-      }
     double ra, rb, ga[3], gb[3];
-    if (a.ns == 1) {
+    if (ns == 1) {
       ra = rb = 0.5 * rho[0];
       for (int k = 0; k < 3; ++k) ga[k] = gb[k] = 0.5 * g[0][k];
     } else {
@@ -481,15 +633,15 @@ __global__ __launch_bounds__(64 * XC_SLICES) void k_xc_point(PointArgs a) {
         gb[k] = g[1][k];
       }
     }
-    const double w = live ? a.pts[4 * p + 3] : 0.0, rt = ra + rb;
-    double e = 0.0, c0[2] = {0.0, 0.0}, vec[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+    const double w = live ? a.pts[4 * (b.p0 + p) + 3] : 0.0, rt = ra + rb;
+    double c0[2] = {0.0, 0.0}, vec[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
     if (live && rt >= RHO_CUT) {
       const double saa = ga[0] * ga[0] + ga[1] * ga[1] + ga[2] * ga[2];
       const double sab = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
       const double sbb = gb[0] * gb[0] + gb[1] * gb[1] + gb[2] * gb[2];
-      const Dual F = energy_density(a.f, var(fmax(ra, RHO_FLOOR), 0), var(fmax(rb, RHO_FLOOR), 1), var(saa, 2),
+      const Dual F = energy_density(f, var(fmax(ra, RHO_FLOOR), 0), var(fmax(rb, RHO_FLOOR), 1), var(saa, 2),
                                     var(sab, 3), var(sbb, 4));
-      e = w * F.v;
+      es += w * F.v;
       c0[0] = 0.5 * w * F.d[0];
       c0[1] = 0.5 * w * F.d[1];
       for (int k = 0; k < 3; ++k) {
@@ -497,37 +649,148 @@ __global__ __launch_bounds__(64 * XC_SLICES) void k_xc_point(PointArgs a) {
         vec[1][k] = w * (2.0 * F.d[4] * gb[k] + F.d[3] * ga[k]);
       }
     }
-    for (int s = 0; s < 2; ++s) {
-      coef[s][0][lane] = c0[s];
-      for (int k = 0; k < 3; ++k) coef[s][k + 1][lane] = vec[s][k];
+    if (live) nel += w * rt;
+    for (int s = 0; s < ns; ++s) {
+      a.coef[(size_t)s * 4 * a.npad + at] = c0[s];
+      for (int k = 0; k < 3; ++k) a.coef[((size_t)s * 4 + k + 1) * a.npad + at] = vec[s][k];
     }
-    red[0][lane] = e;
-    red[1][lane] = w * rt;
   }
-  __syncthreads();
-  if (live)
-    for (int s = 0; s < a.ns; ++s) {
-      const double c = coef[s][0][lane], v0 = coef[s][1][lane], v1 = coef[s][2][lane], v2 = coef[s][3][lane];
-      double* Y = a.Y + s * plane + p;
-      const double* phi = a.phi + p;
-      const double* gp = a.dphi + p;
-      if (a.gga) {
-        for (int m = m0; m < m1; ++m)
-          Y[m * ld] = c * phi[m * ld] + v0 * gp[m * ld] + v1 * gp[plane + m * ld] + v2 * gp[2 * plane + m * ld];
-      } else {
-        for (int m = m0; m < m1; ++m) Y[m * ld] = c * phi[m * ld];
-      }
-    }
-  if (sl == 0) {
-    const double e = wsum(red[0][lane]), nel = wsum(red[1][lane]);
-    if (lane == 0) {
-      atomicAdd(a.acc, e);
-      atomicAdd(a.acc + 1, nel);
-    }
+  es = wsum(es);
+  nel = wsum(nel);
+  if (lane == 0) {
+    atomicAdd(acc, es);
+    atomicAdd(acc + 1, nel);
   }
 }
 
-// ------------------------------------------------------------ gathers and packing
+// Y = c phi + v . grad phi of one tile and spin, as k_ao; zero past the batch's points
+template <bool GGA>
+__global__ __launch_bounds__(256) void k_y(XArgs a) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int2 tl = a.tile[blockIdx.x];
+  const DBatch b = a.batch[tl.x];
+  double r[3];
+  tile_point(a, b, tl.y, lane, r);
+  const double* cf = a.coef + (size_t)blockIdx.y * 4 * a.npad + (size_t)blockIdx.x * TILE + lane;
+  const double c = cf[0], c1 = cf[a.npad], c2 = cf[2 * a.npad], c3 = cf[3 * a.npad];
+  for (int q = wave; q < b.nsh; q += 4) {
+    const int sh = a.shl[b.sh0 + q];
+    double* out = a.Y + (size_t)blockIdx.y * a.ngrp + b.off + (size_t)a.col[b.sh0 + q] * b.ld + tl.y * TILE + lane;
+    ao_shell<GGA>(a.ao, sh, r, [&](int o, double v, double vx, double vy, double vz) {
+      out[(size_t)o * b.ld] = GGA ? c * v + c1 * vx + c2 * vy + c3 * vz : c * v;
+    });
+  }
+}
+
+// One 64 x 64 tile of V_b = phi^T Y over PART points, 32 x 32 per wavefront on the
+// FP64 matrix units, 16 points at a time through LDS (two buffers, the loads of the
+// next PF steps in flight).  A lane takes 4 consecutive points of its rows; which
+// point is the k-th of a matrix instruction does not matter as long as both sides
+// agree.  Bound by the loads' latency next to the matrix units: 4.28 ms for 9.4e10
+// columns^2 points (44 TFLOP/s); one step ahead 4.7, straight from memory without
+// LDS 6.9, tiles of 128 x 128 on eight wavefronts 4.8, columns cut evenly 5.0.
+constexpr int PART = 2048;
+__global__ __launch_bounds__(256) void k_vmat(XArgs a) {
+  constexpr int RS = 18, PF = 2;  // row length in LDS: 16 rows fall on distinct banks
+  __shared__ __align__(16) double s_t[2][2][64 * RS];
+  const int4 e = a.vt[blockIdx.x];
+  if (e.x < 0) return;
+  const DBatch b = a.batch[e.x];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = lane & 15, g = lane >> 4;
+  const int nb = b.nb, ld = b.ld, mw = 32 * (wave & 1), nw = 32 * (wave >> 1);
+  const int m0 = 64 * e.z + mw, n0 = 64 * e.w + nw;
+  // staging: thread = (row, 4 points)
+  const int sr = threadIdx.x >> 2, sp = (threadIdx.x & 3) * 4;
+  const double* A = a.phi + b.off + (size_t)min(64 * e.z + sr, nb - 1) * ld + sp;
+  const double* B = a.Y + (size_t)blockIdx.y * a.ngrp + b.off + (size_t)min(64 * e.w + sr, nb - 1) * ld + sp;
+  v4d acc[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[t][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  const int p0 = e.y * PART, p1 = min(p0 + PART, ld);
+  v2d ra[PF][2], rb[PF][2];
+  auto fetch = [&](int f, int p) {
+    p = min(p, p1 - 16);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      ra[f][h] = *(const v2d*)(A + p + 2 * h);
+      rb[f][h] = *(const v2d*)(B + p + 2 * h);
+    }
+  };
+#pragma unroll
+  for (int f = 0; f < PF; ++f) fetch(f, p0 + 16 * f);
+  int cur = 0;
+  for (int pp = p0; pp < p1; pp += 16 * PF)  // whole tiles of points: a multiple of 64
+#pragma unroll
+    for (int f = 0; f < PF; ++f, cur ^= 1) {
+      double *sa = s_t[cur][0], *sb = s_t[cur][1];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        *(v2d*)(sa + sr * RS + sp + 2 * h) = ra[f][h];
+        *(v2d*)(sb + sr * RS + sp + 2 * h) = rb[f][h];
+      }
+      __syncthreads();
+      fetch(f, pp + 16 * (f + PF));
+      v2d x[2][2], y[2][2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          x[t][h] = *(const v2d*)(sa + (mw + 16 * t + row) * RS + 4 * g + 2 * h);
+          y[t][h] = *(const v2d*)(sb + (nw + 16 * t + row) * RS + 4 * g + 2 * h);
+        }
+      // 16 x 16 sub-tiles past the batch's columns are left out (wavefront-uniform)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (m0 + 16 * t < nb && n0 + 16 * j < nb)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              acc[t][j] =
+                  __builtin_amdgcn_mfma_f64_16x16x4f64(x[t][k / 2][k % 2], y[j][k / 2][k % 2], acc[t][j], 0, 0, 0);
+    }
+  double* V = a.Vb + (size_t)blockIdx.y * a.nvb + b.vb + (size_t)e.y * nb * nb;
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 16 * t + 4 * i + g, n = n0 + 16 * j + row;
+        if (m < nb && n < nb) V[(size_t)m * nb + n] = acc[t][j][i];
+      }
+}
+
+// V(i, .) += the rows of the group's V_b that belong to AO i: block = (i, VCOLS
+// columns), a wavefront per batch that holds i, the row collected in LDS
+constexpr int VCOLS = 4096;
+__global__ __launch_bounds__(512) void k_vsum(XArgs a, const long long* __restrict__ ptr, const int2* __restrict__ ent,
+                                              int nbf, double* V) {
+  extern __shared__ double s_row[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = blockIdx.x, c0 = blockIdx.y * VCOLS, nc = min(VCOLS, nbf - c0);
+  for (int j = threadIdx.x; j < nc; j += 512) s_row[j] = 0.0;
+  __syncthreads();
+  for (long long k = ptr[i] + wave; k < ptr[i + 1]; k += 8) {
+    const int2 e = ent[k];  // batch, column of i
+    const DBatch& b = a.batch[e.x];
+    const int nb = b.nb;
+    const double* x = a.Vb + (size_t)blockIdx.z * a.nvb + b.vb + (size_t)e.y * nb;
+    for (int n = lane; n < nb; n += 64) {
+      double v = 0.0;
+      for (int s = 0; s < b.nparts; ++s) v += x[(size_t)s * nb * nb + n];
+      const int c = a.idx[b.ao0 + n] - c0;
+      if (c >= 0 && c < nc) unsafeAtomicAdd(&s_row[c], v);
+    }
+  }
+  __syncthreads();
+  double* row = V + ((size_t)blockIdx.z * nbf + i) * nbf + c0;
+  for (int j = threadIdx.x; j < nc; j += 512) row[j] += s_row[j];
+}
+
+// ------------------------------------------------------------ packing
 __global__ void k_unpack(const double* pk, int nbf, double* full) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= (long long)nbf * nbf) return;
@@ -536,31 +799,8 @@ __global__ void k_unpack(const double* pk, int nbf, double* full) {
   full[t] = pk[(size_t)hi * (hi + 1) / 2 + lo];
 }
 
-__global__ void k_gather(const double* full, int nbf, const int* idx, int nb, double* out) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)nb * nb) return;
-  const int i = (int)(t / nb), j = (int)(t % nb);
-  out[t] = full[(size_t)idx[i] * nbf + idx[j]];
-}
-
-// V[idx[m], idx[n]] += sum over the nparts partials of Vb(m, n) + Vb(n, m);
-// each partial column-major nb x nb
-__global__ void k_scatter(const double* Vb, int nb, int nparts, const int* idx, int nbf, double* V) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)nb * nb) return;
-  const int m = (int)(t % nb), n = (int)(t / nb);
-  const size_t nb2 = (size_t)nb * nb;
-  double v = 0.0;
-  for (int k = 0; k < nparts; ++k) v += Vb[k * nb2 + (size_t)n * nb + m] + Vb[k * nb2 + (size_t)m * nb + n];
-  V[(size_t)idx[m] * nbf + idx[n]] += v;
-}
-
-// packed lower triangle of the sum of the lanes' matrices
-struct LaneSum {
-  const double* v[4];
-  int n;
-};
-__global__ void k_pack(LaneSum ls, int nbf, double* pk) {
+// packed lower triangle of V + V^T
+__global__ void k_pack(const double* V, int nbf, double* pk) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const long long ntri = (long long)nbf * (nbf + 1) / 2;
   if (t >= ntri) return;
@@ -568,9 +808,7 @@ __global__ void k_pack(LaneSum ls, int nbf, double* pk) {
   while ((long long)i * (i + 1) / 2 > t) --i;
   while ((long long)(i + 1) * (i + 2) / 2 <= t) ++i;
   const int j = (int)(t - (long long)i * (i + 1) / 2);
-  double v = 0.0;
-  for (int k = 0; k < ls.n; ++k) v += ls.v[k][(size_t)i * nbf + j];
-  pk[t] = v;
+  pk[t] = V[(size_t)i * nbf + j] + V[(size_t)j * nbf + i];
 }
 
 inline unsigned nblk(long long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
@@ -605,26 +843,10 @@ struct Batch {
   int npts, sh0, nsh, ao0, nb;
 };
 
-// a stream with its own batch buffers, GEMM handle and Vxc accumulator;
-// batches go round-robin over the lanes so that the GEMMs of one overlap the
-// memory-bound kernels of the others (three measured fastest: two and four
-// lanes were 12 % and 8 % slower)
-constexpr int XC_LANES = 3;
-static_assert(XC_LANES >= 1 && XC_LANES <= 4, "k_pack sums at most four lanes");
-struct Lane {
-  hipStream_t st = nullptr;
-  hipEvent_t done = nullptr;
-  rocblas_handle blas = nullptr;
-  Buf<double> phi, dphi, X, Y, Db, Vb, V;
-  void release() {
-    for (auto* b : {&phi, &dphi, &X, &Y, &Db, &Vb, &V}) b->release();
-    if (blas) rocblas_destroy_handle(blas);
-    if (done) hipEventDestroy(done);
-    if (st) hipStreamDestroy(st);
-    blas = nullptr;
-    done = nullptr;
-    st = nullptr;
-  }
+// batches [b0, b1) built together
+struct Group {
+  int b0, b1;
+  long long tile0, ntile, vt0, nvt, ngrp, nvb;
 };
 
 struct XCState {
@@ -638,18 +860,26 @@ struct XCState {
   bool grid_ready = false;
   std::vector<double> grid;  // kept points (x, y, z, w), atom-major
   std::vector<Batch> batches;
-  int max_nb = 0, max_pts = 0;
-  Buf<double> d_pts, d_xf, d_D, d_pk, d_acc;
+  std::vector<Group> groups;
+  int max_nb = 0;
+  long long max_grp = 0, max_vb = 0, max_tile = 0;  // largest group: phi, V_b, point tiles
+  Buf<double> d_pts, d_xf, d_D, d_pk, d_acc, d_phi, d_Y, d_rho, d_coef, d_Vb, d_V;
+  Buf<DBatch> d_batch;
+  Buf<int2> d_tile;
+  Buf<int4> d_vt;
+  Buf<long long> d_vptr;
+  Buf<int2> d_vent;
   Buf<int> d_shl, d_col, d_idx, d_am, d_harm, d_atom, d_nprim, d_poff;
   Buf<double> d_ex, d_cc, d_xyz;
-  Lane lane[XC_LANES];
-  hipEvent_t ready = nullptr;
   void release() {
-    for (auto* b : {&d_pts, &d_xf, &d_D, &d_pk, &d_acc, &d_ex, &d_cc, &d_xyz}) b->release();
+    for (auto* b : {&d_pts, &d_xf, &d_D, &d_pk, &d_acc, &d_phi, &d_Y, &d_rho, &d_coef, &d_Vb, &d_V, &d_ex, &d_cc, &d_xyz})
+      b->release();
+    d_batch.release();
+    d_tile.release();
+    d_vt.release();
+    d_vptr.release();
+    d_vent.release();
     for (auto* b : {&d_shl, &d_col, &d_idx, &d_am, &d_harm, &d_atom, &d_nprim, &d_poff}) b->release();
-    for (auto& l : lane) l.release();
-    if (ready) hipEventDestroy(ready);
-    ready = nullptr;
     grid_ready = false;
   }
 };
@@ -810,7 +1040,6 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
   std::vector<int> shl, col, idx;
   x->batches.clear();
   x->max_nb = 0;
-  x->max_pts = 0;
   for (long long t0 = 0; t0 < n;) {
     long long t1 = t0;
     while (t1 < n && key[order[t1]] == key[order[t0]] && t1 - t0 < MAX_BATCH) ++t1;
@@ -841,9 +1070,57 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
     if (b.nsh > 0) {
       x->batches.push_back(b);
       x->max_nb = std::max(x->max_nb, b.nb);
-      x->max_pts = std::max(x->max_pts, b.npts);
     }
     t0 = t1;
+  }
+  // groups of batches, their point tiles and V_b tiles
+  std::vector<DBatch> db;
+  std::vector<int2> tile;
+  std::vector<int4> vt;
+  std::vector<long long> vptr;  // per group: nbf + 1 starts in vent
+  std::vector<int2> vent;       // per AO: the batches that hold it and its column there
+  x->groups.clear();
+  long long max_grp = 0, max_vb = 0, max_tile = 0;
+  for (int b0 = 0; b0 < (int)x->batches.size();) {
+    Group g{b0, b0, (long long)tile.size(), 0, (long long)vt.size(), 0, 0, 0};
+    std::vector<int4> list[8];  // tiles of a part stay on one XCD: blocks are dealt to the eight in turn
+    while (g.b1 < (int)x->batches.size()) {
+      const Batch& b = x->batches[g.b1];
+      const int ld = (b.npts + TILE - 1) / TILE * TILE, nparts = (ld + PART - 1) / PART, nt = (b.nb + 63) / 64;
+      const long long phi = (long long)ld * b.nb, vb = (long long)nparts * b.nb * b.nb;
+      if (g.b1 > b0 && (g.ngrp + phi > GROUP_ELEMS || g.nvb + vb > GROUP_ELEMS)) break;
+      db.push_back({b.p0, g.ngrp, g.nvb, b.npts, ld, b.sh0, b.nsh, b.ao0, b.nb, nparts, 0});
+      for (int t = 0; t < ld / TILE; ++t) tile.push_back(int2{g.b1, t});
+      for (int k = 0; k < nparts; ++k) {
+        auto& l = *std::min_element(list, list + 8, [](const auto& p, const auto& q) { return p.size() < q.size(); });
+        for (int m = 0; m < nt; ++m)
+          for (int c = 0; c < nt; ++c) l.push_back(int4{g.b1, k, m, c});
+      }
+      g.ngrp += phi;
+      g.nvb += vb;
+      ++g.b1;
+    }
+    size_t len = 0;
+    for (auto& l : list) len = std::max(len, l.size());
+    for (size_t i = 0; i < len; ++i)
+      for (auto& l : list) vt.push_back(i < l.size() ? l[i] : int4{-1, 0, 0, 0});
+    const size_t p0 = vptr.size(), e0 = vent.size();
+    vptr.resize(p0 + v.nbf + 1, 0);
+    for (int k = b0; k < g.b1; ++k)
+      for (int i = 0; i < x->batches[k].nb; ++i) ++vptr[p0 + 1 + idx[x->batches[k].ao0 + i]];
+    vptr[p0] = (long long)e0;
+    for (int i = 0; i < v.nbf; ++i) vptr[p0 + 1 + i] += vptr[p0 + i];
+    vent.resize((size_t)vptr[p0 + v.nbf]);
+    std::vector<long long> at(vptr.begin() + p0, vptr.end() - 1);
+    for (int k = b0; k < g.b1; ++k)
+      for (int i = 0; i < x->batches[k].nb; ++i) vent[at[idx[x->batches[k].ao0 + i]]++] = int2{k, i};
+    g.ntile = (long long)tile.size() - g.tile0;
+    g.nvt = (long long)vt.size() - g.vt0;
+    max_grp = std::max(max_grp, g.ngrp);
+    max_vb = std::max(max_vb, g.nvb);
+    max_tile = std::max(max_tile, g.ntile);
+    x->groups.push_back(g);
+    b0 = g.b1;
   }
   // device copies
   std::vector<double> xf(400);
@@ -851,16 +1128,19 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
   std::vector<int> harm(v.harm, v.harm + v.nsh);
   int nprim_tot = 0;
   for (int s = 0; s < v.nsh; ++s) nprim_tot = std::max(nprim_tot, v.poff[s] + v.nprim[s]);
-  const size_t mp = (size_t)x->max_pts, mb = (size_t)x->max_nb;
   ok = upload(x->d_pts, sorted.data(), sorted.size(), st) && upload(x->d_xf, xf.data(), xf.size(), st) &&
        upload(x->d_shl, shl.data(), shl.size(), st) && upload(x->d_col, col.data(), col.size(), st) &&
        upload(x->d_idx, idx.data(), idx.size(), st) && upload(x->d_am, v.am, (size_t)v.nsh, st) &&
        upload(x->d_harm, harm.data(), harm.size(), st) && upload(x->d_atom, v.atom, (size_t)v.nsh, st) &&
        upload(x->d_nprim, v.nprim, (size_t)v.nsh, st) && upload(x->d_poff, v.poff, (size_t)v.nsh, st) &&
-       upload(x->d_ex, v.ex, (size_t)nprim_tot, st) && upload(x->d_cc, v.cc, (size_t)nprim_tot, st);
-  for (auto& l : x->lane)
-    ok = ok && l.phi.ensure(mp * mb) && l.dphi.ensure(3 * mp * mb) && l.X.ensure(2 * mp * mb) &&
-         l.Y.ensure(2 * mp * mb) && l.Db.ensure(mb * mb) && l.Vb.ensure((mp / KCHUNK + 1) * mb * mb);
+       upload(x->d_ex, v.ex, (size_t)nprim_tot, st) && upload(x->d_cc, v.cc, (size_t)nprim_tot, st) &&
+       upload(x->d_batch, db.data(), db.size(), st) && upload(x->d_tile, tile.data(), tile.size(), st) &&
+       upload(x->d_vt, vt.data(), vt.size(), st) && upload(x->d_vptr, vptr.data(), vptr.size(), st) &&
+       upload(x->d_vent, vent.data(), vent.size(), st);
+  // workspaces of the largest group, for two spins where a build needs them (vxc_run)
+  x->max_grp = max_grp;
+  x->max_vb = max_vb;
+  x->max_tile = max_tile;
   ok = ok && hipStreamSynchronize(st) == hipSuccess;
   if (!ok) return 3;
   x->grid_ready = true;
@@ -920,103 +1200,60 @@ int vxc_run(oqph_session* s, const double* d, int nfocks, double* fxc, double* e
   if (rc) return rc;
   const int nbf = v.nbf;
   const size_t ntri = (size_t)nbf * (nbf + 1) / 2, nn = (size_t)nbf * nbf;
-  if (!x->ready && hipEventCreateWithFlags(&x->ready, hipEventDisableTiming) != hipSuccess) {
-    x->ready = nullptr;
-    err("oqph_vxc: hipEventCreate failed");
-    return 2;
+  const size_t ns = (size_t)nfocks, npad = (size_t)x->max_tile * TILE;
+  if (!upload(x->d_pk, d, ntri * ns, st) || !x->d_D.ensure(nn * ns) || !x->d_V.ensure(nn * ns) || !x->d_acc.ensure(2) ||
+      !x->d_phi.ensure((size_t)x->max_grp) || !x->d_Y.ensure(ns * x->max_grp) || !x->d_Vb.ensure(ns * x->max_vb) ||
+      !x->d_rho.ensure(4 * ns * npad) || !x->d_coef.ensure(4 * ns * npad)) {
+    hipStreamSynchronize(st);  // the upload reads the caller's array
+    return 3;
   }
-  for (auto& l : x->lane) {
-    if (!l.st && hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking) != hipSuccess) {
-      l.st = nullptr;
-      err("oqph_vxc: hipStreamCreate failed");
-      return 2;
-    }
-    if (!l.done && hipEventCreateWithFlags(&l.done, hipEventDisableTiming) != hipSuccess) {
-      l.done = nullptr;
-      err("oqph_vxc: hipEventCreate failed");
-      return 2;
-    }
-    if (!l.blas && rocblas_create_handle(&l.blas) != rocblas_status_success) {
-      l.blas = nullptr;
-      err("oqph_vxc: rocblas_create_handle failed");
-      return 2;
-    }
-    rocblas_set_stream(l.blas, l.st);
-    if (!l.V.ensure(nn * nfocks)) return 3;
-  }
-  if (!upload(x->d_pk, d, ntri * nfocks, st) || !x->d_D.ensure(nn * nfocks) || !x->d_acc.ensure(2)) return 3;
+  const size_t lds = (size_t)4 * 16 * (TILE + 1) * sizeof(double) + (size_t)x->max_nb * sizeof(int);
   for (int sp = 0; sp < nfocks; ++sp)
     hipLaunchKernelGGL(k_unpack, dim3(nblk((long long)nn, 256)), dim3(256), 0, st, x->d_pk.p + sp * ntri, nbf,
                        x->d_D.p + sp * nn);
   hipMemsetAsync(x->d_acc.p, 0, 2 * sizeof(double), st);
-  hipEventRecord(x->ready, st);
-  for (auto& l : x->lane) {
-    hipStreamWaitEvent(l.st, x->ready, 0);
-    hipMemsetAsync(l.V.p, 0, nn * nfocks * sizeof(double), l.st);
+  hipMemsetAsync(x->d_V.p, 0, nn * ns * sizeof(double), st);
+  XArgs a{};
+  a.ao = {x->d_am.p, x->d_harm.p, x->d_atom.p, x->d_nprim.p, x->d_poff.p, x->d_ex.p, x->d_cc.p, x->d_xyz.p, x->d_xf.p};
+  a.pts = x->d_pts.p;
+  a.batch = x->d_batch.p;
+  a.shl = x->d_shl.p;
+  a.col = x->d_col.p;
+  a.idx = x->d_idx.p;
+  a.phi = x->d_phi.p;
+  a.Y = x->d_Y.p;
+  a.rho = x->d_rho.p;
+  a.coef = x->d_coef.p;
+  a.Vb = x->d_Vb.p;
+  auto kr = x->f.gga ? k_rho<true> : k_rho<false>;
+  auto ky = x->f.gga ? k_y<true> : k_y<false>;
+  if (lds > 64 * 1024) hipFuncSetAttribute((const void*)kr, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  for (size_t gi = 0; gi < x->groups.size(); ++gi) {
+    const Group& g = x->groups[gi];
+    a.tile = x->d_tile.p + g.tile0;
+    a.vt = x->d_vt.p + g.vt0;
+    a.npad = g.ntile * TILE;
+    a.ngrp = g.ngrp;
+    a.nvb = g.nvb;
+    const unsigned nt = (unsigned)g.ntile, sp = (unsigned)nfocks;
+    hipLaunchKernelGGL(k_ao, dim3(nt), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(kr, dim3(nt, sp), dim3(256), lds, st, a, x->d_D.p, nbf);
+    hipLaunchKernelGGL(k_xc_point, dim3(std::min(nblk(g.ntile, 4), 2048u)), dim3(256), 0, st, a, g.ntile, nfocks, x->f,
+                       x->d_acc.p);
+    hipLaunchKernelGGL(ky, dim3(nt, sp), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_vmat, dim3((unsigned)g.nvt, sp), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_vsum, dim3((unsigned)nbf, nblk(nbf, VCOLS), sp), dim3(512),
+                       std::min(nbf, VCOLS) * sizeof(double), st, a, x->d_vptr.p + gi * (nbf + 1), x->d_vent.p, nbf,
+                       x->d_V.p);
   }
-  // on an error, let the work already queued on the lanes finish before the
-  // buffers can be reused
-  auto drain = [&](int code) {
-    for (auto& l : x->lane) hipStreamSynchronize(l.st);
+  for (int sp = 0; sp < nfocks; ++sp)
+    hipLaunchKernelGGL(k_pack, dim3(nblk((long long)ntri, 256)), dim3(256), 0, st, x->d_V.p + sp * nn, nbf,
+                       x->d_pk.p + sp * ntri);
+  hipError_t le = hipGetLastError();
+  if (le != hipSuccess) {
+    err("oqph_vxc: launch failed: %s", hipGetErrorString(le));
     hipStreamSynchronize(st);
-    return code;
-  };
-  const double one = 1.0, zero = 0.0;
-  for (size_t ib = 0; ib < x->batches.size(); ++ib) {
-    const Batch& b = x->batches[ib];
-    Lane& L = x->lane[ib % XC_LANES];
-    hipStream_t ls = L.st;
-    const int np = b.npts, nb = b.nb;
-    AOArgs aa{x->d_pts.p + 4 * b.p0, np, b.nsh, nb, x->d_shl.p + b.sh0, x->d_col.p + b.sh0, x->d_am.p,
-              x->d_harm.p, x->d_atom.p, x->d_nprim.p, x->d_poff.p, x->d_ex.p, x->d_cc.p, x->d_xyz.p, x->d_xf.p,
-              L.phi.p, L.dphi.p, x->f.gga};
-    hipLaunchKernelGGL(k_ao, dim3(nblk((long long)np * b.nsh, 256)), dim3(256), 0, ls, aa);
-    const size_t plane = (size_t)np * nb;
-    for (int sp = 0; sp < nfocks; ++sp) {
-      hipLaunchKernelGGL(k_gather, dim3(nblk((long long)nb * nb, 256)), dim3(256), 0, ls, x->d_D.p + sp * nn, nbf,
-                         x->d_idx.p + b.ao0, nb, L.Db.p);
-      // X (np x nb, column-major) = phi (np x nb) D_b (nb x nb)
-      if (rocblas_dgemm(L.blas, rocblas_operation_none, rocblas_operation_none, np, nb, nb, &one, L.phi.p, np, L.Db.p,
-                        nb, &zero, L.X.p + sp * plane, np) != rocblas_status_success) {
-        err("oqph_vxc: rocblas_dgemm failed");
-        return drain(2);
-      }
-    }
-    PointArgs pa{x->d_pts.p + 4 * b.p0, np, nb, nfocks, x->f.gga, L.phi.p, L.dphi.p, L.X.p, L.Y.p, x->d_acc.p, x->f};
-    hipLaunchKernelGGL(k_xc_point, dim3(nblk(np, 64)), dim3(64 * XC_SLICES), 0, ls, pa);
-    // V_b = phi^T Y, V_b(m, n) = sum_p phi(p, m) Y(p, n), as partial sums over
-    // KCHUNK-point slices (one strided-batched GEMM plus the remainder): the
-    // nb x nb result alone gives too few tiles to fill the device
-    const int nfull = np / KCHUNK, rem = np % KCHUNK, nparts = nfull + (rem > 0 ? 1 : 0);
-    const long long nb2 = (long long)nb * nb;
-    for (int sp = 0; sp < nfocks; ++sp) {
-      const double* Ys = L.Y.p + sp * plane;
-      if (nfull > 0 &&
-          rocblas_dgemm_strided_batched(L.blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, KCHUNK,
-                                        &one, L.phi.p, np, KCHUNK, Ys, np, KCHUNK, &zero, L.Vb.p, nb, nb2,
-                                        nfull) != rocblas_status_success) {
-        err("oqph_vxc: rocblas_dgemm_strided_batched failed");
-        return drain(2);
-      }
-      if (rem > 0 && rocblas_dgemm(L.blas, rocblas_operation_transpose, rocblas_operation_none, nb, nb, rem, &one,
-                                   L.phi.p + (size_t)nfull * KCHUNK, np, Ys + (size_t)nfull * KCHUNK, np, &zero,
-                                   L.Vb.p + nfull * nb2, nb) != rocblas_status_success) {
-        err("oqph_vxc: rocblas_dgemm failed");
-        return drain(2);
-      }
-      hipLaunchKernelGGL(k_scatter, dim3(nblk(nb2, 256)), dim3(256), 0, ls, L.Vb.p, nb, nparts, x->d_idx.p + b.ao0,
-                         nbf, L.V.p + sp * nn);
-    }
-  }
-  for (auto& l : x->lane) {
-    hipEventRecord(l.done, l.st);
-    hipStreamWaitEvent(st, l.done, 0);
-  }
-  for (int sp = 0; sp < nfocks; ++sp) {
-    LaneSum lsum{};
-    lsum.n = XC_LANES;
-    for (int k = 0; k < XC_LANES; ++k) lsum.v[k] = x->lane[k].V.p + sp * nn;
-    hipLaunchKernelGGL(k_pack, dim3(nblk((long long)ntri, 256)), dim3(256), 0, st, lsum, nbf, x->d_pk.p + sp * ntri);
+    return 2;
   }
   double acc[2];
   if (hipMemcpyAsync(fxc, x->d_pk.p, ntri * nfocks * sizeof(double), hipMemcpyDeviceToHost, st) != hipSuccess ||
