@@ -65,6 +65,13 @@ __host__ __device__ constexpr long long flops_grad_prim() {
 // chunk of 64 kets is spread over 64 / kpb wavefronts, each ket on 64 / kpb
 // lanes that take every (64 / kpb)-th primitive quartet and sum at the end.
 // One water's gradient in cc-pVTZ 50.8 -> 25.3 ms, in 6-31G(d) 5.9 -> 2.7.
+// Per root the Gamma block meets the integrals through their adjoint, axis by axis:
+// W_x[ia, ib, ic, id] = sum over the components of Gamma I_y I_z, 6 operations per
+// component, then the three derivatives of every W entry; the product of each
+// component's nine derivative integrals took 27 and more live registers.  Bound by
+// FP64 issue at one or two wavefronts per SIMD.  (H2O)16/cc-pVTZ, one gradient:
+// (pp|ps) 18.7 -> 15.0 ms, (dp|ps) 16.7 -> 14.4, (ds|pp) 10.4 -> 8.7, (dp|ss) 10.0 ->
+// 5.2, (ds|ps) 13.9 -> 11.4, (ps|ss) 16.0 -> 15.1.
 template <int LA, int LB, int LC, int LD, typename R, bool MRSF = false, bool SPLIT = false>
 __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
   extern __shared__ double s_de[];
@@ -191,7 +198,10 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
         const R rz = er * ize, re = zr * ize;
         const R h2z = (R)pp.h, h2e = (R)qq.h, h2ze = (R)0.5 * ize;
         const R a2 = (R)(2.0 * pp.a), b2 = (R)(2.0 * pp.b), c2 = (R)(2.0 * qq.a);
-        constexpr int UR = (NG > 36) ? 1 : NR;
+        // unrolled roots cost a wavefront of occupancy from 18 components on ((ds|ps) 18.9 -> 11.4 ms rolled)
+        constexpr int UR = (NG > 12) ? 1 : NR;
+        constexpr int N2 = (LC + 1) * (LD + 1), N3 = (LB + 1) * N2, N4 = (LA + 1) * N3;
+        constexpr auto n4 = [](int ia, int ib, int ic, int id) { return ia * N3 + ib * N2 + ic * (LD + 1) + id; };
 #pragma unroll UR
         for (int r = 0; r < NR; ++r) {
           const R t2 = rx[r];
@@ -226,44 +236,39 @@ __global__ __launch_bounds__(256) void k_grad(GradParams prm, WaveWork ww) {
 #pragma unroll
             for (int k = 1; k <= LD; ++k) pcd[d][k] = pcd[d][k - 1] * cd;
           }
-          sfor<NA>([&](auto Ai) {
-            constexpr int a = OQPH_CI(Ai);
-            sfor<NB>([&](auto Bi) {
-              constexpr int b = OQPH_CI(Bi);
-              sfor<NC>([&](auto Ci) {
-                constexpr int c = OQPH_CI(Ci);
-                sfor<ND>([&](auto Di) {
-                  constexpr int dd = OQPH_CI(Di);
-                  const R g = Gam[((a * NB + b) * NC + c) * ND + dd];
-                  R I0[3], dA[3], dB[3], dC[3];
-                  sfor<3>([&](auto Xi) {
-                    constexpr int x = OQPH_CI(Xi);
-                    constexpr int ia = c_l(LA, a, x), ib = c_l(LB, b, x), ic = c_l(LC, c, x), id = c_l(LD, dd, x);
-                    const R* pa = pab[x];
-                    const R* pc = pcd[x];
-                    I0[x] = i2d<ia, ib, ic, id>(G[x], pa, pc);
-                    R v = a2 * i2d<ia + 1, ib, ic, id>(G[x], pa, pc);
-                    if constexpr (ia > 0) v -= (R)ia * i2d<ia - 1, ib, ic, id>(G[x], pa, pc);
-                    dA[x] = v;
-                    v = b2 * i2d<ia, ib + 1, ic, id>(G[x], pa, pc);
-                    if constexpr (ib > 0) v -= (R)ib * i2d<ia, ib - 1, ic, id>(G[x], pa, pc);
-                    dB[x] = v;
-                    v = c2 * i2d<ia, ib, ic + 1, id>(G[x], pa, pc);
-                    if constexpr (ic > 0) v -= (R)ic * i2d<ia, ib, ic - 1, id>(G[x], pa, pc);
-                    dC[x] = v;
-                  });
-                  fd[0][0] += g * dA[0] * I0[1] * I0[2];
-                  fd[0][1] += g * I0[0] * dA[1] * I0[2];
-                  fd[0][2] += g * I0[0] * I0[1] * dA[2];
-                  fd[1][0] += g * dB[0] * I0[1] * I0[2];
-                  fd[1][1] += g * I0[0] * dB[1] * I0[2];
-                  fd[1][2] += g * I0[0] * I0[1] * dB[2];
-                  fd[2][0] += g * dC[0] * I0[1] * I0[2];
-                  fd[2][1] += g * I0[0] * dC[1] * I0[2];
-                  fd[2][2] += g * I0[0] * I0[1] * dC[2];
-                });
-              });
+          // transferred integrals at the components' exponents, [axis][ia][ib][ic][id]
+          R I[3][N4];
+          sfor<3 * N4>([&](auto Ni) {
+            constexpr int x = OQPH_CI(Ni) / N4, n = OQPH_CI(Ni) % N4;
+            I[x][n] = i2d<n / N3, n / N2 % (LB + 1), n / (LD + 1) % (LC + 1), n % (LD + 1)>(G[x], pab[x], pcd[x]);
+          });
+          // per axis: the adjoint of its integrals, then its three derivatives
+          sfor<3>([&](auto Xi) {
+            constexpr int x = OQPH_CI(Xi), y = (x + 1) % 3, z = (x + 2) % 3;
+            R W[N4];
+#pragma unroll
+            for (int n = 0; n < N4; ++n) W[n] = (R)0;
+            sfor<NG>([&](auto Gi) {
+              constexpr int i = OQPH_CI(Gi), a = i / (NB * NC * ND), b = i / (NC * ND) % NB, c = i / ND % NC, d = i % ND;
+              constexpr int nx = n4(c_l(LA, a, x), c_l(LB, b, x), c_l(LC, c, x), c_l(LD, d, x));
+              constexpr int ny = n4(c_l(LA, a, y), c_l(LB, b, y), c_l(LC, c, y), c_l(LD, d, y));
+              constexpr int nz = n4(c_l(LA, a, z), c_l(LB, b, z), c_l(LC, c, z), c_l(LD, d, z));
+              W[nx] += (Gam[i] * I[y][ny]) * I[z][nz];
             });
+            R sa = 0, sb = 0, sc = 0, ma = 0, mb = 0, mc = 0;
+            sfor<N4>([&](auto Ni) {
+              constexpr int n = OQPH_CI(Ni), ia = n / N3, ib = n / N2 % (LB + 1), ic = n / (LD + 1) % (LC + 1),
+                            id = n % (LD + 1);
+              sa += W[n] * i2d<ia + 1, ib, ic, id>(G[x], pab[x], pcd[x]);
+              sb += W[n] * i2d<ia, ib + 1, ic, id>(G[x], pab[x], pcd[x]);
+              sc += W[n] * i2d<ia, ib, ic + 1, id>(G[x], pab[x], pcd[x]);
+              if constexpr (ia > 0) ma += (R)ia * W[n] * I[x][n - N3];
+              if constexpr (ib > 0) mb += (R)ib * W[n] * I[x][n - N2];
+              if constexpr (ic > 0) mc += (R)ic * W[n] * I[x][n - (LD + 1)];
+            });
+            fd[0][x] += a2 * sa - ma;
+            fd[1][x] += b2 * sb - mb;
+            fd[2][x] += c2 * sc - mc;
           });
         }
       }

@@ -1,8 +1,8 @@
 // gradc_device.h -- cooperative 2e-gradient kernel of the larger quartet classes.
 //
 // One wavefront (one block) takes the kets of one bra segment and evaluates
-// 64 / W quartets at a time, W = 16, 32 or 64 lanes on each, class known at
-// compile time (as k_jkc for the J/K build).  Per quartet:
+// 64 / W quartets at a time, W lanes on each: one per (a, b), at least three per
+// root, all 64 above 32; class known at compile time.  Per quartet:
 //   0. lane = (a, b): its row Gamma[cd] of the two-particle density in
 //      registers, and the fine screen;
 // per batch of primitive quartets
@@ -22,8 +22,8 @@
 // its time on index arithmetic and LDS round trips.  Here a lane holds one row
 // of Gamma and two small tables, with constant indices; LDS reads and
 // the serial chain of a quartet's primitives and roots remain.  A gradient of
-// (H2O)16/cc-pVTZ 435 -> 247 ms, C20H42/6-31G(d) 18.7 -> 13.9, one water in
-// cc-pVTZ 25.3 -> 9.0; the figures per class are at gradc_class() in session.hip.
+// (H2O)16/cc-pVTZ 435 -> 247 ms, C20H42/6-31G(d) 18.7 -> 13.9 (224 and 12.1 with
+// k_grad as it is now), one water in cc-pVTZ 25.3 -> 9.0; the figures per class are at gradc_class() in session.hip.
 #pragma once
 #include "eri_device.h"
 #include "grad_params.h"
@@ -37,7 +37,11 @@ struct GRC {
   static constexpr int NR = (LA + LB + LC + LD + 1) / 2 + 1;
   static constexpr int LAB = LA + LB + 1, LCD = LC + LD + 1, GA = (LAB + 1) * (LCD + 1);
   // lanes per quartet, quartets per wavefront
-  static constexpr int W = NAB <= 16 ? 16 : (NAB <= 32 ? 32 : 64);
+  // three quartets of up to 21 lanes where 16 do not suffice: (dp|ds) 16.6 -> 13.7 ms,
+  // (dp|pp) 13.9 -> 11.7, (dp|dp) 7.9 -> 6.6 ((H2O)16/cc-pVTZ); groups of 9, 10 and 30
+  // lanes gained nothing where more quartets of unequal length meet
+  static constexpr int WMIN = NAB > 3 * NR ? NAB : 3 * NR;
+  static constexpr int W = WMIN <= 16 ? 16 : WMIN <= 21 ? WMIN : WMIN <= 32 ? 32 : 64;
   static constexpr int NQ = 64 / W, AT = (NAB + W - 1) / W;
   // primitive quartets per batch of phase 1
   static constexpr int PB = W / (3 * NR) < 1 ? 1 : (W / (3 * NR) > 2 ? 2 : W / (3 * NR));
@@ -61,7 +65,9 @@ void k_gradc(GradParams prm, WaveWork ww) {
                 TR = J::TR, NT = J::NT, TT = J::TT, N2 = J::N2;
   __shared__ double s_slot[NQ][J::SLOT];
   extern __shared__ double s_de[];  // 3 natm
-  const int lane = (int)threadIdx.x, l = lane & (W - 1), q = lane / W;
+  // the lanes past the last quartet's take no part
+  const int lane = (int)threadIdx.x, q = min(lane / W, NQ - 1), l = lane - q * W;
+  const bool spare = l >= W;
   for (int i = lane; i < 3 * prm.natm; i += 64) s_de[i] = 0.0;
   // ---- the block's kets: [sub kpb, (sub + 1) kpb) of one 64-ket chunk of one segment
   const int kpb = ww.kpb > 0 ? ww.kpb : 64, per = 64 / kpb;
@@ -92,7 +98,7 @@ void k_gradc(GradParams prm, WaveWork ww) {
 #pragma unroll
   for (int u = 0; u < TT; ++u) {
     const int t = l + W * u, x = t / ((LA + 2) * TB), r = t - x * (LA + 2) * TB, ia = r / TB, ib = r - ia * TB;
-    const bool ok = t < NT && ia + ib <= LAB;
+    const bool ok = !spare && t < NT && ia + ib <= LAB;
     tx[u] = ok ? x : -1;
     trow[u] = ia;
     const double ab = x == 0 ? ABv[0] : x == 1 ? ABv[1] : ABv[2];
@@ -121,7 +127,7 @@ void k_gradc(GradParams prm, WaveWork ww) {
   }
   // phase 1: this lane's (primitive quartet of a batch, root, axis)
   const int pi = l / (3 * NR), r1 = (l - pi * 3 * NR) / 3, d1 = l - pi * 3 * NR - 3 * r1;
-  const bool vrr_lane = l < PB * 3 * NR;
+  const bool vrr_lane = !spare && l < PB * 3 * NR;
   double* G = s_slot[q];
   double* T = G + PB * NR * 3 * GA;
   const double* tabN = prm.rys + RYS_OFF[NR];
@@ -129,7 +135,7 @@ void k_gradc(GradParams prm, WaveWork ww) {
   double fA[3] = {0, 0, 0}, fB[3] = {0, 0, 0};  // the bra centres' sums over the block's kets
   unsigned n_comp = 0, n_skip = 0, n_prim = 0;
   for (int i0 = 0; i0 < nk; i0 += NQ) {
-    const bool on = i0 + q < nk;
+    const bool on = !spare && i0 + q < nk;
     const int jq = ww.ket[ket0 + (on ? i0 + q : 0)];
     const ShellPair Q = prm.pairs[jq];
     const int oc = prm.coff[Q.sa], od = prm.coff[Q.sb];
@@ -138,7 +144,7 @@ void k_gradc(GradParams prm, WaveWork ww) {
 #pragma unroll
     for (int t = 0; t < AT; ++t) {
       const int a = oa + ra[t], b = ob + rb[t];
-      const bool in = l + W * t < NAB;
+      const bool in = !spare && l + W * t < NAB;
       const double dab = 4.0 * prm.cs * Dc[a * n + b];
       double Dac[NC], Dad[ND], Dbc[NC], Dbd[ND];
 #pragma unroll
@@ -162,8 +168,9 @@ void k_gradc(GradParams prm, WaveWork ww) {
         gm = fmax(gm, fabs(Gam[t][i]));
       }
     }
+    // largest of the quartet's lanes: cyclic shifts within the group
 #pragma unroll
-    for (int o = 1; o < W; o <<= 1) gm = fmax(gm, __shfl_xor(gm, o));
+    for (int o = 1; o < W; o <<= 1) gm = fmax(gm, __shfl(gm, q * W + (l + o) % W));
     const bool skip = !on || gm * P.Q * Q.Q < 0.5 * prm.gcut;
     if (l == 0) {
       n_skip += (on && skip) ? 1 : 0;
@@ -177,8 +184,9 @@ void k_gradc(GradParams prm, WaveWork ww) {
     double f0[3] = {0, 0, 0}, f1[3] = {0, 0, 0}, f2[3] = {0, 0, 0};
     const int NP = P.nprim, NPQ = skip ? 0 : NP * Q.nprim;
     int Tmax = NPQ;
+    if (NQ > 1)
 #pragma unroll
-    for (int o = W; o < 64; o <<= 1) Tmax = max(Tmax, __shfl_xor(Tmax, o));
+      for (int o = 1; o < 64; o <<= 1) Tmax = max(Tmax, __shfl_xor(Tmax, o));
     Tmax = __builtin_amdgcn_readfirstlane(Tmax);
     int pb = pi, pk = 0, np = 0;
     while (pb >= NP && pk < Q.nprim) { pb -= NP; ++pk; }
@@ -360,10 +368,20 @@ void k_gradc(GradParams prm, WaveWork ww) {
       double u2 = skip ? 0.0 : deg * f2[x], ud = -(u0 + u1 + u2);
       fA[x] += u0;
       fB[x] += u1;
+      // sums into the group's first lane
+      if constexpr ((W & (W - 1)) == 0) {
 #pragma unroll
-      for (int o = 1; o < W; o <<= 1) {
-        u2 += __shfl_xor(u2, o);
-        ud += __shfl_xor(ud, o);
+        for (int o = 1; o < W; o <<= 1) {
+          u2 += __shfl_xor(u2, o);
+          ud += __shfl_xor(ud, o);
+        }
+      } else {
+#pragma unroll
+        for (int o = 16; o > 0; o >>= 1) {
+          const double v2 = __shfl_down(u2, o), vd = __shfl_down(ud, o);
+          u2 += l + o < W ? v2 : 0.0;
+          ud += l + o < W ? vd : 0.0;
+        }
       }
       if (l == 0 && !skip) {
         atomicAdd(&s_de[3 * at2 + x], u2);

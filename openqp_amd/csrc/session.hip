@@ -1018,12 +1018,12 @@ static long long class_weight(int la, int lb, int lc, int ld, bool runtime) {
 // which are those of more than 64 Cartesian components.  Measured against the
 // per-lane templates (k_grad) and, from 256 components, the run-time-class
 // kernel, summed kernel time of one gradient of (H2O)16/cc-pVTZ and of
-// C20H42/6-31G(d): (dp|pp) 50 -> 13 ms and 3.9 -> 1.6, (pp|pp) 26 -> 20 and
-// 3.4 -> 1.0, (dp|ds) 22 -> 17 and 1.4 -> 1.6, (dd|ps) 13 -> 10 and 1.2 -> 0.9,
-// (dd|ds) 9.7 -> 4.5 and 1.05 -> 0.41, (fs|pp) 11 -> 6.4, (fs|fs) 5.7 -> 3.3, all
-// classes of the run-time kernel 425 -> 110 and 3.6 -> 1.4.  Below the line the
+// C20H42/6-31G(d): (dp|pp) 50 -> 12 ms and 3.9 -> 1.5, (pp|pp) 26 -> 20 and
+// 3.4 -> 1.0, (dp|ds) 22 -> 14 and 1.4 -> 1.3, (dd|ps) 13 -> 10 and 1.2 -> 0.9,
+// (dd|ds) 9.7 -> 3.8 and 1.05 -> 0.33, (fs|pp) 11 -> 6.6, (fs|fs) 5.7 -> 3.3, all
+// classes of the run-time kernel 425 -> 100 and 3.6 -> 1.1.  Below the line the
 // lanes and LDS round trips cost more than they save: (dp|ps), 54 components,
-// 17 -> 34 and 0.9 -> 3.1; (ds|pp) 10 -> 20; (ds|ds) 4.4 -> 13; (fs|ds) 3.9 -> 7.8.
+// 14 against 34 and 0.8 against 3.1; (ds|pp) 8.7 against 20; (ds|ds) 3.8 against 13.
 // The FP32 classes of a mixed gradient and the MRSF gradient keep k_grad / k_gradh.
 static bool gradc_class(const oqph_session* s, int la, int lb, int lc, int ld, KernelRes* r) {
   if (!s->gradc_on || s->grad_all_hl || (s->grad_hl_ng == 0 && grad_template(la, lb, lc, ld))) return false;
