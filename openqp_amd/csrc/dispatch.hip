@@ -1,6 +1,7 @@
 // dispatch.hip -- class dispatch of the J/K and Schwarz kernels, the small
 // per-build kernels, and the host copies of the Rys tables.
 #define OQPH_WANT_RYS_DATA
+#include <algorithm>
 #include <vector>
 #include "eri_device.h"
 #include "grad_device.h"
@@ -343,27 +344,39 @@ bool grad_template(int la, int lb, int lc, int ld) {
 // shell-pair density maxima (shlden, source/integrals/int2.F90:999-1047)
 // shell-pair max |D| (shlden, int2.F90:999-1047); with D2 the max over both
 // densities (nfocks = 2)
+// out (a launch of one block only): the largest of them as well
 __global__ void k_shell_density(const double* D, const double* D2, const int* ao_off, const int* nao, int nsh,
-                                double* dsh) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+                                double* dsh, double* out) {
   const long long np = (long long)nsh * (nsh + 1) / 2;
-  if (t >= np) return;
-  int i = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((long long)i * (i + 1) / 2 > t) --i;
-  while ((long long)(i + 1) * (i + 2) / 2 <= t) ++i;
-  const int j = t - i * (i + 1) / 2;
-  double m = 0.0;
-  for (int a = 0; a < nao[i]; ++a) {
-    const int x = ao_off[i] + a;
-    const int jmax = (i == j) ? a + 1 : nao[j];
-    for (int b = 0; b < jmax; ++b) {
-      const long long xy = tri_idx_(x, ao_off[j] + b);
-      m = fmax(m, fabs(D[xy]));
-      if (D2) m = fmax(m, fabs(D2[xy]));
+  double mx = 0.0;
+  for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < np; t += (long long)gridDim.x * blockDim.x) {
+    int i = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+    while ((long long)i * (i + 1) / 2 > t) --i;
+    while ((long long)(i + 1) * (i + 2) / 2 <= t) ++i;
+    const int j = (int)(t - (long long)i * (i + 1) / 2);
+    double m = 0.0;
+    for (int a = 0; a < nao[i]; ++a) {
+      const int x = ao_off[i] + a;
+      const int jmax = (i == j) ? a + 1 : nao[j];
+      for (int b = 0; b < jmax; ++b) {
+        const long long xy = tri_idx_(x, ao_off[j] + b);
+        m = fmax(m, fabs(D[xy]));
+        if (D2) m = fmax(m, fabs(D2[xy]));
+      }
     }
+    dsh[i * nsh + j] = m;
+    dsh[j * nsh + i] = m;
+    mx = fmax(mx, m);
   }
-  dsh[i * nsh + j] = m;
-  dsh[j * nsh + i] = m;
+  if (!out) return;
+  __shared__ double s_m[16];
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_down(mx, o));
+  if (__lane_id() == 0) s_m[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (unsigned w = 1; w < blockDim.x / 64; ++w) mx = fmax(mx, s_m[w]);
+    *out = mx;
+  }
 }
 
 __global__ void k_max_reduce(const double* x, long long n, unsigned long long* out) {
@@ -374,12 +387,22 @@ __global__ void k_max_reduce(const double* x, long long n, unsigned long long* o
   if (__lane_id() == 0) atomicMax(out, (unsigned long long)__double_as_longlong(m));
 }
 
-void launch_shell_density(const double* D, const double* D2, const int* ao_off, const int* nao, int nsh, double* dsh,
-                          hipStream_t s) {
+// dsh, and the bits of its largest element in max[0].  Up to 8192 shell pairs (127
+// shells) one block does both; more take a launch each and the word cleared in
+// between (one water 13 + 15 us and two gaps less per build).
+hipError_t launch_shell_density(const double* D, const double* D2, const int* ao_off, const int* nao, int nsh,
+                                double* dsh, unsigned long long* max, hipStream_t s) {
   const long long np = (long long)nsh * (nsh + 1) / 2;
+  if (np <= 8192) {
+    hipLaunchKernelGGL(k_shell_density, dim3(1), dim3(1024), 0, s, D, D2, ao_off, nao, nsh, dsh, (double*)max);
+    return hipSuccess;
+  }
   const int bs = 256;
   hipLaunchKernelGGL(k_shell_density, dim3((unsigned)((np + bs - 1) / bs)), dim3(bs), 0, s, D, D2, ao_off, nao, nsh,
-                     dsh);
+                     dsh, (double*)nullptr);
+  const hipError_t e = hipMemsetAsync(max, 0, sizeof(*max), s);
+  hipLaunchKernelGGL(k_max_reduce, dim3(256), dim3(256), 0, s, dsh, (long long)nsh * nsh, max);
+  return e;
 }
 
 // p = c (a + b), m = c (a - b), elementwise over n doubles; p == a and m == b
@@ -417,10 +440,13 @@ __global__ void k_jscatter(const ShellPair* pairs, const int* joff, int npair, i
 }
 
 // The per-pair inputs of a J/K build in device-pair order (JKParams::Dk, dpm),
-// and the ket-side Coulomb buffer cleared; D null (response pass): dpm only
+// and the ket-side Coulomb buffer and the list's arrays cleared in the same launch;
+// D null (response pass): dpm only
 __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, int pure, const double* D,
-                          const double* dsh, int nsh, double* Dk, double* dpm, double* Jk) {
+                          const double* dsh, int nsh, double* Dk, double* dpm, double* Jk, ClearList z) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  for (int k = 0; k < 3; ++k)
+    for (long long t = i; t < z.n[k]; t += (long long)gridDim.x * blockDim.x) z.p[k][t] = 0.0;
   if (i >= npair) return;
   const ShellPair P = pairs[i];
   const int na = (pure && P.la >= 2) ? 2 * P.la + 1 : (P.la + 1) * (P.la + 2) / 2;
@@ -436,10 +462,12 @@ __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, in
 }
 
 void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
-                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s) {
-  if (npair <= 0) return;
-  hipLaunchKernelGGL(k_dgather, dim3((unsigned)((npair + 63) / 64)), dim3(64), 0, s, pairs, joff, npair, pure ? 1 : 0,
-                     D, dsh, nsh, Dk, dpm, Jk);
+                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s, const ClearList& z) {
+  const long long nz = std::max(z.n[0], std::max(z.n[1], z.n[2]));
+  const long long nb = std::max<long long>((npair + 63) / 64, std::min<long long>((nz + 63) / 64, 4096));
+  if (nb <= 0) return;
+  hipLaunchKernelGGL(k_dgather, dim3((unsigned)nb), dim3(64), 0, s, pairs, joff, npair, pure ? 1 : 0, D, dsh, nsh, Dk,
+                     dpm, Jk, z);
 }
 
 void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* Jk, double* F,
@@ -449,9 +477,6 @@ void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pu
                      pure ? 1 : 0, Jk, F);
 }
 
-void launch_max_reduce(const double* x, long long n, unsigned long long* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_max_reduce, dim3(256), dim3(256), 0, s, x, n, out);
-}
 
 
 // the Rys table followed by the Boys table (QTab offsets)

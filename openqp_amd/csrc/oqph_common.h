@@ -195,6 +195,12 @@ struct ColMap {
 // many L2 lines instead of serialising on one; the host sums the slots.
 #define OQPH_CTR_SLOTS 128
 
+// up to three arrays of doubles (or 64-bit counters) to clear
+struct ClearList {
+  double* p[3];
+  long long n[3];
+};
+
 // Arguments of one J/K build launch (shared by host and device code).
 struct JKParams {
   const ShellPair* pairs;

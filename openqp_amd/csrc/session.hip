@@ -44,14 +44,13 @@ int jkt_info(int la, int lb, int lc, int ld, bool pure, size_t* static_lds, size
 bool launch_schwarz(int la, int lb, bool pure, const ShellPair* pairs, const PrimJK* prims, const int* list, int n,
                     const double* tab, const double* xf, double qcut, double imu2, double* Q, hipStream_t s);
 bool kernel_resources(int kind, int la, int lb, int lc, int ld, bool pure, KernelRes* r);
-void launch_shell_density(const double* D, const double* D2, const int* ao_off, const int* nao, int nsh, double* dsh,
-                          hipStream_t s);
+hipError_t launch_shell_density(const double* D, const double* D2, const int* ao_off, const int* nao, int nsh,
+                                double* dsh, unsigned long long* max, hipStream_t s);
 void launch_sumdiff(const double* a, const double* b, double* p, double* m, double c, long long n, hipStream_t s);
 void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* Jk, double* F,
                      hipStream_t s);
 void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
-                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s);
-void launch_max_reduce(const double* x, long long n, unsigned long long* out, hipStream_t s);
+                    int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s, const ClearList& z);
 bool kernels_support(int lmax);
 bool jk_template(int la, int lb, int lc, int ld);
 bool grad_template(int la, int lb, int lc, int ld);
@@ -1991,17 +1990,15 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
       return 1;
     }
   }
-  launch_shell_density(scr_a ? scr_a : dD, scr_b, s->d_aooff.p, s->d_nao.p, s->nsh, dsh, stream);
-  HIPCHK(hipMemsetAsync(ctr0, 0, 8 * sizeof(unsigned long long), stream));
-  launch_max_reduce(dsh, (long long)nsh2, ctr0 + 4, stream);
+  HIPCHK(launch_shell_density(scr_a ? scr_a : dD, scr_b, s->d_aooff.p, s->d_nao.p, s->nsh, dsh, ctr0 + 4, stream));
   unsigned long long mbits = 0;
   HIPCHK(hipMemcpyAsync(&mbits, ctr0 + 4, sizeof(mbits), hipMemcpyDeviceToHost, stream));
   HIPCHK(hipStreamSynchronize(stream));
   double maxden;
   memcpy(&maxden, &mbits, sizeof(double));
-  if (zero_f) HIPCHK(hipMemsetAsync(dF, 0, ntri * sizeof(double), stream));
-  if (zero_f && dF2) HIPCHK(hipMemsetAsync(dF2, 0, ntri * sizeof(double), stream));
   if (maxden <= 0.0) {
+    if (zero_f) HIPCHK(hipMemsetAsync(dF, 0, ntri * sizeof(double), stream));
+    if (zero_f && dF2) HIPCHK(hipMemsetAsync(dF2, 0, ntri * sizeof(double), stream));
     if (st) memset(st, 0, sizeof(*st));
     return 0;
   }
@@ -2046,7 +2043,6 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
     ltasks = s->d_tasks.p;
   }
   for (auto& L : s->launches) bind_lists(s, L, lseg, lchoff, litems, ltasks);
-  HIPCHK(hipMemsetAsync(ctr, 0, nc * nl * sizeof(unsigned long long), stream));
   const bool profile = s->profile && !ss;
   if (profile && s->pev.size() < 2 * nl) {
     for (size_t i = s->pev.size(); i < 2 * nl; ++i) {
@@ -2064,8 +2060,10 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   p.rys = s->d_rys.p;
   p.rys32 = s->d_rys32.p;
   p.xform = s->d_xform.p;
+  const ClearList zero{{(double*)ctr, dF, dF2}, {(long long)(nc * nl), zero_f ? (long long)ntri : 0,
+                                                 zero_f && dF2 ? (long long)ntri : 0}};
   launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, dD, dsh, s->nsh, s->d_dk.p,
-                 s->d_dpm.p, Jk, stream);
+                 s->d_dpm.p, Jk, stream, zero);
   p.Jk = Jk;
   p.Dk = s->d_dk.p;
   p.dpm = s->d_dpm.p;
@@ -2214,7 +2212,7 @@ static int build_general(oqph_session* s, bool dense, int nd, const double* dD, 
     p.Dk = s->d_dk.p;
     p.dpm = s->d_dpm.p;
     launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, nullptr, s->d_dsh.p, s->nsh, nullptr,
-                   s->d_dpm.p, nullptr, stream);
+                   s->d_dpm.p, nullptr, stream, ClearList{});
     HIPCHK(hipMemsetAsync(p.T, 0, (size_t)(npair * n * ldd) * sizeof(double), stream));
   }
   const int nst = s->nstreams;
