@@ -461,6 +461,32 @@ __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, in
   dpm[i] = dsh[(long long)P.si * nsh + P.sj];
 }
 
+// the piecewise copies of the primitive-pair records (JKParams::kt64, kt32)
+__global__ void k_ktrans(const ShellPair* pairs, int npair, const PrimJK* prims, const PrimF32* prims32, double2* kt64,
+                         float2* kt32) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npair) return;
+  const int n = pairs[i].nprim, p0 = pairs[i].prim0;
+  long long at = pairs[i].kt;
+  for (int k = 0; k < n; ++k, at += 192) {
+    const PrimJK r = prims[p0 + k];
+    kt64[at] = double2{r.g, r.Kg};
+    kt64[at + 64] = double2{r.X[0], r.X[1]};
+    kt64[at + 128] = double2{r.X[2], r.h};
+    const PrimF32 f = prims32[p0 + k];
+    kt32[at] = float2{f.g, f.Kg};
+    kt32[at + 64] = float2{f.X[0], f.X[1]};
+    kt32[at + 128] = float2{f.X[2], f.h};
+  }
+}
+
+void launch_ktrans(const ShellPair* pairs, int npair, const PrimJK* prims, const PrimF32* prims32, double* kt64,
+                   float* kt32, hipStream_t s) {
+  if (npair <= 0) return;
+  hipLaunchKernelGGL(k_ktrans, dim3((unsigned)((npair + 63) / 64)), dim3(64), 0, s, pairs, npair, prims, prims32,
+                     (double2*)kt64, (float2*)kt32);
+}
+
 void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
                     int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s, const ClearList& z) {
   const long long nz = std::max(z.n[0], std::max(z.n[1], z.n[2]));

@@ -435,6 +435,15 @@ template <typename R>
 struct PrimV {
   R g, Kg, X[3], h;
 };
+// record k of a ket from the piecewise copies (JKParams::kt64, kt32)
+template <typename R>
+__device__ __forceinline__ PrimV<R> ket_prim(const R* __restrict__ kt, int at, int k) {
+  typedef R R2 __attribute__((ext_vector_type(2)));
+  const R2* t = (const R2*)kt + (at + 192ll * k);
+  const R2 a = t[0], b = t[64], c = t[128];
+  return {a.x, a.y, {b.x, b.y, c.x}, c.y};
+}
+
 template <typename R, typename PP>
 __device__ __forceinline__ PrimV<R> prim_v(const PP& p) {
   return {(R)p.g, (R)p.Kg, {(R)p.X[0], (R)p.X[1], (R)p.X[2]}, (R)p.h};

@@ -176,7 +176,7 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
                                          R (&acc)[Dims<LA, LB, LC, LD>::NE][Dims<LA, LB, LC, LD>::NF],
                                          int& nprim_used, const PrimV<double>* sbra = nullptr,
                                          const PrimV<float>* sbra32 = nullptr, int nbra64 = 0,
-                                         int nbra32 = 0, const Split& sp = split_none()) {
+                                         int nbra32 = 0, const Split& sp = split_none(), const R* kt = nullptr) {
   using Dm = Dims<LA, LB, LC, LD>;
   constexpr bool F32 = sizeof(R) == 4;
 #pragma unroll
@@ -203,16 +203,26 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
     // short, i.e. the larger classes and FP64, it costs more than it hides)
     constexpr bool PREF = F32 && Dm::NE * Dm::NF <= 9;
     const int nq = Q.nprim;
+    // Kets of two s shells carry the longest primitive lists, and the classes up
+    // to (pp|ss) do little per record: reading 64 scattered records per step was
+    // a third of (ps|ss) FP64 on (H2O)64/cc-pVDZ (102.7 -> 80.6 ms from the pieces;
+    // (pp|ss) 23.2 -> 20.4, (ds|ss) 17.1 -> 14.7).  The other classes lose registers
+    // to the address ((ds|ps) 18.1 -> 19.2, (pp|ps) 22.0 -> 22.7) and keep the records.
+    constexpr bool KT = LC + LD == 0 && Dm::NE * Dm::NF <= 9;
+    auto ketp = [&](int k) -> PrimV<R> {
+      if constexpr (KT) return ket_prim(kt, Q.kt, k);
+      else return ket(Q.prim0 + k);
+    };
     auto walk = [&](const int sb, const int sk, const int nb, const int nk, const int nit) {
       PrimV<R> qn{};
-      if (PREF && sk < nq) qn = ket(Q.prim0 + sk);
+      if (PREF && sk < nq) qn = ketp(sk);
       for (int iq = sk; iq < nq; iq += nk) {
         PrimV<R> qq;
         if constexpr (PREF) {
           qq = qn;
-          if (iq + nk < nq) qn = ket(Q.prim0 + iq + nk);
+          if (iq + nk < nq) qn = ketp(iq + nk);
         } else {
-          qq = ket(Q.prim0 + iq);
+          qq = ketp(iq);
         }
         if (fabs(qq.Kg) < qcut) continue;
         R AQ[3];
@@ -360,11 +370,11 @@ __device__ __forceinline__ void quartet_block(const ShellPair& P, const ShellPai
                                               R qcut, R imu2, R (&V)[Dims<LA, LB, LC, LD>::NBLK], int& nprim_used,
                                               const PrimV<double>* sbra = nullptr,
                                               const PrimV<float>* sbra32 = nullptr, int nbra64 = 0,
-                                              int nbra32 = 0, const Split& sp = split_none()) {
+                                              int nbra32 = 0, const Split& sp = split_none(), const R* kt = nullptr) {
   using Dm = Dims<LA, LB, LC, LD>;
   R acc[Dm::NE][Dm::NF];
   contract<LA, LB, LC, LD, R, UNIFORM_BRA>(P, Q, prims, prims32, tabN, tab32N, qcut, imu2, acc, nprim_used, sbra,
-                                           sbra32, nbra64, nbra32, sp);
+                                           sbra32, nbra64, nbra32, sp, kt);
   R AB[3], CD[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
@@ -1061,7 +1071,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
             quartet_block<LA, LB, LC, LD, PURE, float, true>(P, Q, prm.prims, prm.prims32, tabN, tab32N,
                                                              prm.xform, (float)(1.0e-4 * prm.cutoff),
                                                              (float)prm.inv_mu2, Vf, nprim, sbra, sbra32, nbra64,
-                                                             nbra32, sp);
+                                                             nbra32, sp, prm.kt32);
 #pragma unroll
             for (int i = 0; i < NOUT; ++i) V[i] = (double)Vf[i];
           }
@@ -1069,7 +1079,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
         if (!lowp)
           quartet_block<LA, LB, LC, LD, PURE, double, true>(P, Q, prm.prims, prm.prims32, tabN, tab32N,
                                                             prm.xform, 1.0e-4 * prm.cutoff, prm.inv_mu2, V, nprim,
-                                                            sbra, nullptr, nbra64, nbra32, sp);
+                                                            sbra, nullptr, nbra64, nbra32, sp, prm.kt64);
       }
       n_prim += (unsigned)nprim;
       if (sp.n > 1) {  // primitive quartets of the ket, over its lanes

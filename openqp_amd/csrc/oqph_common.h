@@ -28,6 +28,7 @@ struct ShellPair {
   int si, sj;                  // reference order: si >= sj (shell indices)
   int la, lb;                  // angular momenta of a, b (la >= lb)
   int ca, cb;                  // first AO of a, b among the AOs of its angular momentum (ColMap; J/K records)
+  int kt;                      // first piece of its primitive pairs in JKParams::kt64 / kt32
 };
 
 struct PrimPair {              // 64 bytes: one cache line per primitive pair
@@ -222,6 +223,12 @@ struct JKParams {
   // coalesced instead of through three dependent gathers.
   const double* Dk;
   const double* dpm;
+  // The primitive-pair records by pieces of two fields, 64 consecutive pairs of
+  // a list bucket side by side: piece j (0 .. 2) of pair i's record k at
+  // kt + (3 k + j) 64.  A wavefront's kets are consecutive pairs, so each piece
+  // is one contiguous read instead of 64 cache lines.
+  const double* kt64;
+  const float* kt32;
   const double* dsh;    // nsh*nsh shell-pair max |D|
   unsigned long long* counters;  // [0] computed quartets, [1] skipped by fine screen, [2] fp32 quartets
   int nsh;

@@ -51,6 +51,8 @@ void launch_jscatter(const ShellPair* pairs, const int* joff, int npair, bool pu
                      hipStream_t s);
 void launch_dgather(const ShellPair* pairs, const int* joff, int npair, bool pure, const double* D, const double* dsh,
                     int nsh, double* Dk, double* dpm, double* Jk, hipStream_t s, const ClearList& z);
+void launch_ktrans(const ShellPair* pairs, int npair, const PrimJK* prims, const PrimF32* prims32, double* kt64,
+                   float* kt32, hipStream_t s);
 bool kernels_support(int lmax);
 bool jk_template(int la, int lb, int lc, int ld);
 bool grad_template(int la, int lb, int lc, int ld);
@@ -207,6 +209,8 @@ struct oqph_session {
   std::vector<int> h_joff, jbase;
   DBuf<int> d_joff;
   DBuf<double> d_jk;
+  DBuf<double> d_kt64;                       // JKParams::kt64, kt32
+  DBuf<float> d_kt32;
   DBuf<double> d_dk, d_dpm;                  // JKParams::Dk, dpm (allocated with the geometry)
   DBuf<int> d_kbs;                           // per class: bucket starts (NBKT+1)
   std::vector<std::vector<int>> kbs;
@@ -925,6 +929,27 @@ static int prepare_geometry(oqph_session* s) {
         dpr32.push_back(f32_record(dpr.back()));
       }
     }
+    // groups of 64 consecutive pairs of a bucket, each with the records of its longest
+    long long pieces = 0;
+    for (int c = 0; c < 10; ++c)
+      for (int b = 0; b < NBKT; ++b) {
+        const size_t k1 = s->cls_off[c] + s->kbs[c][b + 1];
+        for (size_t g = s->cls_off[c] + s->kbs[c][b]; g < k1; g += 64) {
+          int n = 0;
+          for (size_t i = g; i < std::min(g + 64, k1); ++i) {
+            n = std::max(n, dp[i].nprim);
+            dp[i].kt = (int)(pieces + (long long)(i - g));
+          }
+          pieces += 192ll * n;
+        }
+      }
+    if (pieces > 0x7fffffffll) {
+      set_err("%lld primitive-pair pieces exceed the 32-bit index", pieces);
+      return 3;
+    }
+    if ((rc = s->d_kt64.ensure(std::max<size_t>(2 * (size_t)pieces, 2))) ||
+        (rc = s->d_kt32.ensure(std::max<size_t>(2 * (size_t)pieces, 2))))
+      return rc;
     s->h_dpairs = dp;
     s->h_joff.assign(dp.size() + 1, 0);
     for (size_t i = 0; i < dp.size(); ++i)
@@ -947,6 +972,7 @@ static int prepare_geometry(oqph_session* s) {
                         (rc = upload_sync(s->d_prims32.p, dpr32.data(), dpr32.size() * sizeof(PrimF32), s->stream)) ||
                         (rc = upload_sync(s->d_cls.p, ident.data(), ident.size() * sizeof(int), s->stream))))
       return rc;
+    launch_ktrans(s->d_pairs.p, (int)dp.size(), s->d_prims.p, s->d_prims32.p, s->d_kt64.p, s->d_kt32.p, s->stream);
   }
   build_families(s);
   if ((rc = prepare_chunks(s, prims))) return rc;
@@ -2067,6 +2093,8 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   p.Jk = Jk;
   p.Dk = s->d_dk.p;
   p.dpm = s->d_dpm.p;
+  p.kt64 = s->d_kt64.p;
+  p.kt32 = s->d_kt32.p;
   p.D = dD;
   p.F = dF;
   p.D2 = dF2 ? dD2 : nullptr;
@@ -2349,7 +2377,7 @@ int oqph_session_destroy(oqph_session* s) {
   s->d_xform.release(); s->d_rys32.release(); s->d_kbs.release(); s->d_seg.release(); s->d_choff.release();
   s->d_gpairs.release(); s->d_gprims.release(); s->d_gcls.release(); s->d_coff.release(); s->d_satom.release();
   s->d_am.release(); s->d_pure.release(); s->d_gseg.release(); s->d_gchoff.release(); s->d_Dc.release(); s->d_de.release();
-  s->d_aooff.release(); s->d_nao.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
+  s->d_kt64.release(); s->d_kt32.release(); s->d_aooff.release(); s->d_nao.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
   s->d_tmp.release(); s->d_off.release(); s->d_ctr.release();
   s->d_gD.release(); s->d_gF.release(); s->d_gR.release(); s->d_gT.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
   for (auto e : s->pev) hipEventDestroy(e);
