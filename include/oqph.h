@@ -218,8 +218,8 @@ int oqph_fock_jk_noalloc(oqph_session *s, const double *d_dev, double *f_dev, do
  * launch); oqph_last_profile copies up to maxn entries of the last build:
  * class code la*1000+lb*100+lc*10+ld (plus 10000 when the launch used the
  * bra-row kernel k_jkb rather than k_jk, 20000 for the run-time-class kernel
- * k_jkh of the classes with an f shell, 30000 for the grouped bra-row kernel
- * k_jkg, 60000 for its tiled form; a multi-class launch of k_jkh reports
+ * k_jkh, 30000 for the grouped bra-row kernel k_jkg, 60000 for its tiled form,
+ * 80000 for the cooperative kernel k_jkc; a multi-class launch of k_jkh reports
  * 40000 + its number of classes), device ms, model FLOPs, computed
  * quartets, primitive quartets.  Returns the number of launches.
  * No counterpart in the seam: measurement hooks for benchmarks. */

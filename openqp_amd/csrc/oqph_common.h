@@ -71,8 +71,9 @@ struct WaveWork {
   const int* ket;
   int nseg;
   long long nwaves;
-  // run-time-class kernels: kets of a 64-ket chunk per block (64, 32, 16 or
-  // 8; 0 means 64): a launch takes nwaves * 64 / kpb blocks
+  // run-time-class and cooperative kernels, split gradient templates: kets of a
+  // 64-ket chunk per block or wavefront (a power of two; 0 means 64): a launch
+  // takes nwaves * 64 / kpb of them
   int kpb;
   // J/K class kernels: the ket class's block of the ket-side Coulomb buffer
   // (JKParams::Jk) starts at jbase; ket pair id iq owns the OC*OD entries

@@ -207,7 +207,7 @@ class FockBuilder:
         cls = la*1000 + lb*100 + lc*10 + ld; kernel is "k_jkb" (bra-row kernel), "k_jkg"
         (grouped bra-row kernel), "k_jkt" (its tiled form: bras sharing their first
         shell), "k_jkc" (cooperative kernel), "k_jk" (wavefront tasks) or "k_jkh" (run-time class,
-        the classes with an f shell); a launch of several run-time classes has
+        the few classes with neither); a launch of several run-time classes has
         kernel "k_jkh_multi" and cls 40000 + its number of classes."""
         n = 64
         cls = np.zeros(n, np.int32); ms = np.zeros(n); fl = np.zeros(n)
