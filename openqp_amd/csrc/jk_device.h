@@ -209,7 +209,9 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
     // (pp|ss) 23.2 -> 20.4, (ds|ss) 17.1 -> 14.7).  The other classes lose registers
     // to the address ((ds|ps) 18.1 -> 19.2, (pp|ps) 22.0 -> 22.7) and keep the records.
     constexpr bool KT = LC + LD == 0 && Dm::NE * Dm::NF <= 9;
-    auto ketp = [&](int k) -> PrimV<R> {
+    // (the records come in decreasing |K|: FP32 sums run from the smallest up)
+    auto ketp = [&](int i) -> PrimV<R> {
+      const int k = F32 ? nq - 1 - i : i;
       if constexpr (KT) return ket_prim(kt, Q.kt, k);
       else return ket(Q.prim0 + k);
     };

@@ -168,14 +168,14 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
   constexpr bool PREF = F32 && NE * NF <= 9;
   const int nq = Q.nprim;
   PrimV<R> qn{};
-  if (PREF && sp.sk < nq) qn = ket(Q.prim0 + sp.sk);
+  if (PREF && sp.sk < nq) qn = ket(Q.prim0 + (F32 ? nq - 1 - (sp.sk) : sp.sk));
   for (int iq = sp.sk; iq < nq; iq += nk) {
     PrimV<R> qq;
     if constexpr (PREF) {
       qq = qn;
-      if (iq + nk < nq) qn = ket(Q.prim0 + iq + nk);
+      if (iq + nk < nq) qn = ket(Q.prim0 + (F32 ? nq - 1 - (iq + nk) : iq + nk));
     } else {
-      qq = ket(Q.prim0 + iq);
+      qq = ket(Q.prim0 + (F32 ? nq - 1 - (iq) : iq));
     }
     const R kq = qq.Kg;
     if (fabs(kq) < qcut) continue;
