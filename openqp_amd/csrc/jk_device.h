@@ -233,11 +233,26 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
         // (eta <= zeta + eta), no later one passes the primitive screen
         const R stop = qcut2 * qq.g;
         auto run = [&](auto bra) {
-          for (int ip = 0; ip < nit; ip += nb) {
-            const PrimV<R> pp = bra(ip + sb);
-            const R fq = pp.Kg * qq.Kg;
-            if (fq * fq < stop) break;
+          auto add = [&](const PrimV<R>& pp) {
             nprim_used += rys_accumulate<LA, LB, LC, LD, R>(pp, qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
+          };
+          if constexpr (F32) {
+            // upwards: a sum that starts with its largest terms drops most of the
+            // small ones, always with their sign ((H2O)32/cc-pVDZ at an FP32 cutoff
+            // of 1e-3: energy 3.4e-8 Eh too low)
+            for (int ip = nit - nb; ip >= 0; ip -= nb) {
+              const PrimV<R> pp = bra(ip + sb);
+              const R fq = pp.Kg * qq.Kg;
+              if (fq * fq < stop) continue;
+              add(pp);
+            }
+          } else {
+            for (int ip = 0; ip < nit; ip += nb) {
+              const PrimV<R> pp = bra(ip + sb);
+              const R fq = pp.Kg * qq.Kg;
+              if (fq * fq < stop) break;
+              add(pp);
+            }
           }
         };
         // (the classes with an FP32 copy of the bra records always have it in
@@ -257,13 +272,14 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
     if constexpr (F32) return prim_v<float>(UNIFORM_BRA ? load_uniform(prims32, i) : prims32[i]);
     else return prim_v<double>(UNIFORM_BRA ? load_uniform(prims, i) : prims[i]);
   };
+  // (in decreasing |K|; FP32 sums run from the smallest up)
   for (int iq = 0; iq < Q.nprim; ++iq) {
-    const PrimV<R> qq = ket(Q.prim0 + iq);
+    const PrimV<R> qq = ket(Q.prim0 + (F32 ? Q.nprim - 1 - iq : iq));
     if (fabs(qq.Kg) < qcut) continue;
     R AQ[3];
     ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
     for (int ip = 0; ip < npp; ++ip) {
-      const PrimV<R> pp = bra(pp0 + ip);
+      const PrimV<R> pp = bra(pp0 + (F32 ? npp - 1 - ip : ip));
       if (fabs(pp.Kg) < qcut) continue;
       nprim_used += rys_accumulate<LA, LB, LC, LD, R>(pp, qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
     }

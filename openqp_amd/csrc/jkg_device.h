@@ -84,14 +84,15 @@ __device__ __forceinline__ void contract_tile(const ShellPair& Q, const double (
   constexpr bool PREF = F32 && NE * NF <= 9;
   const int nq = Q.nprim;
   PrimV<R> qn{};
-  if (PREF && nq > 0) qn = ket(Q.prim0);
+  // (records in decreasing |K|; FP32 sums run from the smallest up)
+  if (PREF && nq > 0) qn = ket(Q.prim0 + nq - 1);
   for (int iq = 0; iq < nq; ++iq) {
     PrimV<R> qq;
     if constexpr (PREF) {
       qq = qn;
-      if (iq + 1 < nq) qn = ket(Q.prim0 + iq + 1);
+      if (iq + 1 < nq) qn = ket(Q.prim0 + nq - 2 - iq);
     } else {
-      qq = ket(Q.prim0 + iq);
+      qq = ket(Q.prim0 + (F32 ? nq - 1 - iq : iq));
     }
     if (fabs(qq.Kg) < qcut) continue;
     R AQ[3];
@@ -100,9 +101,9 @@ __device__ __forceinline__ void contract_tile(const ShellPair& Q, const double (
     for (int m = 0; m < NM; ++m) {
       if (m >= nmem) break;  // uniform
       if (!((live >> m) & 1u)) continue;
-      const int p1 = moff[m + 1];
-      for (int ip = moff[m]; ip < p1; ++ip) {
-        const PrimV<R> pp = bp[ip];
+      const int p0 = moff[m], p1 = moff[m + 1];
+      for (int ip = p0; ip < p1; ++ip) {
+        const PrimV<R> pp = bp[F32 ? p0 + p1 - 1 - ip : ip];
         if (fabs(pp.Kg) < qcut) continue;
         np[m] += rys_accumulate<LA, LB, LC, LD, R>(pp, qq, AQ, qcut2, imu2, tabN, tab32N, acc[m]) ? 1 : 0;
       }
@@ -181,8 +182,12 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
     if (fabs(kq) < qcut) continue;
     R AQ[3];
     ket_offset<LA, LB, LC, LD, R>(AC, qq, AQ);
-    for (int ip = sp.sb; ip < nit + sp.sb; ip += nb) {
-      const R* r = rec + ip * stride;
+    // records in decreasing prefactor: FP64 ends at the first that cannot pass, FP32
+    // sums run upwards (as contract() in jk_device.h)
+    const R stop = qcut2 * qq.g;
+    for (int i = 0; i < nit; i += nb) {
+      const int ip = F32 ? nit - nb - i : i;
+      const R* r = rec + (ip + sp.sb) * stride;
       PrimV<R> pp;
       pp.g = r[0];
       pp.X[0] = r[1];
@@ -194,7 +199,7 @@ __device__ __forceinline__ int contract_group(const ShellPair& Q, const double (
       const R ze = zeta + eta + zeta * eta * imu2;
       const R fq = pp.Kg * kq;  // the largest member prefactor: no member passes below it
       const R fq2 = fq * fq;
-      if (fq2 < qcut2 * eta) break;  // records in decreasing prefactor: none of the rest passes
+      if (!F32 && fq2 < stop) break;  // none of the rest passes
       if (fq2 < qcut2 * ze) continue;
       const R sq = F32 ? (R)__builtin_amdgcn_rsqf((float)ze) : (R)rsq64((double)ze);
       const R ize = sq * sq;
