@@ -233,26 +233,17 @@ __device__ __forceinline__ void contract(const ShellPair& P, const ShellPair& Q,
         // (eta <= zeta + eta), no later one passes the primitive screen
         const R stop = qcut2 * qq.g;
         auto run = [&](auto bra) {
-          auto add = [&](const PrimV<R>& pp) {
+          // FP32 upwards: a sum that starts with its largest terms drops most of the
+          // small ones, always with their sign ((H2O)32/cc-pVDZ at an FP32 cutoff of
+          // 1e-3: energy 3.4e-8 Eh too low)
+          for (int i = 0; i < nit; i += nb) {
+            const PrimV<R> pp = bra((F32 ? nit - nb - i : i) + sb);
+            const R fq = pp.Kg * qq.Kg;
+            if (fq * fq < stop) {
+              if constexpr (F32) continue;
+              break;
+            }
             nprim_used += rys_accumulate<LA, LB, LC, LD, R>(pp, qq, AQ, qcut2, imu2, tabN, tab32N, acc) ? 1 : 0;
-          };
-          if constexpr (F32) {
-            // upwards: a sum that starts with its largest terms drops most of the
-            // small ones, always with their sign ((H2O)32/cc-pVDZ at an FP32 cutoff
-            // of 1e-3: energy 3.4e-8 Eh too low)
-            for (int ip = nit - nb; ip >= 0; ip -= nb) {
-              const PrimV<R> pp = bra(ip + sb);
-              const R fq = pp.Kg * qq.Kg;
-              if (fq * fq < stop) continue;
-              add(pp);
-            }
-          } else {
-            for (int ip = 0; ip < nit; ip += nb) {
-              const PrimV<R> pp = bra(ip + sb);
-              const R fq = pp.Kg * qq.Kg;
-              if (fq * fq < stop) break;
-              add(pp);
-            }
           }
         };
         // (the classes with an FP32 copy of the bra records always have it in
@@ -434,6 +425,22 @@ __device__ __forceinline__ void count_wave(unsigned long long* ctr, bool pred) {
   const unsigned long long act = __ballot(1);
   if (m != 0ull && __lane_id() == (unsigned)(__ffsll((long long)act) - 1))
     atomicAdd(ctr, (unsigned long long)__popcll(m));
+}
+
+// Bound of the quartet of bra pair ip and ket pair iq when the screens keep it
+// (int2.F90:763-800), else -1.
+__device__ __forceinline__ double quartet_bound(const JKParams& prm, int ip, int iq) {
+  const ShellPair& P = prm.pairs[ip];
+  const ShellPair& Q = prm.pairs[iq];
+  const bool p_first = (P.si > Q.si) || (P.si == Q.si && P.sj >= Q.sj);
+  if (prm.own && !prm.own[p_first ? ip : iq]) return -1.0;
+  const int n = prm.nsh;
+  const double* ds = prm.dsh;
+  double dm = 4.0 * fmax(prm.dpm[ip], prm.dpm[iq]);
+  dm = fmax(dm, fmax(ds[P.sj * n + Q.sj], ds[P.sj * n + Q.si]));
+  dm = fmax(dm, fmax(ds[P.si * n + Q.sj], ds[P.si * n + Q.si]));
+  const double bound = P.Q * Q.Q * dm;
+  return (p_first ? P.Q : Q.Q) * prm.maxden < prm.cutoff || bound < prm.cutoff ? -1.0 : bound;
 }
 
 // One integral (xy|zw) of the dense response pass into its places of prm.T
@@ -911,9 +918,9 @@ struct JKB {
   static constexpr int NEF = Dims<LA, LB, LC, LD>::NE * Dims<LA, LB, LC, LD>::NF;
   static constexpr int threads = NEF <= 4 ? OQPH_JKB_SMALL_THREADS : (NEF <= 9 ? 1024 : 512);
   // waves per SIMD the register allocation aims at: (ss|ss) 5 (96 VGPRs; 6 and
-  // 8 spill: 14.9 -> 18.5, 23.7 ms FP64 on (H2O)64/cc-pVDZ), the others
-  // unhinted ((ps|ss) 122 VGPRs, 4 waves; 5 and 6 spill: 103 -> 136, 182 ms)
-  static constexpr int min_waves = NEF == 1 ? 5 : 1;
+  // 8 spill: 14.9 -> 18.5, 23.7 ms FP64 on (H2O)64/cc-pVDZ), (ps|ss) 4 (128 VGPRs;
+  // 129 unhinted, 5 and 6 spill: 103 -> 136, 182 ms), the others unhinted
+  static constexpr int min_waves = NEF == 1 ? 5 : NEF <= 4 ? 4 : 1;
 };
 
 template <int LA, int LB, int LC, int LD, bool PURE, bool TWO>
@@ -1081,7 +1088,18 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       for (int i = 0; i < NOUT; ++i) V[i] = 0.0;
       int nprim = 0;
       bool lowp = false;
-      if constexpr (T32) lowp = prm.mixed && __ballot(!skip && bound >= prm.fp32_cut) == 0ull;
+      if constexpr (T32)
+        if (prm.mixed) {
+          bool high = !skip && bound >= prm.fp32_cut;
+          // 64 consecutive kets take FP32 together, also where a wavefront holds
+          // only some of them: spreading kets over lanes must not move quartets
+          // from FP64 to FP32 ((H2O)4/6-31G: a fifth more)
+          if (sp.n > 1) {
+            const int kc = (k0 & ~63) + lane;
+            high = kc < n && quartet_bound(prm, ip, bw.kofs + kbase + kc) >= prm.fp32_cut;
+          }
+          lowp = __ballot(high) == 0ull;
+        }
       if (!skip) {
         if constexpr (T32) {
           if (lowp) {

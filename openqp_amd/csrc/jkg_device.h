@@ -442,7 +442,18 @@ void k_jkg(JKParams prm, BraWork bw, ColMap cm, ChunkView cv) {
       }
       n_comp += head ? __popc(live) : 0;
       bool lowp = false;
-      if constexpr (T32) lowp = prm.mixed && __ballot(live != 0u && bmax >= prm.fp32_cut) == 0ull;
+      if constexpr (T32)
+        if (prm.mixed) {
+          bool high = live != 0u && bmax >= prm.fp32_cut;
+          if (!TILE && sp.n > 1) {  // by 64 consecutive kets, as in k_jkb
+            const int kc = (k0 & ~63) + lane, ic = bw.kofs + kbase + kc;
+            high = false;
+#pragma unroll 1
+            for (int m = 0; m < nmem; ++m)
+              if (kc < n && (!SAME || ic <= mi[m][0])) high |= quartet_bound(prm, mi[m][0], ic) >= prm.fp32_cut;
+          }
+          lowp = __ballot(high) == 0ull;
+        }
       // each member's final AO block; the (e0|f0) accumulators live only
       // inside the precision branch that fills them
       double Vall[NM][NBLK];
