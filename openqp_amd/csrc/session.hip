@@ -363,8 +363,9 @@ static unsigned long long g_serial = 0;  // last session serial handed out (unde
 
 // ------------------------------------------------ no-allocation scratch
 // Device memory of oqph_fock_jk_noalloc: the shell-pair density maxima, the
-// statistics counters and the work lists of one build, in a static array
-// that every GPU the library runs on holds until the process ends.  Host code
+// statistics counters, the work lists, the ket-side Coulomb buffer and the
+// gathered density of one build, in a static array that every GPU the library
+// runs on holds until the process ends.  Host code
 // never uses the array's name as an address: each device's copy is looked up
 // once with hipGetSymbolAddress (oqph_session_create, device current) and
 // that pointer is what kernels, memsets and copies receive.
@@ -1998,7 +1999,7 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   const size_t ntri = (size_t)s->nbf * (s->nbf + 1) / 2;
   const size_t nsh2 = (size_t)s->nsh * s->nsh;
   // scratch layout: counters 0..7 (density maximum), dsh, per-launch
-  // counters, work lists; 256-byte aligned slices
+  // counters, work lists, Jk, Dk, dpm; 256-byte aligned slices
   size_t off = 0;
   auto carve = [&](size_t bytes) -> unsigned char* {
     unsigned char* q = ss->base + off;
@@ -2037,7 +2038,7 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   int* litems;
   HLTask* ltasks;
   const size_t njk = std::max<size_t>(s->h_joff.empty() ? 0 : (size_t)s->h_joff.back(), 1);
-  double* Jk = nullptr;
+  double *Jk = nullptr, *Dk = s->d_dk.p, *dpm = s->d_dpm.p;
   if (ss) {
     const ListSizes n = list_sizes(s);
     ctr = (unsigned long long*)carve(nc * std::max<size_t>(nl, 1) * sizeof(unsigned long long));
@@ -2046,10 +2047,12 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
     litems = (int*)carve(n.items * sizeof(int));
     ltasks = (HLTask*)carve(n.tasks * sizeof(HLTask));
     Jk = (double*)carve(njk * sizeof(double));
+    Dk = (double*)carve(njk * sizeof(double));
+    dpm = (double*)carve(std::max<size_t>(s->h_dpairs.size(), 1) * sizeof(double));
     if (off > ss->bytes) {
       set_err("no-allocation build: this basis and density need %zu bytes of scratch (shell-pair maxima, "
-              "counters, work lists and the ket-side Coulomb buffer); the static scratch holds %zu", off,
-              ss->bytes);
+              "counters, work lists, the ket-side Coulomb buffer and the gathered density); the static scratch "
+              "holds %zu", off, ss->bytes);
       return 1;
     }
     if (*ss->serial != s->serial || *ss->gen != s->list_gen) {
@@ -2088,11 +2091,11 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
   p.xform = s->d_xform.p;
   const ClearList zero{{(double*)ctr, dF, dF2}, {(long long)(nc * nl), zero_f ? (long long)ntri : 0,
                                                  zero_f && dF2 ? (long long)ntri : 0}};
-  launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, dD, dsh, s->nsh, s->d_dk.p,
-                 s->d_dpm.p, Jk, stream, zero);
+  launch_dgather(s->d_pairs.p, s->d_joff.p, (int)(s->h_joff.size() - 1), s->pure, dD, dsh, s->nsh, Dk, dpm, Jk, stream,
+                 zero);
   p.Jk = Jk;
-  p.Dk = s->d_dk.p;
-  p.dpm = s->d_dpm.p;
+  p.Dk = Dk;
+  p.dpm = dpm;
   p.kt64 = s->d_kt64.p;
   p.kt32 = s->d_kt32.p;
   p.D = dD;
