@@ -461,7 +461,7 @@ __global__ void k_dgather(const ShellPair* pairs, const int* joff, int npair, in
   dpm[i] = dsh[(long long)P.si * nsh + P.sj];
 }
 
-// the piecewise copies of the primitive-pair records (JKParams::kt64, kt32)
+// the piecewise copies of the primitive-pair records of npair pairs (JKParams::kt64, kt32)
 __global__ void k_ktrans(const ShellPair* pairs, int npair, const PrimJK* prims, const PrimF32* prims32, double2* kt64,
                          float2* kt32) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

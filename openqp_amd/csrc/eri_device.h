@@ -435,9 +435,9 @@ template <typename R>
 struct PrimV {
   R g, Kg, X[3], h;
 };
-// record k of a ket from the piecewise copies (JKParams::kt64, kt32)
+// record k of a ket of two s shells from the piecewise copies (JKParams::kt64, kt32)
 template <typename R>
-__device__ __forceinline__ PrimV<R> ket_prim(const R* __restrict__ kt, int at, int k) {
+__device__ __forceinline__ PrimV<R> ket_prim(const R* __restrict__ kt, unsigned at, int k) {
   typedef R R2 __attribute__((ext_vector_type(2)));
   const R2* t = (const R2*)kt + (at + 192ll * k);
   const R2 a = t[0], b = t[64], c = t[128];

@@ -28,7 +28,7 @@ struct ShellPair {
   int si, sj;                  // reference order: si >= sj (shell indices)
   int la, lb;                  // angular momenta of a, b (la >= lb)
   int ca, cb;                  // first AO of a, b among the AOs of its angular momentum (ColMap; J/K records)
-  int kt;                      // first piece of its primitive pairs in JKParams::kt64 / kt32
+  unsigned kt;                 // pairs of two s shells: first piece of its primitive pairs in JKParams::kt64 / kt32
 };
 
 struct PrimPair {              // 64 bytes: one cache line per primitive pair
@@ -137,10 +137,9 @@ struct KernelRes {
 // Bra-row work of one J/K class-pair launch: block i takes bra pair
 // item[i*(1+OQPH_NBKT)] and, for each ket bucket b, the first
 // item[i*(1+OQPH_NBKT) + 1 + b] kets of that bucket
-// (ket[kb[b] ...]); blocks are ordered by decreasing cost.
+// (device pairs kofs + kb[b] ...); blocks are ordered by decreasing cost.
 struct BraWork {
   const int* item;
-  const int* ket;
   int kb[OQPH_NBKT + 1];
   int nitem;
   int jbase, kofs;  // as WaveWork
@@ -224,7 +223,7 @@ struct JKParams {
   // coalesced instead of through three dependent gathers.
   const double* Dk;
   const double* dpm;
-  // The primitive-pair records by pieces of two fields, 64 consecutive pairs of
+  // The primitive-pair records of two s shells by pieces of two fields, 64 consecutive pairs of
   // a list bucket side by side: piece j (0 .. 2) of pair i's record k at
   // kt + (3 k + j) 64.  A wavefront's kets are consecutive pairs, so each piece
   // is one contiguous read instead of 64 cache lines.

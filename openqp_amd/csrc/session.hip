@@ -930,21 +930,19 @@ static int prepare_geometry(oqph_session* s) {
         dpr32.push_back(f32_record(dpr.back()));
       }
     }
-    // groups of 64 consecutive pairs of a bucket, each with the records of its longest
+    // pairs of two s shells (class 0, the only kets read by pieces): groups of 64
+    // consecutive pairs of a bucket, each with the records of its longest
     long long pieces = 0;
-    for (int c = 0; c < 10; ++c)
-      for (int b = 0; b < NBKT; ++b) {
-        const size_t k1 = s->cls_off[c] + s->kbs[c][b + 1];
-        for (size_t g = s->cls_off[c] + s->kbs[c][b]; g < k1; g += 64) {
-          int n = 0;
-          for (size_t i = g; i < std::min(g + 64, k1); ++i) {
-            n = std::max(n, dp[i].nprim);
-            dp[i].kt = (int)(pieces + (long long)(i - g));
-          }
-          pieces += 192ll * n;
+    for (int b = 0; b < NBKT; ++b)
+      for (size_t g = s->kbs[0][b]; g < (size_t)s->kbs[0][b + 1]; g += 64) {
+        int n = 0;
+        for (size_t i = g; i < std::min(g + 64, (size_t)s->kbs[0][b + 1]); ++i) {
+          n = std::max(n, dp[i].nprim);
+          dp[i].kt = (unsigned)(pieces + (long long)(i - g));
         }
+        pieces += 192ll * n;
       }
-    if (pieces > 0x7fffffffll) {
+    if (pieces > 0xffffffffll) {
       set_err("%lld primitive-pair pieces exceed the 32-bit index", pieces);
       return 3;
     }
@@ -973,7 +971,7 @@ static int prepare_geometry(oqph_session* s) {
                         (rc = upload_sync(s->d_prims32.p, dpr32.data(), dpr32.size() * sizeof(PrimF32), s->stream)) ||
                         (rc = upload_sync(s->d_cls.p, ident.data(), ident.size() * sizeof(int), s->stream))))
       return rc;
-    launch_ktrans(s->d_pairs.p, (int)dp.size(), s->d_prims.p, s->d_prims32.p, s->d_kt64.p, s->d_kt32.p, s->stream);
+    launch_ktrans(s->d_pairs.p, (int)s->cls_off[1], s->d_prims.p, s->d_prims32.p, s->d_kt64.p, s->d_kt32.p, s->stream);
   }
   build_families(s);
   if ((rc = prepare_chunks(s, prims))) return rc;
@@ -1766,7 +1764,6 @@ static int prepare_lists(oqph_session* s, double maxden, bool two) {
     L.ch0 = p.ch0;
     L.item0 = p.item0;
     if (p.rows) {
-      L.bw.ket = s->d_cls.p + s->cls_off[p.ck];
       L.bw.jbase = s->jbase[p.ck];
       L.bw.kofs = (int)s->cls_off[p.ck];
       for (int b = 0; b <= NBKT; ++b) L.bw.kb[b] = s->kbs[p.ck][b];
