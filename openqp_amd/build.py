@@ -63,7 +63,7 @@ def _cost(c):
 # headers each translation unit depends on (cache key = unit + these + flags)
 DEPS = {
     "jk_class.hip": ["jk_device.h", "jkg_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
-    "jkc_class.hip": ["jkc_device.h", "jk_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
+    "jkc_class.hip": ["jkc_device.h", "launch_grid.h", "jk_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                       "rys_table_f32.inc"],
     "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "session.hip": ["oqph_common.h", "response.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],

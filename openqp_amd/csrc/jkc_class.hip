@@ -2,6 +2,7 @@
 // class (XA XB | XC XD): Cartesian and pure AOs, closed- and open-shell pass.
 // Built once per class with -DXA=.. -DXB=.. -DXC=.. -DXD=..
 #include "jkc_device.h"
+#include "launch_grid.h"
 
 namespace oqph {
 
@@ -13,8 +14,8 @@ static_assert(jkc_fits<XA, XB, XC, XD>(), "the class does not fit the cooperativ
 template <bool PURE, bool TWO>
 static void go(const JKParams& p, const WaveWork& ww, hipStream_t s) {
   const int kpb = ww.kpb > 0 ? ww.kpb : 64;
-  const unsigned nb = (unsigned)(ww.nwaves * (64 / kpb));
-  hipLaunchKernelGGL((k_jkc<XA, XB, XC, XD, PURE, TWO>), dim3(nb), dim3(64), 0, s, p, ww);
+  const Grid2 g = wave_grid(ww.nwaves * (64 / kpb));
+  hipLaunchKernelGGL((k_jkc<XA, XB, XC, XD, PURE, TWO>), dim3(g.x, g.y), dim3(64), 0, s, p, ww);
 }
 
 void OQPH_JKC_NAME(launch_jkc_, XA, XB, XC, XD)(bool pure, const JKParams& p, const WaveWork& ww, hipStream_t s) {

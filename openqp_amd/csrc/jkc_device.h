@@ -76,8 +76,8 @@ void k_jkc(JKParams prm, WaveWork ww) {
   const int lane = (int)threadIdx.x, l = lane & (W - 1), q = lane / W;
   // ---- the block's kets: [sub kpb, (sub + 1) kpb) of one 64-ket chunk of one segment
   const int kpb = ww.kpb > 0 ? ww.kpb : 64, per = 64 / kpb;
-  const long long wave = (long long)blockIdx.x / per;
-  const int sub = (int)((long long)blockIdx.x - wave * per);
+  const long long block = (long long)blockIdx.y * gridDim.x + blockIdx.x, wave = block / per;
+  const int sub = (int)(block - wave * per);
   if (wave >= ww.nwaves) return;  // block-uniform
   int lo = 0, hi = ww.nseg;
   while (hi - lo > 1) {
