@@ -1054,6 +1054,16 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
     const Split sp = bra_lds && 2 * n <= nw * 64 ? split_of(n, nw * 64, nbra64, b, lane) : split_none();
     const int kw = 64 >> sp.lg;  // kets per wavefront
     const bool head = sp.sub == 0;
+    // 64 consecutive kets take FP32 together, also where a wavefront holds only
+    // some of them (in one pass of the loop: n lanes per ket fit the block):
+    // spreading kets over lanes must not move quartets from FP64 to FP32
+    // ((H2O)4/6-31G: a fifth more)
+    bool low = false;
+    if constexpr (T32)
+      if (prm.mixed && sp.n > 1) {
+        const int kc = (wv * kw & ~63) + lane;
+        low = __ballot(kc < n && quartet_bound(prm, ip, bw.kofs + kbase + kc) >= prm.fp32_cut) == 0ull;
+      }
     for (int k0 = wv * kw; k0 < n; k0 += nw * kw) {
       const int k = k0 + (lane >> sp.lg);
       const bool active = k < n;
@@ -1089,17 +1099,7 @@ __attribute__((amdgpu_waves_per_eu(JKB<LA, LB, LC, LD>::min_waves))) void k_jkb(
       int nprim = 0;
       bool lowp = false;
       if constexpr (T32)
-        if (prm.mixed) {
-          bool high = !skip && bound >= prm.fp32_cut;
-          // 64 consecutive kets take FP32 together, also where a wavefront holds
-          // only some of them: spreading kets over lanes must not move quartets
-          // from FP64 to FP32 ((H2O)4/6-31G: a fifth more)
-          if (sp.n > 1) {
-            const int kc = (k0 & ~63) + lane;
-            high = kc < n && quartet_bound(prm, ip, bw.kofs + kbase + kc) >= prm.fp32_cut;
-          }
-          lowp = __ballot(high) == 0ull;
-        }
+        lowp = prm.mixed && (sp.n > 1 ? low : __ballot(!skip && bound >= prm.fp32_cut) == 0ull);
       if (!skip) {
         if constexpr (T32) {
           if (lowp) {

@@ -391,6 +391,16 @@ void k_jkg(JKParams prm, BraWork bw, ColMap cm, ChunkView cv) {
     const Split sp = TILE || 2 * n > nw * 64 ? split_none() : split_of(n, nw * 64, ncp, b, lane);
     const int kw = 64 >> sp.lg;  // kets per wavefront
     const bool head = sp.sub == 0;
+    bool low = false;  // kets over several lanes: FP32 by 64 consecutive kets, as in k_jkb
+    if constexpr (T32 && !TILE)
+      if (prm.mixed && sp.n > 1) {
+        const int kc = (wv * kw & ~63) + lane, ic = bw.kofs + kbase + kc;
+        bool high = false;
+#pragma unroll 1
+        for (int m = 0; m < nmem; ++m)
+          if (kc < n && (!SAME || ic <= s_mi[m][0])) high |= quartet_bound(prm, s_mi[m][0], ic) >= prm.fp32_cut;
+        low = __ballot(high) == 0ull;
+      }
     for (int k0 = wv * kw; k0 < n; k0 += nw * kw) {
       // the member tables are read from LDS where they are used: an opaque
       // zero offset keeps the compiler from hoisting every member's fields
@@ -443,17 +453,7 @@ void k_jkg(JKParams prm, BraWork bw, ColMap cm, ChunkView cv) {
       n_comp += head ? __popc(live) : 0;
       bool lowp = false;
       if constexpr (T32)
-        if (prm.mixed) {
-          bool high = live != 0u && bmax >= prm.fp32_cut;
-          if (!TILE && sp.n > 1) {  // by 64 consecutive kets, as in k_jkb
-            const int kc = (k0 & ~63) + lane, ic = bw.kofs + kbase + kc;
-            high = false;
-#pragma unroll 1
-            for (int m = 0; m < nmem; ++m)
-              if (kc < n && (!SAME || ic <= mi[m][0])) high |= quartet_bound(prm, mi[m][0], ic) >= prm.fp32_cut;
-          }
-          lowp = __ballot(high) == 0ull;
-        }
+        lowp = prm.mixed && (!TILE && sp.n > 1 ? low : __ballot(live != 0u && bmax >= prm.fp32_cut) == 0ull);
       // each member's final AO block; the (e0|f0) accumulators live only
       // inside the precision branch that fills them
       double Vall[NM][NBLK];
