@@ -10,7 +10,7 @@
 // bound the kernel, not the matrix units.  Adding every quartet into nd matrices
 // instead costs 12 nd atomics and as many gathers per s quartet.  (H2O)8/6-31G, 28
 // densities: 50.9 ms per pass then, now 0.31 + 0.12 ms for the two products (4.5
-// TB/s of T) and 1.75 ms in all; other sizes at response_dense() in session.hip.
+// TB/s of T) and 1.75 ms in all; other sizes at response_elems() in session.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -25,22 +25,24 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 // raw[y][w][c][v] (v fastest) -> M[q = v nmat + c][y][w], rows of ld doubles, the tail cleared
 __global__ void k_rsp_pack(const double* __restrict__ raw, int n, int ld, int nmat, int nf, double* __restrict__ M) {
   const int nd = nmat * nf;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)n * ld * nd) return;
-  const int k = (int)(i % nd);  // c nf + v
-  const long long yw = i / nd;
-  const int w = (int)(yw % ld), y = (int)(yw / ld);
-  const int q = (k % nf) * nmat + k / nf;
-  M[((size_t)q * n + y) * ld + w] = w < n ? raw[((size_t)y * n + w) * nd + k] : 0.0;
+  const long long m = (long long)n * ld * nd, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += step) {
+    const int k = (int)(i % nd);  // c nf + v
+    const long long yw = i / nd;
+    const int w = (int)(yw % ld), y = (int)(yw / ld);
+    const int q = (k % nf) * nmat + k / nf;
+    M[((size_t)q * n + y) * ld + w] = w < n ? raw[((size_t)y * n + w) * nd + k] : 0.0;
+  }
 }
 
 // F[q][y][w] -> raw[y][w][c][v]
 __global__ void k_rsp_unpack(const double* __restrict__ F, int n, int nmat, int nf, double* __restrict__ raw) {
   const int nd = nmat * nf;
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)n * n * nd) return;
-  const int k = (int)(i % nd), q = (k % nf) * nmat + k / nf;
-  raw[i] = F[(size_t)q * n * n + i / nd];
+  const long long m = (long long)n * n * nd, step = (long long)gridDim.x * blockDim.x;
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += step) {
+    const int k = (int)(i % nd), q = (k % nf) * nmat + k / nf;
+    raw[i] = F[(size_t)q * n * n + i / nd];
+  }
 }
 
 // A block takes 16 CT rows and 16 NV densities; its eight wavefronts take every
@@ -131,14 +133,17 @@ __global__ __launch_bounds__(512) void k_response(ResponseParams r) {
   }
 }
 
+// blocks of 256 for m elements, at most 64 per CU: one thread per element would end at 2^32
+static unsigned rsp_blocks(long long m) { return (unsigned)std::min<long long>((m + 255) / 256, 16384); }
+
 void launch_rsp_pack(const double* raw, int n, int ld, int nmat, int nf, double* M, hipStream_t s) {
   const long long m = (long long)n * ld * nmat * nf;
-  hipLaunchKernelGGL(k_rsp_pack, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, raw, n, ld, nmat, nf, M);
+  hipLaunchKernelGGL(k_rsp_pack, dim3(rsp_blocks(m)), dim3(256), 0, s, raw, n, ld, nmat, nf, M);
 }
 
 void launch_rsp_unpack(const double* F, int n, int nmat, int nf, double* raw, hipStream_t s) {
   const long long m = (long long)n * n * nmat * nf;
-  hipLaunchKernelGGL(k_rsp_unpack, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, F, n, nmat, nf, raw);
+  hipLaunchKernelGGL(k_rsp_unpack, dim3(rsp_blocks(m)), dim3(256), 0, s, F, n, nmat, nf, raw);
 }
 
 template <int NV, bool COUL>

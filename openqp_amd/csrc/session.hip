@@ -219,7 +219,6 @@ struct oqph_session {
   // per build
   DBuf<double> d_D, d_F, d_dsh, d_tmp;
   DBuf<double> d_gD, d_gF;  // response-pass densities (nd x nbf x row length) and outputs (nd x nbf x nbf)
-  DBuf<double> d_gR;        // the caller's array, before and after
   DBuf<double> d_gT;        // integrals of the dense response pass
   DBuf<int> d_gcoul;        // per density: Coulomb or not; then the two column lists of k_response
   DBuf<long long> d_off;
@@ -2174,11 +2173,14 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
 // 0.66 ms, (H2O)8/6-31G 50.9 -> 1.75, (H2O)14/6-31G 137 -> 8.1, (H2O)8/cc-pVDZ (192
 // AOs, 5.7 GB) 391 -> 14.6, one water/cc-pVTZ 51 -> 5.5; 7 densities of (H2O)8/6-31G
 // 32 -> 1.4: dense wins at every size it fits.
-static bool response_dense(oqph_session* s) {
+static size_t response_elems(const oqph_session* s) {  // 0: not dense
   const char* e = getenv("OQPH_RESPONSE");  // 0: never
-  if (e && e[0] == '0') return false;
+  if (e && e[0] == '0') return 0;
   const size_t n = (size_t)s->nbf, ld = (n + 15) & ~(size_t)15, need = n * (n + 1) / 2 * n * ld;
-  if (need * sizeof(double) > ((size_t)16 << 30)) return false;
+  return need * sizeof(double) > ((size_t)16 << 30) ? 0 : need;
+}
+// after the pass's other buffers, so that these never fail for it
+static bool response_alloc(oqph_session* s, size_t need) {
   if (need <= s->d_gT.n && s->d_gT.p) return true;
   size_t avail = 0, total = 0;
   if (hipMemGetInfo(&avail, &total) != hipSuccess || 2 * need * sizeof(double) > avail || s->d_gT.ensure(need)) {
@@ -2379,7 +2381,7 @@ int oqph_session_destroy(oqph_session* s) {
   s->d_am.release(); s->d_pure.release(); s->d_gseg.release(); s->d_gchoff.release(); s->d_Dc.release(); s->d_de.release();
   s->d_kt64.release(); s->d_kt32.release(); s->d_aooff.release(); s->d_nao.release(); s->d_colao.release(); s->d_items.release(); s->d_Dt.release(); s->d_D.release(); s->d_F.release(); s->d_dsh.release();
   s->d_tmp.release(); s->d_off.release(); s->d_ctr.release();
-  s->d_gD.release(); s->d_gF.release(); s->d_gR.release(); s->d_gT.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
+  s->d_gD.release(); s->d_gF.release(); s->d_gT.release(); s->d_gcoul.release(); s->d_gM.release(); s->d_gMc.release();
   for (auto e : s->pev) hipEventDestroy(e);
   if (s->ev0) hipEventDestroy(s->ev0);
   if (s->ev1) hipEventDestroy(s->ev1);
@@ -2705,24 +2707,27 @@ int oqph_mrsf_int2(oqph_session* s, int nf, int nmat, int ncoul, const double* d
       dsh[(size_t)si * nsh + sj] = dsh[(size_t)sj * nsh + si] = dm;
       maxden = std::max(maxden, dm);
     }
-  const bool dense = response_dense(s);
-  const int ldd = dense ? (nbf + 15) & ~15 : nbf;
-  if ((rc = s->d_dsh.ensure((size_t)nsh * nsh)) || (rc = s->d_gD.ensure(nd * nbf * ldd)) ||
-      (rc = s->d_gR.ensure(nd * n2)) || (rc = s->d_gF.ensure(nd * n2)) || (rc = s->d_gcoul.ensure(3 * nd)))
+  const size_t need = response_elems(s);
+  const int ldp = need ? (nbf + 15) & ~15 : nbf;
+  if ((rc = s->d_dsh.ensure((size_t)nsh * nsh)) || (rc = s->d_gD.ensure(nd * nbf * ldp)) ||
+      (rc = s->d_gF.ensure(nd * n2)) || (rc = s->d_gcoul.ensure(3 * nd)))
     return rc;
+  const bool dense = need && response_alloc(s, need);
+  const int ldd = dense ? ldp : nbf;
   // synchronous: dsh and coul are host locals that an early return frees
-  if ((rc = upload_sync(s->d_gR.p, d3, nd * n2 * sizeof(double), s->stream)) ||
+  if ((rc = upload_sync(s->d_gF.p, d3, nd * n2 * sizeof(double), s->stream)) ||
       (rc = upload_sync(s->d_dsh.p, dsh.data(), dsh.size() * sizeof(double), s->stream)) ||
       (rc = upload_sync(s->d_gcoul.p, coul.data(), coul.size() * sizeof(int), s->stream)))
     return rc;
-  // the reference's (v, c, mu, nu) order into one matrix per density, and back
-  launch_rsp_pack(s->d_gR.p, nbf, ldd, nmat, nf, s->d_gD.p, s->stream);
+  // the reference's (v, c, mu, nu) order, uploaded into the output slabs, into one
+  // matrix per density; and back through the density slabs
+  launch_rsp_pack(s->d_gF.p, nbf, ldd, nmat, nf, s->d_gD.p, s->stream);
   if ((rc = build_general(s, dense, (int)nd, s->d_gD.p, ldd, s->d_gF.p, s->d_gcoul.p, (int)nco, maxden, se, sc, st,
                           s->stream)))
     return rc;
-  launch_rsp_unpack(s->d_gF.p, nbf, nmat, nf, s->d_gR.p, s->stream);
+  launch_rsp_unpack(s->d_gF.p, nbf, nmat, nf, s->d_gD.p, s->stream);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(f3, s->d_gR.p, nd * n2 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
+  HIPCHK(hipMemcpyAsync(f3, s->d_gD.p, nd * n2 * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HIPCHK(hipStreamSynchronize(s->stream));
   return 0;
 }
