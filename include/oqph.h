@@ -237,6 +237,16 @@ int oqph_last_profile(oqph_session *s, int maxn, int *cls, double *ms, double *f
  * launches copied. */
 int oqph_last_counters(oqph_session *s, int maxn, unsigned long long *ctr);
 
+/* Kernels of the last two-electron gradient, up to maxn entries: class code as
+ * oqph_last_profile, plus 10000 for the split form of k_grad (a ket's primitive
+ * quartets over several lanes), 20000 for the run-time-class kernel k_gradh (40000 +
+ * its number of classes for a multi-class launch), 80000 for the cooperative kernel
+ * k_gradc.  Returns the number of launches.  No counterpart in the seam. */
+int oqph_last_gradient_kernels(oqph_session *s, int maxn, int *cls);
+/* 1: the last response pass stored its integrals and contracted them; 0: it added
+ * quartet by quartet; -1: there was none.  No counterpart in the seam. */
+int oqph_last_response_dense(oqph_session *s);
+
 /* Schwarz table (nsh*nsh, symmetric) of the current geometry. */
 int oqph_schwarz(oqph_session *s, double *q);
 

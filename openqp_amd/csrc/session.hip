@@ -220,6 +220,7 @@ struct oqph_session {
   DBuf<double> d_D, d_F, d_dsh, d_tmp;
   DBuf<double> d_gD, d_gF;  // response-pass densities (nd x nbf x row length) and outputs (nd x nbf x nbf)
   DBuf<double> d_gT;        // integrals of the dense response pass
+  int response_kind = -1;   // the last response pass: 1 dense, 0 quartet by quartet
   DBuf<int> d_gcoul;        // per density: Coulomb or not; then the two column lists of k_response
   DBuf<long long> d_off;
   DBuf<unsigned long long> d_ctr;
@@ -2534,6 +2535,20 @@ int oqph_last_counters(oqph_session* s, int maxn, unsigned long long* ctr) {
   return n;
 }
 
+int oqph_last_gradient_kernels(oqph_session* s, int maxn, int* cls) {
+  if (!s || !cls) return -4;
+  const int n = (int)std::min<size_t>((size_t)std::max(maxn, 0), s->glaunches.size());
+  for (int i = 0; i < n; ++i) {
+    const auto& L = s->glaunches[i];
+    const bool split = !L.coop && !L.hl && L.ww.kpb > 0 && L.ww.kpb < 64;
+    cls[i] = L.multi ? 40000 + L.tl.ntask
+                     : (L.coop ? 80000 : L.hl ? 20000 : split ? 10000 : 0) + L.la * 1000 + L.lb * 100 + L.lc * 10 + L.ld;
+  }
+  return n;
+}
+
+int oqph_last_response_dense(oqph_session* s) { return s ? s->response_kind : -4; }
+
 int oqph_schwarz(oqph_session* s, double* q) {
   if (!s || !q) return 4;
   int rc = prepare_geometry(s);
@@ -2714,6 +2729,7 @@ int oqph_mrsf_int2(oqph_session* s, int nf, int nmat, int ncoul, const double* d
     return rc;
   const bool dense = need && response_alloc(s, need);
   const int ldd = dense ? ldp : nbf;
+  s->response_kind = dense ? 1 : 0;
   // synchronous: dsh and coul are host locals that an early return frees
   if ((rc = upload_sync(s->d_gF.p, d3, nd * n2 * sizeof(double), s->stream)) ||
       (rc = upload_sync(s->d_dsh.p, dsh.data(), dsh.size() * sizeof(double), s->stream)) ||

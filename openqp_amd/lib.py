@@ -33,7 +33,7 @@ EXPORTS = ["routec_fock_jk", "routec_grad2", "oqph_session_create", "oqph_sessio
            "oqph_fock_jk_noalloc", "oqph_last_counters", "oqph_session_set_grad_precision", "oqph_mrsf_int2",
            "routec_sig_init", "routec_sig_set_scale", "routec_sig_iter", "routec_sig_free", "oqph_grad2_mrsf",
            "routec_grad2_mrsf", "routec_vxc", "oqph_session_set_xc", "oqph_xc_functional_info", "oqph_vxc",
-           "oqph_xc_grid", "oqph_xc_grid_stats"]
+           "oqph_xc_grid", "oqph_xc_grid_stats", "oqph_last_gradient_kernels", "oqph_last_response_dense"]
 
 
 class OqphError(RuntimeError):
@@ -85,6 +85,8 @@ def load(path: str | None = None):
     L.oqph_session_set_profiling.argtypes = [vp, C.c_int]
     _pl = np.ctypeslib.ndpointer(dtype=np.int64, flags="C_CONTIGUOUS")
     L.oqph_last_profile.argtypes = [vp, C.c_int, _pi, _pd, _pd, _pl, _pl]
+    L.oqph_last_gradient_kernels.argtypes = [vp, C.c_int, _pi]
+    L.oqph_last_response_dense.argtypes = [vp]
     L.oqph_last_counters.argtypes = [vp, C.c_int, np.ctypeslib.ndpointer(dtype=np.uint64, flags="C_CONTIGUOUS")]
     L.oqph_int1e.argtypes = [C.c_int, _pi, _pi, _pi, _pi, _pd, _pd, C.c_int, _pd, _pd, C.c_void_p, C.c_void_p,
                              C.c_void_p]
@@ -222,6 +224,21 @@ class FockBuilder:
                      flops=float(fl[i]), quartets=int(q[i]), prims=int(pq[i]), prims_eval=int(ctr[8 * i + 5]),
                      screened=int(ctr[8 * i + 1]), slots=int(ctr[8 * i + 6]))
                 for i in range(max(m, 0))]
+
+    def last_gradient_kernels(self):
+        """(class code, kernel) of every launch of the last gradient: "k_gradc" (cooperative
+        kernel), "k_grad", "k_grad_split" (a ket over several lanes), "k_gradh" or, for several
+        run-time classes (class code 40000 + their number), "k_gradh_multi"."""
+        cls = np.zeros(256, np.int32)
+        m = load().oqph_last_gradient_kernels(self._s, cls.size, cls)
+        kern = lambda c: ("k_gradc" if c >= 80000 else "k_gradh_multi" if c >= 40000 else "k_gradh" if c >= 20000
+                          else "k_grad_split" if c >= 10000 else "k_grad")
+        return [(c if 40000 <= c < 50000 else c % 10000, kern(c)) for c in (int(x) for x in cls[:max(m, 0)])]
+
+    def last_response_dense(self):
+        """Whether the last mrsf_int2 stored its integrals (None: there was none)."""
+        r = load().oqph_last_response_dense(self._s)
+        return None if r < 0 else bool(r)
 
     def schwarz(self) -> np.ndarray:
         q = np.zeros(self.bas.nsh * self.bas.nsh)
