@@ -334,9 +334,9 @@ __global__ void k_grid(GridArgs g) {
 }
 
 // ------------------------------------------------------------ batches and groups
-// The batches are cut into groups of at most GROUP_ELEMS basis-function values;
-// a build takes one launch of each kernel per group, over all its batches.  A
-// launch per batch, three gathers of the density and three library products with
+// The batches are cut into groups of at most GROUP_ELEMS basis-function values (fewer
+// where the device is short of memory); a build takes one launch of each kernel per
+// group, over all its batches.  A launch per batch, three gathers of the density and three library products with
 // phi, its gradient, X and Y in memory took 65 ms for (H2O)32/6-31G(d) with its
 // 1045 batches of 4 bohr; this 15.9 (groups of 2^25 values: 28.1 against 23.8 for
 // 2^28, both on boxes of 4 bohr).
@@ -862,6 +862,8 @@ struct XCState {
   std::vector<Batch> batches;
   std::vector<Group> groups;
   int max_nb = 0;
+  std::vector<int> idx;                             // AO of every column (d_idx)
+  long long limit = 0;                              // elements of a group (build_groups)
   long long max_grp = 0, max_vb = 0, max_tile = 0;  // largest group: phi, V_b, point tiles
   Buf<double> d_pts, d_xf, d_D, d_pk, d_acc, d_phi, d_Y, d_rho, d_coef, d_Vb, d_V;
   Buf<DBatch> d_batch;
@@ -944,6 +946,96 @@ bool upload(Buf<T>& b, const T* h, size_t n, hipStream_t st) {
     return false;
   }
   return true;
+}
+
+// Cuts the batches into groups of at most `limit` basis-function values and V_b
+// elements, with their point tiles and V_b tiles, and uploads them.
+int build_groups(XCState* x, const oqph::SessionView& v, long long limit) {
+  std::vector<DBatch> db;
+  std::vector<int2> tile;
+  std::vector<int4> vt;
+  std::vector<long long> vptr;  // per group: nbf + 1 starts in vent
+  std::vector<int2> vent;       // per AO: the batches that hold it and its column there
+  x->groups.clear();
+  long long max_grp = 0, max_vb = 0, max_tile = 0;
+  for (int b0 = 0; b0 < (int)x->batches.size();) {
+    Group g{b0, b0, (long long)tile.size(), 0, (long long)vt.size(), 0, 0, 0};
+    std::vector<int4> list[8];  // tiles of a part stay on one XCD: blocks are dealt to the eight in turn
+    while (g.b1 < (int)x->batches.size()) {
+      const Batch& b = x->batches[g.b1];
+      const int ld = (b.npts + TILE - 1) / TILE * TILE, nparts = (ld + PART - 1) / PART, nt = (b.nb + 63) / 64;
+      const long long phi = (long long)ld * b.nb, vb = (long long)nparts * b.nb * b.nb;
+      if (g.b1 > b0 && (g.ngrp + phi > limit || g.nvb + vb > limit)) break;
+      db.push_back({b.p0, g.ngrp, g.nvb, b.npts, ld, b.sh0, b.nsh, b.ao0, b.nb, nparts, 0});
+      for (int t = 0; t < ld / TILE; ++t) tile.push_back(int2{g.b1, t});
+      for (int k = 0; k < nparts; ++k) {
+        auto& l = *std::min_element(list, list + 8, [](const auto& p, const auto& q) { return p.size() < q.size(); });
+        for (int m = 0; m < nt; ++m)
+          for (int c = 0; c < nt; ++c) l.push_back(int4{g.b1, k, m, c});
+      }
+      g.ngrp += phi;
+      g.nvb += vb;
+      ++g.b1;
+    }
+    size_t len = 0;
+    for (auto& l : list) len = std::max(len, l.size());
+    for (size_t i = 0; i < len; ++i)
+      for (auto& l : list) vt.push_back(i < l.size() ? l[i] : int4{-1, 0, 0, 0});
+    const size_t p0 = vptr.size(), e0 = vent.size();
+    vptr.resize(p0 + v.nbf + 1, 0);
+    for (int k = b0; k < g.b1; ++k)
+      for (int i = 0; i < x->batches[k].nb; ++i) ++vptr[p0 + 1 + x->idx[x->batches[k].ao0 + i]];
+    vptr[p0] = (long long)e0;
+    for (int i = 0; i < v.nbf; ++i) vptr[p0 + 1 + i] += vptr[p0 + i];
+    vent.resize((size_t)vptr[p0 + v.nbf]);
+    std::vector<long long> at(vptr.begin() + p0, vptr.end() - 1);
+    for (int k = b0; k < g.b1; ++k)
+      for (int i = 0; i < x->batches[k].nb; ++i) vent[at[x->idx[x->batches[k].ao0 + i]]++] = int2{k, i};
+    g.ntile = (long long)tile.size() - g.tile0;
+    g.nvt = (long long)vt.size() - g.vt0;
+    max_grp = std::max(max_grp, g.ngrp);
+    max_vb = std::max(max_vb, g.nvb);
+    max_tile = std::max(max_tile, g.ntile);
+    x->groups.push_back(g);
+    b0 = g.b1;
+  }
+  x->limit = limit;
+  x->max_grp = max_grp;
+  x->max_vb = max_vb;
+  x->max_tile = max_tile;
+  hipStream_t st = v.stream;
+  const bool ok = upload(x->d_batch, db.data(), db.size(), st) && upload(x->d_tile, tile.data(), tile.size(), st) &&
+                  upload(x->d_vt, vt.data(), vt.size(), st) && upload(x->d_vptr, vptr.data(), vptr.size(), st) &&
+                  upload(x->d_vent, vent.data(), vent.size(), st);
+  return hipStreamSynchronize(st) == hipSuccess && ok ? 0 : 3;
+}
+
+// Device memory of a build: D, V and the packed matrices, and for the largest group phi,
+// Y and V_b (up to 2 GB, and 4 GB each for two spins), rho and its coefficients.  Where
+// the device has not that much left the groups get smaller, down to one batch each.
+int workspace(XCState* x, const oqph::SessionView& v, size_t ns) {
+  const size_t nbf = (size_t)v.nbf, ntri = nbf * (nbf + 1) / 2, nn = nbf * nbf;
+  if (!x->d_pk.ensure(ntri * ns) || !x->d_D.ensure(nn * ns) || !x->d_V.ensure(nn * ns) || !x->d_acc.ensure(2)) return 3;
+  const char* e = getenv("OQPH_XC_WORKSPACE");  // bytes of the group arrays counted as available (tests)
+  const double most = e ? atof(e) : 1e300;
+  for (;;) {
+    const size_t npad = (size_t)x->max_tile * TILE;
+    const double bytes = 8.0 * ((1.0 + ns) * x->max_grp + (double)ns * x->max_vb + 8.0 * ns * npad);
+    if (bytes <= most && x->d_phi.ensure((size_t)x->max_grp) && x->d_Y.ensure(ns * x->max_grp) &&
+        x->d_Vb.ensure(ns * x->max_vb) && x->d_rho.ensure(4 * ns * npad) && x->d_coef.ensure(4 * ns * npad))
+      return 0;
+    (void)hipGetLastError();  // out of memory
+    if (x->groups.size() == x->batches.size()) {
+      err("XC: no device memory for a group of one batch (%.0f bytes)", bytes);
+      return 3;
+    }
+    for (auto* b : {&x->d_phi, &x->d_Y, &x->d_Vb, &x->d_rho, &x->d_coef}) b->release();
+    const long long limit = std::max<long long>(std::min(x->limit, std::max(x->max_grp, x->max_vb)) / 4, 1);
+    if (const int rc = build_groups(x, v, limit)) {
+      x->grid_ready = false;
+      return rc;
+    }
+  }
 }
 
 int build_grid(XCState* x, const oqph::SessionView& v) {
@@ -1073,55 +1165,6 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
     }
     t0 = t1;
   }
-  // groups of batches, their point tiles and V_b tiles
-  std::vector<DBatch> db;
-  std::vector<int2> tile;
-  std::vector<int4> vt;
-  std::vector<long long> vptr;  // per group: nbf + 1 starts in vent
-  std::vector<int2> vent;       // per AO: the batches that hold it and its column there
-  x->groups.clear();
-  long long max_grp = 0, max_vb = 0, max_tile = 0;
-  for (int b0 = 0; b0 < (int)x->batches.size();) {
-    Group g{b0, b0, (long long)tile.size(), 0, (long long)vt.size(), 0, 0, 0};
-    std::vector<int4> list[8];  // tiles of a part stay on one XCD: blocks are dealt to the eight in turn
-    while (g.b1 < (int)x->batches.size()) {
-      const Batch& b = x->batches[g.b1];
-      const int ld = (b.npts + TILE - 1) / TILE * TILE, nparts = (ld + PART - 1) / PART, nt = (b.nb + 63) / 64;
-      const long long phi = (long long)ld * b.nb, vb = (long long)nparts * b.nb * b.nb;
-      if (g.b1 > b0 && (g.ngrp + phi > GROUP_ELEMS || g.nvb + vb > GROUP_ELEMS)) break;
-      db.push_back({b.p0, g.ngrp, g.nvb, b.npts, ld, b.sh0, b.nsh, b.ao0, b.nb, nparts, 0});
-      for (int t = 0; t < ld / TILE; ++t) tile.push_back(int2{g.b1, t});
-      for (int k = 0; k < nparts; ++k) {
-        auto& l = *std::min_element(list, list + 8, [](const auto& p, const auto& q) { return p.size() < q.size(); });
-        for (int m = 0; m < nt; ++m)
-          for (int c = 0; c < nt; ++c) l.push_back(int4{g.b1, k, m, c});
-      }
-      g.ngrp += phi;
-      g.nvb += vb;
-      ++g.b1;
-    }
-    size_t len = 0;
-    for (auto& l : list) len = std::max(len, l.size());
-    for (size_t i = 0; i < len; ++i)
-      for (auto& l : list) vt.push_back(i < l.size() ? l[i] : int4{-1, 0, 0, 0});
-    const size_t p0 = vptr.size(), e0 = vent.size();
-    vptr.resize(p0 + v.nbf + 1, 0);
-    for (int k = b0; k < g.b1; ++k)
-      for (int i = 0; i < x->batches[k].nb; ++i) ++vptr[p0 + 1 + idx[x->batches[k].ao0 + i]];
-    vptr[p0] = (long long)e0;
-    for (int i = 0; i < v.nbf; ++i) vptr[p0 + 1 + i] += vptr[p0 + i];
-    vent.resize((size_t)vptr[p0 + v.nbf]);
-    std::vector<long long> at(vptr.begin() + p0, vptr.end() - 1);
-    for (int k = b0; k < g.b1; ++k)
-      for (int i = 0; i < x->batches[k].nb; ++i) vent[at[idx[x->batches[k].ao0 + i]]++] = int2{k, i};
-    g.ntile = (long long)tile.size() - g.tile0;
-    g.nvt = (long long)vt.size() - g.vt0;
-    max_grp = std::max(max_grp, g.ngrp);
-    max_vb = std::max(max_vb, g.nvb);
-    max_tile = std::max(max_tile, g.ntile);
-    x->groups.push_back(g);
-    b0 = g.b1;
-  }
   // device copies
   std::vector<double> xf(400);
   oqph_host::build_xform(reinterpret_cast<double(*)[2][10][10]>(xf.data()));
@@ -1133,16 +1176,11 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
        upload(x->d_idx, idx.data(), idx.size(), st) && upload(x->d_am, v.am, (size_t)v.nsh, st) &&
        upload(x->d_harm, harm.data(), harm.size(), st) && upload(x->d_atom, v.atom, (size_t)v.nsh, st) &&
        upload(x->d_nprim, v.nprim, (size_t)v.nsh, st) && upload(x->d_poff, v.poff, (size_t)v.nsh, st) &&
-       upload(x->d_ex, v.ex, (size_t)nprim_tot, st) && upload(x->d_cc, v.cc, (size_t)nprim_tot, st) &&
-       upload(x->d_batch, db.data(), db.size(), st) && upload(x->d_tile, tile.data(), tile.size(), st) &&
-       upload(x->d_vt, vt.data(), vt.size(), st) && upload(x->d_vptr, vptr.data(), vptr.size(), st) &&
-       upload(x->d_vent, vent.data(), vent.size(), st);
-  // workspaces of the largest group, for two spins where a build needs them (vxc_run)
-  x->max_grp = max_grp;
-  x->max_vb = max_vb;
-  x->max_tile = max_tile;
-  ok = ok && hipStreamSynchronize(st) == hipSuccess;
+       upload(x->d_ex, v.ex, (size_t)nprim_tot, st) && upload(x->d_cc, v.cc, (size_t)nprim_tot, st);
+  ok = hipStreamSynchronize(st) == hipSuccess && ok;
   if (!ok) return 3;
+  x->idx.swap(idx);
+  if (const int rc = build_groups(x, v, GROUP_ELEMS)) return rc;
   x->grid_ready = true;
   return 0;
 }
@@ -1200,10 +1238,9 @@ int vxc_run(oqph_session* s, const double* d, int nfocks, double* fxc, double* e
   if (rc) return rc;
   const int nbf = v.nbf;
   const size_t ntri = (size_t)nbf * (nbf + 1) / 2, nn = (size_t)nbf * nbf;
-  const size_t ns = (size_t)nfocks, npad = (size_t)x->max_tile * TILE;
-  if (!upload(x->d_pk, d, ntri * ns, st) || !x->d_D.ensure(nn * ns) || !x->d_V.ensure(nn * ns) || !x->d_acc.ensure(2) ||
-      !x->d_phi.ensure((size_t)x->max_grp) || !x->d_Y.ensure(ns * x->max_grp) || !x->d_Vb.ensure(ns * x->max_vb) ||
-      !x->d_rho.ensure(4 * ns * npad) || !x->d_coef.ensure(4 * ns * npad)) {
+  const size_t ns = (size_t)nfocks;
+  if ((rc = workspace(x, v, ns))) return rc;
+  if (!upload(x->d_pk, d, ntri * ns, st)) {
     hipStreamSynchronize(st);  // the upload reads the caller's array
     return 3;
   }
