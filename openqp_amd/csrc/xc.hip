@@ -24,6 +24,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -1105,18 +1106,33 @@ int build_grid(XCState* x, const oqph::SessionView& v) {
     }
   long long nbx[3];
   for (int k = 0; k < 3; ++k) nbx[k] = std::max<long long>(1, (long long)((hi[k] - lo[k]) / BOX) + 1);
-  std::vector<long long> key(n);
-  for (long long t = 0; t < n; ++t) {
-    long long b[3];
-    for (int k = 0; k < 3; ++k) b[k] = std::min(nbx[k] - 1, (long long)((x->grid[4 * t + k] - lo[k]) / BOX));
-    key[t] = (b[0] * nbx[1] + b[1]) * nbx[2] + b[2];
+  std::vector<long long> key(n), order(n);
+  auto box = [&](long long t, int k) { return std::min(nbx[k] - 1, (long long)((x->grid[4 * t + k] - lo[k]) / BOX)); };
+  // Sorted by box, atom-major within a box: by counting while the boxes are not many more
+  // than the points; a sparse system (far fragments) has empty boxes by the billion, and
+  // its points are sorted by their box instead.
+  const double most = 8.0 * (double)n + (1 << 20);
+  if ((double)nbx[0] * nbx[1] * nbx[2] <= most) {
+    const long long nkeys = nbx[0] * nbx[1] * nbx[2];
+    std::vector<long long> start(nkeys + 1, 0);
+    for (long long t = 0; t < n; ++t) {
+      key[t] = (box(t, 0) * nbx[1] + box(t, 1)) * nbx[2] + box(t, 2);
+      ++start[key[t] + 1];
+    }
+    for (long long k = 0; k < nkeys; ++k) start[k + 1] += start[k];
+    for (long long t = 0; t < n; ++t) order[start[key[t]]++] = t;
+  } else {
+    std::vector<std::array<long long, 3>> at(n);
+    for (long long t = 0; t < n; ++t) {
+      at[t] = {box(t, 0), box(t, 1), box(t, 2)};
+      order[t] = t;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](long long i, long long j) { return at[i] < at[j]; });
+    for (long long i = 0, k = 0; i < n; ++i) {
+      if (i > 0 && at[order[i]] != at[order[i - 1]]) ++k;
+      key[order[i]] = k;
+    }
   }
-  // counting sort by box (stable: atom-major order within a box)
-  const long long nkeys = nbx[0] * nbx[1] * nbx[2];
-  std::vector<long long> start(nkeys + 1, 0), order(n);
-  for (long long t = 0; t < n; ++t) ++start[key[t] + 1];
-  for (long long k = 0; k < nkeys; ++k) start[k + 1] += start[k];
-  for (long long t = 0; t < n; ++t) order[start[key[t]]++] = t;
   std::vector<double> sorted((size_t)n * 4);
   for (long long t = 0; t < n; ++t) memcpy(&sorted[4 * t], &x->grid[4 * order[t]], 4 * sizeof(double));
   // batches and their shells
