@@ -66,7 +66,7 @@ DEPS = {
     "jkc_class.hip": ["jkc_device.h", "launch_grid.h", "jk_device.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc",
                       "rys_table_f32.inc"],
     "dispatch.hip": ["eri_device.h", "grad_device.h", "grad_params.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
-    "session.hip": ["oqph_common.h", "response.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
+    "session.hip": ["oqph_common.h", "pair_order.h", "response.h", "grad_params.h", "ao_xform.h", "session_view.h", "../../include/oqph.h"],
     "grad_class.hip": ["grad_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc", "rys_table.inc", "rys_table_f32.inc"],
     "gradc_class.hip": ["gradc_device.h", "grad_params.h", "eri_device.h", "oqph_common.h", "boys_table.inc",
                         "rys_table.inc", "rys_table_f32.inc"],

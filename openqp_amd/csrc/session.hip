@@ -27,6 +27,7 @@
 #include "../../include/oqph.h"
 #include "oqph_common.h"
 #include "grad_params.h"
+#include "pair_order.h"
 #include "response.h"
 #include "session_view.h"
 
@@ -859,7 +860,7 @@ static int prepare_geometry(oqph_session* s) {
   for (size_t pid = 0; pid < np; ++pid) {
     s->pairs[pid].Q = s->Q[pid];
     PrimPair* pp = prims.data() + s->pairs[pid].prim0;
-    const auto more = [](const PrimPair& x, const PrimPair& y) { return std::fabs(x.Kg) > std::fabs(y.Kg); };
+    const auto more = [](const PrimPair& x, const PrimPair& y) { return larger_k(x.Kg, y.Kg); };
     if (s->pairs[pid].nprim > 1) std::sort(pp, pp + s->pairs[pid].nprim, more);
   }
   // class lists of significant pairs, Q descending
