@@ -202,14 +202,13 @@ int oqph_fock_jk_device(oqph_session *s, const double *d_dev, double *f_dev, int
  * oqph_fock_jk_device with nfocks = 1; d_dev, f_dev are device pointers
  * supplied by the caller.  The build's own device memory -- shell-pair
  * density maxima, statistics counters, work lists, ket-side Coulomb buffer,
- * gathered density -- lives in a static array of OQPH_NOALLOC_SCRATCH_BYTES
- * that each GPU the library runs on holds until the process ends; a
- * basis/density that needs more declines with code 1 and a message giving
- * the size.  The call performs no hipMalloc,
- * hipFree or other device allocation: the session must have been prepared
- * first (oqph_session_prepare, which does allocate; also after a change of
- * basis, geometry, thresholds or share).  All calls on one GPU share its
- * array: calls that overlap on one GPU (other streams, other host threads'
+ * gathered density -- lives in an array of OQPH_NOALLOC_SCRATCH_BYTES per
+ * GPU, allocated with the first session there and held until the process
+ * ends; a basis/density that needs more declines with code 1 and a message
+ * giving the size.  The call performs no hipMalloc, hipFree or other device
+ * allocation: the session must have been prepared first
+ * (oqph_session_prepare, which does allocate; also after a change of basis,
+ * geometry, thresholds or share).  All calls on one GPU share its array: calls that overlap on one GPU (other streams, other host threads'
  * kernels still running) race; the library serialises its own host side. */
 #define OQPH_NOALLOC_SCRATCH_BYTES (320ull << 20)
 int oqph_fock_jk_noalloc(oqph_session *s, const double *d_dev, double *f_dev, double se, double sc,

@@ -365,18 +365,16 @@ static unsigned long long g_serial = 0;  // last session serial handed out (unde
 // ------------------------------------------------ no-allocation scratch
 // Device memory of oqph_fock_jk_noalloc: the shell-pair density maxima, the
 // statistics counters, the work lists, the ket-side Coulomb buffer and the
-// gathered density of one build, in a static array that every GPU the library
-// runs on holds until the process ends.  Host code
-// never uses the array's name as an address: each device's copy is looked up
-// once with hipGetSymbolAddress (oqph_session_create, device current) and
-// that pointer is what kernels, memsets and copies receive.
-static __device__ __align__(256) unsigned char scratch[OQPH_NOALLOC_SCRATCH_BYTES];
+// gathered density of one build, in one array per GPU that the first session
+// there allocates and that stays until the process ends.  (As a __device__ array
+// it is filled when the code object is loaded, 0.4 ms per MiB: the first session
+// of a process took 35 ms with 64 MiB of it, 137 with these 320.)
 #define OQPH_MAX_DEVICES 64
 struct ScratchSlot {
-  unsigned char* ptr = nullptr;     // this device's copy of scratch
-  int looked_up = 0;                // 1 after hipGetSymbolAddress ran (ptr null if it failed)
+  unsigned char* ptr = nullptr;     // the device's array
+  int looked_up = 0;                // 1 after the allocation was tried (ptr null if it failed)
   unsigned long long serial = 0;    // session and list generation whose work
-  unsigned long long gen = 0;       // lists the copy holds
+  unsigned long long gen = 0;       // lists the array holds
 };
 static ScratchSlot g_scratch[OQPH_MAX_DEVICES];
 
@@ -384,7 +382,7 @@ static ScratchSlot g_scratch[OQPH_MAX_DEVICES];
 static void scratch_lookup(int device) {
   if (device < 0 || device >= OQPH_MAX_DEVICES || g_scratch[device].looked_up) return;
   void* ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+  const hipError_t e = hipMalloc(&ptr, OQPH_NOALLOC_SCRATCH_BYTES);
   g_scratch[device].looked_up = 1;
   g_scratch[device].ptr = (e == hipSuccess) ? (unsigned char*)ptr : nullptr;
   if (e != hipSuccess) (void)hipGetLastError();  // leave no sticky error for the next call
@@ -1020,8 +1018,8 @@ static int prepare_attenuated(oqph_session* s, double mu) {
 // multi-class forms): their blocks are one wavefront, LDS-limited to per_cu
 // per CU, and walk a chunk's surviving quartets one after another, so a
 // launch of few 64-ket chunks (a small molecule's f or (dd|dd) classes) would
-// leave most of the device idle; such launches split each chunk over 2, 4 or
-// 8 blocks until they have two rounds of resident blocks.
+// leave most of the device idle; such launches split each chunk over up to 64 /
+// `least` blocks until they have two rounds of resident blocks.
 static int hl_kpb(const oqph_session* s, long long chunks, int lds, int least = 1) {
   if (s->hl_kpb > 0) return s->hl_kpb;
   const long long per_cu = std::min<long long>(16, (long long)(s->lds_max / (size_t)std::max(lds, 1)));
@@ -1049,7 +1047,10 @@ static long long class_weight(int la, int lb, int lc, int ld, bool runtime) {
 // classes of the run-time kernel 425 -> 100 and 3.6 -> 1.1.  Below the line the
 // lanes and LDS round trips cost more than they save: (dp|ps), 54 components,
 // 14 against 34 and 0.8 against 3.1; (ds|pp) 8.7 against 20; (ds|ds) 3.8 against 13.
-// The FP32 classes of a mixed gradient and the MRSF gradient keep k_grad / k_gradh.
+// The MRSF gradient keeps k_grad / k_gradh, and so does the FP32 part of a class in a
+// mixed gradient: there is no FP32 form of k_gradc.  With it the mixed gradient of
+// (H2O)16/cc-pVTZ, whose classes are mostly on k_gradc in FP64, is no faster than the
+// FP64 one (262 against 251 ms; 358 against 501 with every class on k_grad / k_gradh).
 static bool gradc_class(const oqph_session* s, int la, int lb, int lc, int ld, KernelRes* r) {
   if (!s->gradc_on || s->grad_all_hl || (s->grad_hl_ng == 0 && grad_template(la, lb, lc, ld))) return false;
   if (!s->f_templates && (la == 3 || lc == 3)) return false;
@@ -1950,10 +1951,9 @@ static void bind_lists(const oqph_session* s, oqph_session::WLaunch& L, const in
   L.ww.choff = choff + L.ch0;
 }
 
-// The no-allocation entry point's scratch: the calling device's copy of the
-// static array, and a host record of which session's work lists it holds.
+// The no-allocation entry point's scratch: the device's array and a host record of which session's work lists it holds.
 struct StaticScratch {
-  unsigned char* base;        // device address from hipGetSymbolAddress
+  unsigned char* base;
   size_t bytes;
   unsigned long long* serial;  // session serial and list generation of the
   unsigned long long* gen;     // lists last uploaded into it
@@ -1985,7 +1985,7 @@ static int streams_join(oqph_session* s, hipStream_t main, int n) {
 // G[D] on device buffers; D already on the device.  The screening densities
 // scr_a (and scr_b) default to D; zero_f = false accumulates into dF.  mu > 0:
 // the erf(mu r)/r attenuated pass (pair records with the attenuated bounds).
-// ss: run in the static scratch of the no-allocation entry point instead of
+// ss: run in the scratch array of the no-allocation entry point instead of
 // the session's buffers (no device allocation; profiling is off there).
 static int build_device(oqph_session* s, const double* dD, double* dF, double se, double sc, oqph_stats* st,
                         hipStream_t stream, const double* scr_a = nullptr, const double* scr_b = nullptr,
@@ -2011,7 +2011,7 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
     dsh = (double*)carve(nsh2 * sizeof(double));
     if (off > ss->bytes) {
       set_err("no-allocation build: %zu shells need %zu bytes of scratch for the shell-pair maxima alone; the "
-              "static scratch holds %zu", (size_t)s->nsh, off, ss->bytes);
+              "scratch array holds %zu", (size_t)s->nsh, off, ss->bytes);
       return 1;
     }
   }
@@ -2049,7 +2049,7 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
     dpm = (double*)carve(std::max<size_t>(s->h_dpairs.size(), 1) * sizeof(double));
     if (off > ss->bytes) {
       set_err("no-allocation build: this basis and density need %zu bytes of scratch (shell-pair maxima, "
-              "counters, work lists, the ket-side Coulomb buffer and the gathered density); the static scratch "
+              "counters, work lists, the ket-side Coulomb buffer and the gathered density); the scratch array "
               "holds %zu", off, ss->bytes);
       return 1;
     }
@@ -2168,13 +2168,16 @@ static int build_device(oqph_session* s, const double* dD, double* dF, double se
 }
 
 // The response pass stores its integrals and contracts them with k_response
-// (session buffer d_gT, npair x nbf x nbf doubles, given back with the session)
-// up to 16 GiB of them (nbf about 250) when that is at most half of the free
-// memory; beyond that, or if the allocation fails, k_jkh adds every quartet into
-// all densities.  One pass, 28 densities, k_jkh -> dense: one water/6-31G 1.9 ->
-// 0.66 ms, (H2O)8/6-31G 50.9 -> 1.75, (H2O)14/6-31G 137 -> 8.1, (H2O)8/cc-pVDZ (192
-// AOs, 5.7 GB) 391 -> 14.6, one water/cc-pVTZ 51 -> 5.5; 7 densities of (H2O)8/6-31G
-// 32 -> 1.4: dense wins at every size it fits.
+// (session buffer d_gT, npair x nbf x nbf doubles) up to 16 GiB of them (nbf about
+// 250) when that is at most half of the free memory; beyond that, or if the
+// allocation fails, k_jkh adds every quartet into all densities.  The buffer is
+// cleared and filled by every pass; it is allocated by the session's first one and
+// stays, for other geometries too, until the session is destroyed.  One pass, 28
+// densities, k_jkh -> dense: one water/6-31G 1.9 -> 0.66 ms, (H2O)8/6-31G 50.9 -> 1.75,
+// (H2O)14/6-31G 137 -> 8.1, (H2O)8/cc-pVDZ (192 AOs, 5.5 GB) 391 -> 14.6, one
+// water/cc-pVTZ 51 -> 5.5; 7 densities of (H2O)8/6-31G 32 -> 1.4: dense wins at every
+// size it fits.  A new session with its first pass, 7 densities: one water/6-31G 4.7 ->
+// 2.1 ms, (H2O)8/6-31G(d) 49 -> 9.2, (H2O)8/cc-pVDZ 323 -> 27.
 static size_t response_elems(const oqph_session* s) {  // 0: not dense
   const char* e = getenv("OQPH_RESPONSE");  // 0: never
   if (e && e[0] == '0') return 0;
@@ -2635,7 +2638,7 @@ int oqph_fock_jk_noalloc(oqph_session* s, const double* d_dev, double* f_dev, do
   std::lock_guard<std::mutex> lk(g_mtx);  // the scratch tag of the device
   ScratchSlot* slot = (s->device < OQPH_MAX_DEVICES) ? &g_scratch[s->device] : nullptr;
   if (!slot || !slot->ptr) {
-    set_err("no-allocation build: the static scratch of device %d is unavailable", s->device);
+    set_err("no-allocation build: the scratch array of device %d is unavailable", s->device);
     return 2;
   }
   const StaticScratch ss{slot->ptr, (size_t)OQPH_NOALLOC_SCRATCH_BYTES, &slot->serial, &slot->gen};

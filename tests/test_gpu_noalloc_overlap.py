@@ -1,4 +1,4 @@
-"""A no-allocation build keeps all of its device memory in the static array, so it
+"""A no-allocation build keeps all of its device memory in an array of its own, so it
 may run while a device build of the same session is still in flight on another
 stream: both are issued without statistics (nothing then waits for the device),
 with densities of different size, and each result is that of the build alone.  Two
