@@ -208,8 +208,9 @@ int oqph_fock_jk_device(oqph_session *s, const double *d_dev, double *f_dev, int
  * giving the size.  The call performs no hipMalloc, hipFree or other device
  * allocation: the session must have been prepared first
  * (oqph_session_prepare, which does allocate; also after a change of basis,
- * geometry, thresholds or share).  All calls on one GPU share its array: calls that overlap on one GPU (other streams, other host threads'
- * kernels still running) race; the library serialises its own host side. */
+ * geometry, thresholds or share).  All calls on one GPU share its array:
+ * calls that overlap on one GPU (other streams, other host threads' kernels
+ * still running) race; the library serialises its own host side. */
 #define OQPH_NOALLOC_SCRATCH_BYTES (320ull << 20)
 int oqph_fock_jk_noalloc(oqph_session *s, const double *d_dev, double *f_dev, double se, double sc,
                          oqph_stats *stats, void *stream);

@@ -9,8 +9,9 @@
 // element of T read (twice for K, once for J) meets nd columns and the reads of T
 // bound the kernel, not the matrix units.  Adding every quartet into nd matrices
 // instead costs 12 nd atomics and as many gathers per s quartet.  (H2O)8/6-31G, 28
-// densities: 50.9 ms per pass then, now 0.31 + 0.12 ms for the two products (4.5
-// TB/s of T) and 1.75 ms in all; other sizes at response_elems() in session.hip.
+// densities: 50.9 ms per pass then, now 0.31 + 0.12 ms for the two products (T, 0.51 GB,
+// read twice for K and once for J: 3.3 and 4.4 TB/s) and 1.75 ms in all; other sizes at
+// response_elems() in session.hip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
