@@ -51,7 +51,7 @@ constexpr double RHO_FLOOR = 1e-30;  // spin densities are floored here
 constexpr double SSF_A = 0.64;
 // bohr; the smaller, the fewer functions reach a batch and the more V_b there are.
 // (H2O)32/6-31G(d): 4 bohr 23.2 ms per build (1.7e11 functions^2 points), 3 19.6, 2 15.9
-// (0.94e11), 1.5 15.5 with twice the batches (13820) of 2
+// (0.94e11), 1.5 15.5 with twice the batches (13820) of 2, all at a cut-off of 1e-12
 constexpr double BOX = 2.0;
 constexpr int MAX_BATCH = 32768;
 constexpr long long GROUP_ELEMS = 1ll << 28;  // basis-function values of a group of batches: 2 GB
@@ -339,8 +339,8 @@ __global__ void k_grid(GridArgs g) {
 // where the device is short of memory); a build takes one launch of each kernel per
 // group, over all its batches.  A launch per batch, three gathers of the density and three library products with
 // phi, its gradient, X and Y in memory took 65 ms for (H2O)32/6-31G(d) with its
-// 1045 batches of 4 bohr; this 15.9 (groups of 2^25 values: 28.1 against 23.8 for
-// 2^28, both on boxes of 4 bohr).
+// 1045 batches of 4 bohr; this 15.9, and 17.0 with the present cut-off (groups of 2^25
+// values: 28.1 against 23.8 for 2^28, both on boxes of 4 bohr).
 struct DBatch {
   long long p0;   // first point of the grid
   long long off;  // first element of the batch's matrices in the group's arrays
